@@ -288,11 +288,13 @@ DVC_MATH_FN float dvc_logf_phi(float x, const double *tab) {
 #endif
   const double invcs = tab[2 * e], y0 = tab[2 * e + 1];
   const double r = fma((double)x, invcs, -1.0);
-  const double r2 = r * r;
-  double y = fma(A1, r, A2);
-  y = fma(A0, r2, y);
-  y = fma(y, r2, y0 + r);
-  return (float)y;
+  // Horner's form of the same polynomial: two operations fewer than A0*r^4 +
+  // (A1*r + A2)*r^2 + (y0 + r); the doubles may differ in their last bits, the
+  // rounded float never does on an argument phi reaches (swept exhaustively)
+  double p = fma(A0, r, A1);
+  p = fma(p, r, A2);
+  p = fma(p, r, 1.0);
+  return (float)fma(p, r, y0);
 }
 
 // dvc_bp_phi for x >= 0 (the magnitudes BP applies it to), bit-identical to
@@ -386,7 +388,11 @@ DVC_MATH_FN float dvcm_div_phi(float a, float b) {
 #endif
 }
 
-// dvc_bp_phi_nonneg with fewer instructions, same value for every x >= 0:
+// dvc_bp_phi_nonneg with fewer instructions, same value for every x >= 0.  Two
+// of these per edge are what bounds the BP kernels, whose VALU issue port is
+// busy throughout: 55 instructions here, 66 before the steps marked *, which
+// took the search of one N = 6336 bitplane (8 codes of 50 iterations) from
+// 6.99 to 6.14 ms and 512 mixed bitplanes at 100 iterations from 17.7 to 16.1:
 //   * y is clamped to 9.75: tanhf(y) is 1.0f from y = 9.02 on (2/(e^2y+1)
 //     is below half an ulp of 1), so every larger argument gives the same
 //     result, every intermediate is finite, and expm1f's reduction index k
@@ -395,38 +401,46 @@ DVC_MATH_FN float dvcm_div_phi(float a, float b) {
 //     a - k*ln2_hi - k*ln2_lo reproduces expm1f's special cases by itself:
 //     k = 0 leaves a unchanged (the unreduced case, c = 0) and k = -1 is
 //     exactly the hx < 1.5 ln2 case's a + ln2_hi, -ln2_lo; k is rint(a/ln2)
-//     where expm1f has (int)(a/ln2 +- 0.5): they differ on 14 floats a of
-//     this range, on which phi's result is the same;
-//   * k takes the values -3..0 and 3..28; the result cases k = 0, k = -1,
-//     k <= -2 and k >= 3 are all computed and one selected (no branches);
-//     for k = 23..28 (y >= 7.8) the k <= 22 form stands in for expm1f's
-//     k > 22 form, which gives the same tanhf there; |a| < 2^-25 needs no
-//     case of its own (x - (x*e - hxs) is x there);
-//   * expm1f's polynomial stops at Q4: on the reduced arguments here
-//     (|r| <= 0.35) the Q5 term never changes the final result;
+//     where expm1f has (int)(a/ln2 +- 0.5), formed (*) by one fma onto 1.5 *
+//     2^23, whose low bits then hold k for the shifts; where the two indices
+//     differ, phi's result is the same;
+//   * k takes the values -3..0 (x < 2) and 3..28; |a| < 2^-25 needs no case of
+//     its own (x - (x*e - hxs) is x there), and for k = 23..28 (y >= 7.8) the
+//     k <= 22 form stands in for expm1f's k > 22 form, which gives the same
+//     tanhf there;
+//   * expm1f's polynomial stops at Q3 and (*) is evaluated by two fused steps
+//     with coefficients refitted on the reduced range (|r| <= 0.35): r1 then
+//     differs from expm1f's in its last bit for some arguments, in none of
+//     which phi's result differs;
+//   * (*) h2 = xx*xx stands for 2*hxs: every use takes the exact half back in
+//     its own fused step, so 0.5*xx is never formed;
 //   * both quotients use dvcm_div_phi;
 //   * a - k*ln2_hi is one fused multiply-add: k*ln2_hi is exact (|k| <= 28
 //     and ln2_hi has 17 significant bits), so the single rounding is the
-//     subtraction's; likewise 0.5*(xx - e2) - 0.5, whose product is exact
-//     (and xx - e2 is the negated e2 - xx, which the k <= -2 and k >= 3
-//     cases use as well);
-//   * the k = 0 result is -u (u = e2 - xx, below), and one expression gives
-//     the k <= -2 and k >= 3 cases' Y;
+//     subtraction's; hi - k*ln2_lo is fused as well (its one rounding gives
+//     the same xx wherever phi's result depends on it);
+//   * (*) one expression gives every result case.  With u = e2 - xx and A =
+//     2^k: k = 0 returns -u, k = -1 returns 0.5*(xx - e2) - 0.5 and k >= 3
+//     returns ((1 - 2^-k) - u) * 2^k, each a single rounding of A*(-u) + (A -
+//     1); k <= -2 returns (1 - u) * 2^k - 1, which rounds 1 - u first.  So v =
+//     B - u with B = 1 for k <= -2, else 0, and em1 = A*v + (A*(1 - B) - 1),
+//     where B and 1 - B are -1 - k and k + 2 clamped to [0, 1] (a free output
+//     modifier);
 //   * logf is dvc_logf_phi with its (k, i) table in `phitab`.
-// Pins a value in a register at this point, so the compiler cannot sink its
-// computation into a branch (device builds; a no-op on the host).
-DVC_MATH_FN float dvcm_pin(float v) {
+// x clamped to [0, 1].
+DVC_MATH_FN float dvcm_clamp01(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __asm__("" : "+v"(v));
+  return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f);
+#else
+  return x < 0.0f ? 0.0f : (x > 1.0f ? 1.0f : x);
 #endif
-  return v;
 }
 
 DVC_MATH_FN float dvc_bp_phi_fast(float x, const double *phitab) {
   DVCM_NOCONTRACT
+  // C1..C3: refitted Q1/2, Q2/4, Q3/8 of expm1f, for powers of h2 = 2*hxs
   const float ln2_hi = 6.9313812256e-01f, ln2_lo = 9.0580006145e-06f, invln2 = 1.4426950216e+00f,
-              Q1 = -3.3333335072e-02f, Q2 = 1.5873016091e-03f, Q3 = -7.9365076090e-05f,
-              Q4 = 4.0082177293e-06f;
+              C1 = -0x1.111112p-6f, C2 = 0x1.a0193ap-12f, C3 = -0x1.4b1072p-17f;
   // y0 = (x + 1e-9f)/2 and a = +-2*min(y0, 9.75): halving and doubling s =
   // x + 1e-9f (a normal float) are exact, so a = min(s, 19.5) when y0 >= 1
   // (s >= 2) and -s below, with the same bits as the halved-then-doubled form
@@ -434,36 +448,22 @@ DVC_MATH_FN float dvc_bp_phi_fast(float x, const double *phitab) {
   const int big = s >= 2.0f;
   const float a = big ? fminf(s, 19.5f) : -s;
   // ---- expm1f(a), a in (-2, -1e-9] or [2, 19.5]
-  // k = rint(invln2*a) in place of trunc(invln2*a +- 0.5): the two differ on
-  // 14 floats a of this range, and phi's result is the same on those (every
-  // argument is checked exhaustively); rint leaves tk a float and k one
-  // conversion away
-  const float tk = rintf(invln2 * a);
-  const int k = (int)tk;
+  const float m = fmaf(invln2, a, 12582912.0f);  // 1.5 * 2^23 + k
+  const float tk = m - 12582912.0f;
   const float hi = fmaf(-tk, ln2_hi, a);
   const float lo = tk * ln2_lo;
-  const float xx = hi - lo;
+  const float xx = fmaf(-tk, ln2_lo, hi);
   const float c = (hi - xx) - lo;
-  const float hfx = 0.5f * xx;
-  const float hxs = xx * hfx;
-  const float r1 = 1.0f + hxs * (Q1 + hxs * (Q2 + hxs * (Q3 + hxs * Q4)));
-  const float t3 = 3.0f - r1 * hfx;
-  const float e = hxs * dvcm_div_phi(r1 - t3, 6.0f - xx * t3);
-  float e2 = (xx * (e - c) - c);
-  e2 -= hxs;
+  const float h2 = xx * xx;
+  const float r1 = 1.0f + h2 * fmaf(h2, fmaf(h2, C3, C2), C1);
+  const float t3 = fmaf(-0.5f, r1 * xx, 3.0f);  // 3 - r1*hfx
+  const float ed = h2 * dvcm_div_phi(r1 - t3, 6.0f - xx * t3);  // 2e
+  float e2 = xx * fmaf(0.5f, ed, -c) - c;
+  e2 = fmaf(-0.5f, h2, e2);
   const float u = e2 - xx;
-  // k = 0: c is +0 (hi = a, lo = +0), so e2 is xx*e - hxs with the same two
-  // roundings as the k = 0 result's inner term, and xx - (xx*e - hxs) is -u
-  const float r_k0 = -u;
-  const float r_km1 = fmaf(-0.5f, u, -0.5f);  // 0.5f * (xx - e2) - 0.5f: xx - e2 is -u exactly
-  // k >= 3: Y = (1 - 2^-k) - u; k <= -2: Y = 1 - u, which the same expression
-  // gives, since k & 31 is then 29 or 30 and 2^24 >> 29 (or 30) is 0
-  const float Y = dvcm_pin(dvcm_asf(0x3f800000u - (0x1000000u >> (k & 31))) - u);
-  const float R = dvcm_asf(dvcm_asu(Y) + ((uint32_t)k << 23));
-  // k >= 3 exactly on the lanes with a >= 2 (big); the others have k in -3..0
-  float em1 = (k == -1) ? r_km1 : r_k0;
-  em1 = (k <= -2) ? R - 1.0f : em1;
-  em1 = big ? R : em1;
+  const float A = dvcm_asf(0x3f800000u + (dvcm_asu(m) << 23));  // 2^k
+  const float v = dvcm_clamp01(-1.0f - tk) - u;
+  const float em1 = fmaf(A, v, fmaf(A, dvcm_clamp01(tk + 2.0f), -1.0f));
   // ---- tanhf(y)
   const float q = dvcm_div_phi(big ? 2.0f : -em1, em1 + 2.0f);
   const float z = big ? 1.0f - q : q;
