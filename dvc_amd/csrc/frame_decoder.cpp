@@ -127,6 +127,10 @@ struct Job {
 
 static size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// Bytes of FrameDev::npPart for N blocks, and of FrameDev::npMom.
+static size_t np_part_bytes(size_t N) { return sizeof(uint2) * 16 * ((N + 255) / 256); }
+constexpr size_t kNpMomBytes = sizeof(float2) * 16;
+
 // Device bytes one frame needs (the layout alloc_job carves).
 static size_t job_bytes(const Job &j) {
   const int W = j.W, H = j.H, N = j.N, FS = W * H;
@@ -135,9 +139,9 @@ static size_t job_bytes(const Job &j) {
   size_t t = 0;
   for (size_t b : {(size_t)FS, 4 * (size_t)FS, 4 * (size_t)FS, 4 * (size_t)FS, 4 * (size_t)FS,
                    (size_t)64 * (W - 3) * (H - 3), (size_t)4 * (W - 3) * (H - 3), (size_t)4 * 81 * N, (size_t)4 * N * std::max(maxStride, 1),
-                   4 * (size_t)N, (size_t)N, (size_t)FS, sizeof(MVd) * (size_t)(FS / 256), sizeof(MVd) * (size_t)(FS / 64),
-                   sizeof(MVd) * (size_t)(FS / 64), sizeof(MVd) * (size_t)(FS / 256), 16 * (size_t)(FS / 256),
-                   8 * (size_t)(FS / 64), (size_t)j.nbp * (N / 8),
+                   4 * (size_t)N, (size_t)N, (size_t)FS, sizeof(MVs) * (size_t)(FS / 64),
+                   sizeof(MVd) * (size_t)(FS / 256), 16 * (size_t)(FS / 256), np_part_bytes(N), kNpMomBytes,
+                   (size_t)j.nbp * (N / 8),
                    sizeof(PlaneState) * (size_t)j.nbp, sizeof(int4) * kMaxCodes * (size_t)j.nbp, 4 * (size_t)N,
                    (size_t)N, 4 * kMaxCodes * (size_t)j.nbp, (size_t)FS / 64, j.intra.size() * sizeof(int32_t),
                    j.deblock ? (size_t)FS : 0, j.deblock ? 2 * (size_t)N : 0, j.deblock ? 16 * (size_t)N : 0,
@@ -157,9 +161,9 @@ static void carve_job(Job &j, uint8_t *base) {
                o_al = take(4 * (size_t)FS), o_oct = take((size_t)64 * (W - 3) * (H - 3)),
                o_ob = take((size_t)4 * (W - 3) * (H - 3)), o_smf = take((size_t)4 * 81 * N),
                o_dist = take((size_t)4 * N * std::max(maxStride, 1)), o_lr = take(4 * (size_t)N), o_dec = take(N),
-               o_rec = take(FS), o_mb = take(sizeof(MVd) * (size_t)(FS / 256)), o_bmv = take(sizeof(MVd) * (size_t)(FS / 64)),
-               o_bmvt = take(sizeof(MVd) * (size_t)(FS / 64)), o_fwd = take(sizeof(MVd) * (size_t)(FS / 256)),
-               o_holes = take(16 * (size_t)(FS / 256)), o_mse = take(8 * (size_t)(FS / 64)),
+               o_rec = take(FS), o_bmv = take(sizeof(MVs) * (size_t)(FS / 64)),
+               o_fwd = take(sizeof(MVd) * (size_t)(FS / 256)), o_holes = take(16 * (size_t)(FS / 256)),
+               o_npp = take(np_part_bytes(N)), o_npm = take(kNpMomBytes),
                o_acc = take((size_t)j.nbp * (N / 8)), o_state = take(sizeof(PlaneState) * (size_t)j.nbp),
                o_recd = take(sizeof(int4) * kMaxCodes * (size_t)j.nbp), o_llr = take(4 * (size_t)N),
                o_carry = take(N), o_bcase = take(4 * kMaxCodes * (size_t)j.nbp), o_mode = take((size_t)FS / 64),
@@ -173,9 +177,9 @@ static void carve_job(Job &j, uint8_t *base) {
   f.reconsTrans = (int *)(base + o_rt); f.alpha = (float *)(base + o_al); f.oct = (int *)(base + o_oct);
   f.octBand = (int *)(base + o_ob);
   f.smf = (float *)(base + o_smf); f.dist = (float *)(base + o_dist); f.LR = (float *)(base + o_lr);
-  f.decoded = base + o_dec; f.recons = base + o_rec; f.mbmv = (MVd *)(base + o_mb); f.bmv = (MVd *)(base + o_bmv);
-  f.bmv_tmp = (MVd *)(base + o_bmvt); f.fwd = (MVd *)(base + o_fwd); f.holes = (double *)(base + o_holes);
-  f.mse = (double *)(base + o_mse);
+  f.decoded = base + o_dec; f.recons = base + o_rec; f.bmv = (MVs *)(base + o_bmv);
+  f.fwd = (MVd *)(base + o_fwd); f.holes = (double *)(base + o_holes);
+  f.npPart = (uint2 *)(base + o_npp); f.npMom = (float2 *)(base + o_npm);
   j.d_acc = base + o_acc; j.d_state = (PlaneState *)(base + o_state); j.d_rec = (int4 *)(base + o_recd);
   j.d_LLR = (float *)(base + o_llr);
   j.d_carry = base + o_carry;
@@ -1103,8 +1107,8 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
   for (int i = 0; i < n; i++) {
     const size_t FS = (size_t)reqs[i].width * reqs[i].height;
     size_t t = 0;
-    for (size_t b : {6 * FS, 6 * FS, FS, 4 * FS, 4 * FS, 4 * FS, sizeof(MVd) * (FS / 256), sizeof(MVd) * (FS / 64),
-                     sizeof(MVd) * (FS / 64), sizeof(MVd) * (FS / 256), 16 * (FS / 256), 8 * (FS / 64)})
+    for (size_t b : {6 * FS, 6 * FS, FS, 4 * FS, 4 * FS, 4 * FS, sizeof(MVs) * (FS / 64), sizeof(MVd) * (FS / 256),
+                     16 * (FS / 256), np_part_bytes(FS / 16), kNpMomBytes})
       t = align_up(t + b);
     base[i + 1] = base[i] + t;
     maxN = std::max(maxN, (int)(FS / 16));
@@ -1144,12 +1148,11 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
       f.residue = (int *)take(4 * FS);
       f.sideTrans = (int *)take(4 * FS);
       f.alpha = (float *)take(4 * FS);
-      f.mbmv = (MVd *)take(sizeof(MVd) * (FS / 256));
-      f.bmv = (MVd *)take(sizeof(MVd) * (FS / 64));
-      f.bmv_tmp = (MVd *)take(sizeof(MVd) * (FS / 64));
+      f.bmv = (MVs *)take(sizeof(MVs) * (FS / 64));
       f.fwd = (MVd *)take(sizeof(MVd) * (FS / 256));
       f.holes = (double *)take(16 * (FS / 256));
-      f.mse = (double *)take(8 * (FS / 64));
+      f.npPart = (uint2 *)take(np_part_bytes(FS / 16));
+      f.npMom = (float2 *)take(kNpMomBytes);
       list[i] = i;
       DVC_HIP(hipMemcpyAsync(kp, r.past, FS, hipMemcpyHostToDevice, s));
       DVC_HIP(hipMemcpyAsync(kf, r.fut, FS, hipMemcpyHostToDevice, s));

@@ -13,6 +13,10 @@ struct MVd {                 // MV of global.h:170-174: past, future, vector (x,
   double px, py, fx, fy, vx, vy;
 };
 
+// A block's motion vector on the half-pel grid while the side information is
+// made: its positions in the future and past frames (vector = past - future).
+struct MVs { short fx, fy, px, py; };
+
 struct FrameDev {
   // geometry
   int W, H, N;               // N = number of 4x4 blocks = LDPCA code length
@@ -53,12 +57,12 @@ struct FrameDev {
   float *LR;                 // N likelihood ratios of the current bitplane
   uint8_t *decoded;          // N decoded bits of the current bitplane
   uint8_t *recons;           // W*H reconstruction
-  MVd *mbmv;                 // macroblock MVs (W/16*H/16)
-  MVd *bmv;                  // 8x8 block MVs (W/8*H/8)
-  MVd *bmv_tmp;              // 8x8 MVs after the vector-median filter
+  MVd *mbmv;                 // macroblock MVs (W/16*H/16; forwardME alone)
+  MVs *bmv;                  // 8x8 block MVs after the bidirectional refinement (W/8*H/8)
   MVd *fwd;                  // forward-ME result per macroblock
   double *holes;             // 2 per macroblock
-  double *mse;               // per 8x8 block
+  uint2 *npPart;             // per 256 blocks and coefficient: sums of the residue transform's magnitudes and squares
+  float2 *npMom;             // 16 per frame: mean and variance of a band's magnitudes
   // per-band parameters (set by the host before the band's kernels)
   int band;                  // zig-zag band number
   int index;                 // coefficient index in the 4x4 block (zigzag[band])

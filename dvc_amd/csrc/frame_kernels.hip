@@ -195,175 +195,256 @@ __global__ __launch_bounds__(256) void k_forward_me(const FrameDev *F, const int
 }
 
 // ------------------------------------------------------------ bidirectional ME chain
+// Sums over the aligned groups of LEN (8 or 16) lanes, the same on each of
+// them (quad permutes, then the mirrored half row and row).
+template <int LEN>
+__device__ __forceinline__ uint32_t group_sum(uint32_t v) {
+  v += __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, false);   // quad_perm [1, 0, 3, 2]
+  v += __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, false);   // quad_perm [2, 3, 0, 1]
+  v += __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, false);  // row_half_mirror
+  if (LEN == 16) v += __builtin_amdgcn_mov_dpp(v, 0x140, 0xf, 0xf, false);  // row_mirror
+  return v;
+}
+// Eight samples two bytes apart (a half-pel row's full-pel samples), packed in
+// two words; the 16 bytes read need not be aligned.
+__device__ __forceinline__ uint2 even_bytes(const uint8_t *p) {
+  uint4 v;
+  __builtin_memcpy(&v, p, 16);
+  return make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x06040200), __builtin_amdgcn_perm(v.w, v.z, 0x06040200));
+}
+
 // One bidirectional search step of bidirectME (sideInfoCreation.cpp:250-306)
 // for block blk, run by one wave; the block's range is bounded by its
-// neighbours' current MVs (up/left already refined, down/right not yet).
-__device__ void bidir_block(const FrameDev &f, MVd *mv, int blk, int bw, int bh, int blockLen, int lane) {
-  const int i = blk / bw, j = blk % bw, W2 = 2 * f.W, H2 = 2 * f.H, bl2 = blockLen * 2;
-  const int bot = H2 - bl2, right = W2 - bl2, y2 = i * bl2, x2 = j * bl2;
-  const int sT = (i - 1 >= 0) ? (int)mv[blk - bw].fy + bl2 : (int)mv[blk].fy;
-  const int sB = (i + 1 < bh) ? (int)mv[blk + bw].fy - bl2 : (int)mv[blk].fy;
-  const int sL = (j - 1 >= 0) ? (int)mv[blk - 1].fx + bl2 : (int)mv[blk].fx;
-  const int sR = (j + 1 < bw) ? (int)mv[blk + 1].fx - bl2 : (int)mv[blk].fx;
+// neighbours' current MVs (up/left already refined, down/right not yet).  A
+// lane takes one row of one candidate's LEN x LEN samples (two or four 16-byte
+// reads), 64 / LEN candidates at a time in raster order.  A lone candidate is taken without its cost, which is below the
+// search's limit of 10^7 whatever the pixels (at most 255 * 16 * 16 * (1 +
+// 0.05 * 996)).
+struct HalfPair {  // a frame's two half-pel key frames, for the sweeps
+  const uint8_t *past, *fut;
+  int W2, H2;
+  double scale;  // iPC / iFC
+};
+template <int LEN>
+__device__ __forceinline__ void bidir_block(const HalfPair &f, MVs *mv, int blk, int i, int j, int bw, int bh,
+                                            int lane) {
+  constexpr int L2 = 2 * LEN, G = 64 / LEN;
+  const int W2 = f.W2, bot = f.H2 - L2, right = W2 - L2, y2 = i * L2, x2 = j * L2;
+  const MVs own = mv[blk];
+  const int sT = i > 0 ? mv[blk - bw].fy + L2 : own.fy;
+  const int sB = i + 1 < bh ? mv[blk + bw].fy - L2 : own.fy;
+  const int sL = j > 0 ? mv[blk - 1].fx + L2 : own.fx;
+  const int sR = j + 1 < bw ? mv[blk + 1].fx - L2 : own.fx;
   const int nx = sR - sL + 1, ny = sB - sT + 1;
-  const double scale = f.iPC / f.iFC;
+  if (nx <= 0 || ny <= 0) return;
+  const int n = nx * ny, row = lane % LEN, g = lane / LEN;
+  // c / nx: (c + 0.5) / nx lies at least 0.5 / nx > 7e-4 from an integer and
+  // below 576, so the float quotient's error (under 2e-4) never reaches one
+  const float rnx = 1.0f / (float)nx;
+  auto pos = [&](int c, int &fy, int &fx, int &py, int &px) {
+    const int q = (int)(((float)c + 0.5f) * rnx);
+    fy = sT + q;
+    fx = sL + c - q * nx;
+    py = end_point(y2, (double)(y2 - fy), f.scale, 0, bot);
+    px = end_point(x2, (double)(x2 - fx), f.scale, 0, right);
+  };
   double best = DBL_MAX;
-  int bidx = 0x7fffffff;
-  if (nx > 0 && ny > 0) {
-    for (int c = lane; c < nx * ny; c += 64) {
-      const int fy = sT + c / nx, fx = sL + c % nx;
-      const int py = end_point(y2, (double)(y2 - fy), scale, 0, bot);
-      const int px = end_point(x2, (double)(x2 - fx), scale, 0, right);
-      int mad = 0;
-      for (int m = 0; m < bl2; m += 2) {
-        const uint8_t *pr = f.past_half + (py + m) * W2 + px;
-        const uint8_t *fr = f.fut_half + (fy + m) * W2 + fx;
-        for (int q = 0; q < bl2; q += 2) mad += abs((int)fr[q] - (int)pr[q]);
+  int bidx = n == 1 ? 0 : 0x7fffffff, fy, fx, py, px;
+  if (n > 1) {
+    for (int c0 = 0; c0 < n; c0 += G) {
+      const int c = imin(c0 + g, n - 1);
+      pos(c, fy, fx, py, px);
+      const uint8_t *pr = f.past + (size_t)(py + 2 * row) * W2 + px;
+      const uint8_t *fr = f.fut + (size_t)(fy + 2 * row) * W2 + fx;
+      uint32_t sad = 0;
+#pragma unroll
+      for (int h = 0; h < LEN; h += 8) {
+        const uint2 a = even_bytes(pr + 2 * h), b = even_bytes(fr + 2 * h);
+        sad = __builtin_amdgcn_sad_u8(a.x, b.x, sad);
+        sad = __builtin_amdgcn_sad_u8(a.y, b.y, sad);
       }
-      const double cost = cost_func((double)mad, (double)(px - fx), (double)(py - fy));
-      if (cost < 10000000.0 && (cost < best)) { best = cost; bidx = c; }
+      const double cost = cost_func((double)(int)group_sum<LEN>(sad), (double)(px - fx), (double)(py - fy));
+      if (c0 + g < n && cost < 10000000.0 && cost < best) { best = cost; bidx = c; }
+    }
+#pragma unroll
+    for (int o = LEN; o < 64; o <<= 1) {
+      const double c2 = __shfl_xor(best, o);
+      const int i2 = __shfl_xor(bidx, o);
+      if (c2 < best || (c2 == best && i2 < bidx)) { best = c2; bidx = i2; }
     }
   }
-  wave_argmin(best, bidx);
   if (lane == 0 && bidx != 0x7fffffff) {
-    const int fy = sT + bidx / nx, fx = sL + bidx % nx;
-    const int py = end_point(y2, (double)(y2 - fy), scale, 0, bot);
-    const int px = end_point(x2, (double)(x2 - fx), scale, 0, right);
-    MVd r;
-    r.fx = (double)fx; r.fy = (double)fy; r.px = (double)px; r.py = (double)py;
-    r.vx = (double)(px - fx); r.vy = (double)(py - fy);
-    mv[blk] = r;
+    pos(bidx, fy, fx, py, px);
+    mv[blk] = MVs{(short)fx, (short)fy, (short)px, (short)py};
   }
 }
 
 // Anti-diagonal sweep: blocks on diagonal d = i + j depend only on diagonal
 // d-1 (refined) and d+1 (not yet refined), so this order equals the raster
 // order of the in-place reference loop.
-__device__ void bidir_sweep(const FrameDev &f, MVd *mv, int blockLen) {
-  const int bw = f.W / blockLen, bh = f.H / blockLen;
+template <int LEN>
+__device__ __forceinline__ void bidir_sweep(const HalfPair &f, MVs *mv) {
+  const int bw = f.W2 / (2 * LEN), bh = f.H2 / (2 * LEN);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwaves = blockDim.x >> 6;
   for (int d = 0; d <= bw + bh - 2; d++) {
     const int i0 = imax(0, d - (bw - 1)), i1 = imin(bh - 1, d);
-    for (int i = i0 + wave; i <= i1; i += nwaves) bidir_block(f, mv, i * bw + (d - i), bw, bh, blockLen, lane);
-    __threadfence_block();
+    for (int i = i0 + wave; i <= i1; i += nwaves) bidir_block<LEN>(f, mv, i * bw + (d - i), i, d - i, bw, bh, lane);
     __syncthreads();
   }
 }
 
-// The rest of createSideInfo (sideInfoCreation.cpp:119-143, 510-550) and
-// motionFilterAndComp (:312-436) for one frame per workgroup.  With
+// The serial part of createSideInfo (sideInfoCreation.cpp:119-143, 510-550)
+// for one frame per workgroup: each macroblock's nearest hole, the 16x16 and
+// the 8x8 bidirectional refinements, with the motion vectors in LDS.  With
 // fwdOnly set it stops after forwardME's nearest-hole assignment (:119-143)
 // and leaves the macroblock MVs unscaled (forwardME's own output).
-__global__ __launch_bounds__(1024) void k_si_chain(const FrameDev *F, const int *list, int fwdOnly) {
+// The two sweeps' 118 dependent diagonals (CIF) bound it.  With the vectors in
+// global memory, a lane per candidate reading its samples byte by byte, and
+// the filter and compensation below in the same single workgroup, this took
+// 1930 us for a CIF frame and 550 for QCIF; now 403 and 89, and 8.5 for the
+// filter and compensation in a grid of their own.
+__global__ __launch_bounds__(1024) void k_si_sweep(const FrameDev *F, const int *list, int fwdOnly) {
   const FrameDev &f = F[list[blockIdx.x]];
-  const int tid = threadIdx.x, T = blockDim.x, W = f.W, H = f.H;
-  const int bw16 = W / 16, nmb = bw16 * (H / 16), bw8 = W / 8, bh8 = H / 8, nb8 = bw8 * bh8;
-  const int W2 = 2 * W, H2 = 2 * H;
-  // nearest hole per macroblock (:120-142) and the x2 half-pel scaling (:511-521)
-  const double maxDst = W * W + H * H;
-  for (int i = tid; i < nmb; i += T) {
+  const int tid = threadIdx.x, W = f.W, H = f.H;
+  const int bw16 = W / 16, nmb = bw16 * (H / 16), bw8 = W / 8, nb8 = bw8 * (H / 8);
+  __shared__ double2 s_hole[22 * 18];
+  __shared__ MVs s_mb[22 * 18];
+  __shared__ MVs s_blk[44 * 36];
+  for (int i = tid; i < nmb; i += 1024) s_hole[i] = make_double2(f.holes[2 * i], f.holes[2 * i + 1]);
+  __syncthreads();
+  // nearest hole per macroblock (:120-142), the holes split over two lanes,
+  // and the x2 half-pel scaling (:511-521); ties go to the lower index
+  if (tid < 2 * nmb) {
+    const int i = tid >> 1, half = (nmb + 1) >> 1;
     const int top = (i / bw16) * 16, left = (i % bw16) * 16;
-    double minDst = maxDst;
+    double minDst = W * W + H * H;
     int best = 0;
-    for (int jj = 0; jj < nmb; jj++) {
-      const double hx = f.holes[2 * jj], hy = f.holes[2 * jj + 1];
-      const double dst = (left - hx) * (left - hx) + (top - hy) * (top - hy);
+    for (int jj = (tid & 1) * half; jj < ((tid & 1) ? nmb : half); jj++) {
+      const double2 h = s_hole[jj];
+      const double dst = (left - h.x) * (left - h.x) + (top - h.y) * (top - h.y);
       if (dst < minDst) { minDst = dst; best = jj; }
     }
-    const MVd b = f.fwd[best];
-    MVd o;
-    o.fx = (double)end_point(left, -b.vx, f.iFC, 0, W - 16);
-    o.fy = (double)end_point(top, -b.vy, f.iFC, 0, H - 16);
-    o.px = (double)end_point(left, b.vx, f.iPC, 0, W - 16);
-    o.py = (double)end_point(top, b.vy, f.iPC, 0, H - 16);
-    if (!fwdOnly) { o.fx *= 2; o.fy *= 2; o.px *= 2; o.py *= 2; }
-    o.vx = o.px - o.fx; o.vy = o.py - o.fy;
-    f.mbmv[i] = o;
+    const double d2 = __shfl_xor(minDst, 1);
+    const int b2 = __shfl_xor(best, 1);
+    if ((tid & 1) == 0) {
+      if (d2 < minDst) best = b2;
+      const double vx = f.fwd[best].vx, vy = f.fwd[best].vy;
+      const int fx = end_point(left, -vx, f.iFC, 0, W - 16), fy = end_point(top, -vy, f.iFC, 0, H - 16);
+      const int px = end_point(left, vx, f.iPC, 0, W - 16), py = end_point(top, vy, f.iPC, 0, H - 16);
+      s_mb[i] = MVs{(short)(2 * fx), (short)(2 * fy), (short)(2 * px), (short)(2 * py)};
+      if (fwdOnly) {
+        MVd o;
+        o.fx = fx; o.fy = fy; o.px = px; o.py = py;
+        o.vx = px - fx; o.vy = py - fy;
+        f.mbmv[i] = o;
+      }
+    }
   }
   if (fwdOnly) return;
-  __threadfence_block();
   __syncthreads();
-  bidir_sweep(f, f.mbmv, 16);
+  const HalfPair hp = {f.past_half, f.fut_half, 2 * W, 2 * H, f.iPC / f.iFC};
+  bidir_sweep<16>(hp, s_mb);
   // 8x8 initial MVs from the 16x16 vectors (:524-545)
-  for (int b = tid; b < nb8; b += T) {
+  for (int b = tid; b < nb8; b += 1024) {
     const int i = b / bw8, j = b % bw8, y2 = i << 4, x2 = j << 4;
-    const MVd m = f.mbmv[(i >> 1) * bw16 + (j >> 1)];
-    MVd r;
-    r.fx = (double)end_point(x2, -m.vx, f.iFC, 0, (W - 8) << 1);
-    r.fy = (double)end_point(y2, -m.vy, f.iFC, 0, (H - 8) << 1);
-    r.px = (double)end_point(x2, m.vx, f.iPC, 0, (W - 8) << 1);
-    r.py = (double)end_point(y2, m.vy, f.iPC, 0, (H - 8) << 1);
-    r.vx = r.px - r.fx; r.vy = r.py - r.fy;
-    f.bmv[b] = r;
+    const MVs m = s_mb[(i >> 1) * bw16 + (j >> 1)];
+    const double vx = m.px - m.fx, vy = m.py - m.fy;
+    s_blk[b] = MVs{(short)end_point(x2, -vx, f.iFC, 0, (W - 8) << 1), (short)end_point(y2, -vy, f.iFC, 0, (H - 8) << 1),
+                   (short)end_point(x2, vx, f.iPC, 0, (W - 8) << 1), (short)end_point(y2, vy, f.iPC, 0, (H - 8) << 1)};
   }
-  __threadfence_block();
   __syncthreads();
-  bidir_sweep(f, f.bmv, 8);
-  // MSE per 8x8 block (:324-342); integer-valued sums are exact in double
-  for (int b = tid; b < nb8; b += T) {
-    const MVd m = f.bmv[b];
-    const int fy = (int)m.fy, fx = (int)m.fx, py = (int)m.py, px = (int)m.px;
-    double mse = 0.0;
-    for (int a = 0; a < 16; a += 2)
-      for (int q = 0; q < 16; q += 2) {
-        const double d = (double)f.fut_half[(fy + a) * W2 + fx + q] - (double)f.past_half[(py + a) * W2 + px + q];
-        mse += d * d;
-      }
-    f.mse[b] = mse / 64;
-  }
-  __threadfence_block();
-  __syncthreads();
-  // weighted vector-median filter over the 3x3 neighbourhood (:345-405)
-  for (int b = tid; b < nb8; b += T) {
-    const int i = b / bw8, j = b % bw8, y2 = i << 4, x2 = j << 4;
-    int nbr[9], cnt = 0;
-    for (int m = i - 1; m <= i + 1; m++) {
-      if (m < 0 || m >= bh8) continue;
-      for (int q = j - 1; q <= j + 1; q++) {
-        if (q < 0 || q >= bw8) continue;
-        nbr[cnt++] = m * bw8 + q;
-      }
+  bidir_sweep<8>(hp, s_blk);
+  for (int b = tid; b < nb8; b += 1024) f.bmv[b] = s_blk[b];
+}
+
+// motionFilterAndComp (sideInfoCreation.cpp:312-436): weighted vector-median
+// filter over the 3x3 neighbourhood of 8x8 blocks, then motion compensation.
+// One workgroup per 4x4 tile of 8x8 blocks; the tile's and its border's blocks'
+// MSEs first (a lane per row of 8 samples), then 16 lanes per block, one per
+// candidate vector, then a lane per four output pixels.
+constexpr int SF_T = 4, SF_H = SF_T + 2;  // tile side and its side with the border
+__global__ __launch_bounds__(256) void k_si_finish(const FrameDev *F, const int *list) {
+  const FrameDev &f = F[list[blockIdx.y]];
+  const int tid = threadIdx.x, W = f.W, H = f.H, W2 = 2 * W, H2 = 2 * H, bw8 = W / 8, bh8 = H / 8;
+  const int tw = (bw8 + SF_T - 1) / SF_T, th = (bh8 + SF_T - 1) / SF_T;
+  if ((int)blockIdx.x >= tw * th) return;  // uniform over the workgroup
+  const int ti = (blockIdx.x / tw) * SF_T, tj = (blockIdx.x % tw) * SF_T;
+  __shared__ double s_mse[SF_H * SF_H];
+  __shared__ MVs s_mv[SF_H * SF_H], s_new[SF_T * SF_T];
+  __shared__ double s_w[SF_T * SF_T][9];
+  // MSE per 8x8 block (:324-342): the sum of squared integer differences is
+  // exact in double, so it equals the integer sum, formed as sum(a^2) +
+  // sum(b^2) - 2 sum(a*b)
+  for (int t = tid; t < SF_H * SF_H * 8; t += 256) {
+    const int hb = t >> 3, row = t & 7, i = ti - 1 + hb / SF_H, j = tj - 1 + hb % SF_H;
+    if (i < 0 || i >= bh8 || j < 0 || j >= bw8) continue;  // uniform over the block's 8 lanes
+    const MVs m = f.bmv[i * bw8 + j];
+    const uint2 a = even_bytes(f.fut_half + (size_t)(m.fy + 2 * row) * W2 + m.fx);
+    const uint2 b = even_bytes(f.past_half + (size_t)(m.py + 2 * row) * W2 + m.px);
+    uint32_t sq = __builtin_amdgcn_udot4(a.x, a.x, 0u, false), ab = __builtin_amdgcn_udot4(a.x, b.x, 0u, false);
+    sq = __builtin_amdgcn_udot4(a.y, a.y, sq, false);
+    sq = __builtin_amdgcn_udot4(b.x, b.x, sq, false);
+    sq = __builtin_amdgcn_udot4(b.y, b.y, sq, false);
+    ab = __builtin_amdgcn_udot4(a.y, b.y, ab, false);
+    const uint32_t sse = group_sum<8>(sq - 2u * ab);
+    if (row == 0) {
+      s_mse[hb] = (double)(int)sse / 64;
+      s_mv[hb] = m;
     }
-    double minW = 0.0;
-    int best = nbr[0];
-    for (int k = 1; k < cnt; k++) {
-      const double dx = f.bmv[best].vx - f.bmv[nbr[k]].vx, dy = f.bmv[best].vy - f.bmv[nbr[k]].vy;
-      minW += f.mse[best] / f.mse[nbr[k]] * sqrt(dx * dx + dy * dy);
-    }
-    for (int c = 1; c < cnt; c++) {
-      const int cand = nbr[c];
-      double w = 0.0;
-      for (int k = 0; k < cnt; k++) {
-        if (c == k) continue;
-        const double dx = f.bmv[cand].vx - f.bmv[nbr[k]].vx, dy = f.bmv[cand].vy - f.bmv[nbr[k]].vy;
-        w += f.mse[cand] / f.mse[nbr[k]] * sqrt(dx * dx + dy * dy);
-      }
-      if (w < minW) { minW = w; best = cand; }
-    }
-    const double vx = f.bmv[best].vx, vy = f.bmv[best].vy;
-    MVd r;
-    r.fx = (double)end_point(x2, -vx, f.iFC, 0, W2 - 16);
-    r.fy = (double)end_point(y2, -vy, f.iFC, 0, H2 - 16);
-    r.px = (double)end_point(x2, vx, f.iPC, 0, W2 - 16);
-    r.py = (double)end_point(y2, vy, f.iPC, 0, H2 - 16);
-    r.vx = r.px - r.fx; r.vy = r.py - r.fy;
-    f.bmv_tmp[b] = r;
   }
-  __threadfence_block();
   __syncthreads();
-  // motion compensation (:407-434)
-  for (int p = tid; p < W * H; p += T) {
-    const int y = p / W, x = p % W, b = (y >> 3) * bw8 + (x >> 3);
-    const MVd m = f.bmv_tmp[b];
-    const int a = (y & 7) << 1, q = (x & 7) << 1;
-    const int fv = f.fut_half[((int)m.fy + a) * W2 + (int)m.fx + q];
-    const int pv = f.past_half[((int)m.py + a) * W2 + (int)m.px + q];
-    f.si[p] = (uint8_t)(int)((double)fv * f.iFC + (double)pv * f.iPC);
-    f.residue[p] = (fv - pv) >> 1;
+  const int lb = tid >> 4, c = tid & 15, bi = ti + lb / SF_T, bj = tj + lb % SF_T;
+  const bool live = bi < bh8 && bj < bw8;
+  // the block's neighbourhood in raster order: rows r0.., ncol columns from q0
+  const int r0 = imax(0, bi - 1), q0 = imax(0, bj - 1);
+  const int ncol = imin(bw8 - 1, bj + 1) - q0 + 1, cnt = ncol * (imin(bh8 - 1, bi + 1) - r0 + 1);
+  auto nbr = [&](int k) { return (r0 + k / ncol - ti + 1) * SF_H + q0 + k % ncol - tj + 1; };
+  if (live && c < cnt) {
+    const int me = nbr(c);
+    const MVs m = s_mv[me];
+    const double mse = s_mse[me], vx = m.px - m.fx, vy = m.py - m.fy;
+    double w = 0.0;
+    for (int k = 0; k < cnt; k++) {
+      if (c == k) continue;
+      const int o = nbr(k);
+      const MVs n = s_mv[o];
+      const double dx = vx - (n.px - n.fx), dy = vy - (n.py - n.fy);
+      w += mse / s_mse[o] * sqrt(dx * dx + dy * dy);
+    }
+    s_w[lb][c] = w;
   }
-  __threadfence_block();
   __syncthreads();
-  for (int b = tid; b < nb8; b += T) f.bmv[b] = f.bmv_tmp[b];
+  if (live && c == 0) {
+    double minW = s_w[lb][0];
+    int best = 0;
+    for (int k = 1; k < cnt; k++)
+      if (s_w[lb][k] < minW) { minW = s_w[lb][k]; best = k; }
+    const MVs m = s_mv[nbr(best)];
+    const int y2 = bi << 4, x2 = bj << 4;
+    const double vx = m.px - m.fx, vy = m.py - m.fy;
+    s_new[lb] = MVs{(short)end_point(x2, -vx, f.iFC, 0, W2 - 16), (short)end_point(y2, -vy, f.iFC, 0, H2 - 16),
+                    (short)end_point(x2, vx, f.iPC, 0, W2 - 16), (short)end_point(y2, vy, f.iPC, 0, H2 - 16)};
+  }
+  __syncthreads();
+  if (!live) return;
+  // motion compensation (:407-434): pixels 4 * (c & 1) .. of row c >> 1
+  const MVs m = s_new[lb];
+  const int row = c >> 1, x = 4 * (c & 1);
+  uint2 fw, pw;
+  __builtin_memcpy(&fw, f.fut_half + (size_t)(m.fy + 2 * row) * W2 + m.fx + 2 * x, 8);
+  __builtin_memcpy(&pw, f.past_half + (size_t)(m.py + 2 * row) * W2 + m.px + 2 * x, 8);
+  const uint32_t fb = __builtin_amdgcn_perm(fw.y, fw.x, 0x06040200), pb = __builtin_amdgcn_perm(pw.y, pw.x, 0x06040200);
+  uint32_t out = 0;
+  int res[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int fv = (fb >> (8 * q)) & 0xff, pv = (pb >> (8 * q)) & 0xff;
+    out |= (uint32_t)(uint8_t)(int)((double)fv * f.iFC + (double)pv * f.iPC) << (8 * q);
+    res[q] = (fv - pv) >> 1;
+  }
+  const size_t o = (size_t)(8 * bi + row) * W + 8 * bj + x;
+  *(uint32_t *)(f.si + o) = out;
+  *(int4 *)(f.residue + o) = make_int4(res[0], res[1], res[2], res[3]);
 }
 
 // ------------------------------------------------------------ transform helpers
@@ -442,54 +523,128 @@ __constant__ int c_qbits[9][16] = {
 
 // ------------------------------------------------------------ noise parameter
 // forwardTransform of the residue (transform.cpp:153-190) and noiseParameter
-// (noiseModel.cpp:9-75) for one frame per workgroup.  The band means and
-// second moments are float sums over all blocks in raster order, one band per
-// thread, as the reference's loop accumulates them.
-__global__ __launch_bounds__(1024) void k_noise_param(const FrameDev *F, const int *list) {
-  const FrameDev &f = F[list[blockIdx.x]];
-  const int tid = threadIdx.x, T = blockDim.x, W = f.W, N = f.N, bw = W / 4;
-  __shared__ float s_mean[16], s_var[16];
-  __shared__ int s_nbands;
-  for (int b = tid; b < N; b += T) {
-    const int top = (b / bw) * 4, left = (b % bw) * 4;
-    int blk[16];
-    for (int m = 0; m < 4; m++)
-      for (int n = 0; n < 4; n++) blk[4 * m + n] = f.residue[(top + m) * W + left + n];
+// (noiseModel.cpp:9-75).  The reference's band means and second moments are
+// float sums over all blocks in raster order.  Every term is a non-negative
+// integer, so while a total stays at or below 2^24 every partial sum is exact
+// and the float sum equals the integer sum in any order: the coefficients, at
+// most 512 in magnitude for a residue in [-128, 127], always stay there (6336 *
+// 512 < 2^22), their squares do unless the mean square exceeds 2648 (CIF), and
+// only then is the sum taken in order.  Three launches: transform and integer
+// partial sums per 256 blocks, the bands' moments, alpha.  One workgroup per
+// frame with each band's sum on one thread took 955 us for a CIF frame and 205
+// for QCIF, a chain of N dependent loads and additions; now 17 and 15.
+// Per 256 4x4 blocks: sideTrans and the 16 coefficients' partial sums.
+__global__ __launch_bounds__(256) void k_residue_transform(const FrameDev *F, const int *list) {
+  const FrameDev &f = F[list[blockIdx.y]];
+  const int tid = threadIdx.x, W = f.W, bw = W / 4, b0 = blockIdx.x * 256;
+  if (b0 >= f.N) return;  // uniform over the workgroup
+  __shared__ short s_c[256][17];
+  __shared__ uint2 s_part[4][16];
+  const int b = b0 + tid, top = (b / bw) * 4, left = (b % bw) * 4;
+  int blk[16] = {};
+  if (b < f.N) {
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      const int4 v = *(const int4 *)(f.residue + (size_t)(top + m) * W + left);
+      blk[4 * m] = v.x; blk[4 * m + 1] = v.y; blk[4 * m + 2] = v.z; blk[4 * m + 3] = v.w;
+    }
     forward44(blk);
+#pragma unroll
     for (int m = 0; m < 4; m++)
-      for (int n = 0; n < 4; n++) f.sideTrans[(top + m) * W + left + n] = blk[4 * m + n];
+      *(int4 *)(f.sideTrans + (size_t)(top + m) * W + left) =
+          make_int4(blk[4 * m], blk[4 * m + 1], blk[4 * m + 2], blk[4 * m + 3]);
+  }
+#pragma unroll
+  for (int k = 0; k < 16; k++) s_c[tid][k] = (short)abs(blk[k]);
+  __syncthreads();
+  // thread (part, coefficient) sums 16 blocks, then the 4 parts of a wave and
+  // the 4 waves (a workgroup's sums of squares stay below 2^27)
+  const int k = tid & 15, part = tid >> 4;
+  uint32_t s1 = 0, s2 = 0;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const uint32_t c = s_c[part * 16 + i][k];
+    s1 += c;
+    s2 += c * c;
+  }
+  for (int o = 16; o < 64; o <<= 1) {
+    s1 += __shfl_xor(s1, o);
+    s2 += __shfl_xor(s2, o);
+  }
+  if ((tid & 63) < 16) s_part[tid >> 6][k] = make_uint2(s1, s2);
+  __syncthreads();
+  if (tid >= 16) return;
+  for (int w = 1; w < 4; w++) {
+    s1 += s_part[w][k].x;
+    s2 += s_part[w][k].y;
+  }
+  f.npPart[blockIdx.x * 16 + k] = make_uint2(s1, s2);
+}
+// One workgroup per (band, frame): mean and variance of the band's magnitudes.
+__global__ __launch_bounds__(256) void k_noise_moments(const FrameDev *F, const int *list) {
+  const FrameDev &f = F[list[blockIdx.y]];
+  const int tid = threadIdx.x, index = c_zigzag[blockIdx.x], N = f.N, W = f.W, bw = W / 4;
+  if (c_qbits[f.qindex][index] <= 0) return;  // uniform: not one of the frame's bands
+  __shared__ __align__(16) float s_sq[6336 + 64];
+  const int parts = (N + 255) / 256;  // at most 25
+  uint2 p = tid < parts ? f.npPart[tid * 16 + index] : make_uint2(0, 0);
+  uint32_t sq = p.y;  // the squares total at most 6336 * 512^2 < 2^31
+  if (tid < 64)
+    for (int o = 32; o > 0; o >>= 1) {
+      p.x += __shfl_xor(p.x, o);
+      sq += __shfl_xor(sq, o);
+    }
+  float var = (float)sq;
+  // (the first wave holds the totals)
+  const int inOrder = __syncthreads_or(tid < 64 && sq > (1u << 24));
+  if (inOrder) {
+    // the squares past 2^24: their float sum in raster order
+    for (int b = tid; b < N; b += 256) {
+      const float c = (float)f.sideTrans[((b / bw) * 4 + (index >> 2)) * W + (b % bw) * 4 + (index & 3)];
+      s_sq[b] = c * c;
+    }
+    if (tid < 64) s_sq[N + tid] = 0.0f;  // +0 past the last block leaves the sum as it is
+    __syncthreads();
+    if (tid >= 64) return;
+    var = 0.0f;
+    for (int b = 0; b < N; b += 64) {
+      const float4 *q = (const float4 *)(s_sq + b);
+      float4 a[16];
+#pragma unroll
+      for (int i = 0; i < 16; i++) a[i] = q[i];
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        var += a[i].x;
+        var += a[i].y;
+        var += a[i].z;
+        var += a[i].w;
+      }
+    }
   }
   if (tid == 0) {
-    int nb = 0;
-    while (nb < 16 && c_qbits[f.qindex][c_zigzag[nb]] > 0) nb++;
-    s_nbands = nb;
+    const float mean = (float)p.x / (float)N;
+    f.npMom[index] = make_float2(mean, var / (float)N - mean * mean);
   }
-  __threadfence_block();
-  __syncthreads();
-  const int nb = s_nbands;
-  if (tid < nb) {
-    const int index = c_zigzag[tid];
-    float mean = 0.0f, var = 0.0f;
-    for (int b = 0; b < N; b++) {
-      const int top = (b / bw) * 4, left = (b % bw) * 4;
-      const float c = fabsf((float)f.sideTrans[(top + (index >> 2)) * W + left + (index & 3)]);
-      mean += c;
-      var += c * c;
+}
+// alpha of every block at the frame's bands, a thread per 4x4 block.
+__global__ __launch_bounds__(256) void k_noise_alpha(const FrameDev *F, const int *list) {
+  const FrameDev &f = F[list[blockIdx.y]];
+  const int b = blockIdx.x * 256 + threadIdx.x, W = f.W, bw = W / 4;
+  if (b >= f.N) return;
+  const int top = (b / bw) * 4, left = (b % bw) * 4;
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    const size_t o = (size_t)(top + m) * W + left;
+    const int4 v = *(const int4 *)(f.sideTrans + o);
+    const int c4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+      if (c_qbits[f.qindex][4 * m + n] <= 0) continue;  // uniform
+      const float2 mom = f.npMom[4 * m + n];
+      const float dst = (float)abs(c4[n]) - mom.x;
+      const float dst2 = dst * dst;
+      f.alpha[o + n] = dst2 > mom.y ? sqrtf(2 / dst2) : sqrtf(2 / mom.y);
     }
-    mean /= (float)N;
-    var = var / (float)N - mean * mean;
-    s_mean[tid] = mean;
-    s_var[tid] = var;
-  }
-  __syncthreads();
-  for (int e = tid; e < N * nb; e += T) {
-    const int b = e / nb, band = e % nb, index = c_zigzag[band];
-    const int top = (b / bw) * 4, left = (b % bw) * 4;
-    const int ci = (top + (index >> 2)) * W + left + (index & 3);
-    const float c = fabsf((float)f.sideTrans[ci]);
-    const float dst = (float)(int)c - s_mean[band];
-    const float dst2 = dst * dst;
-    f.alpha[ci] = dst2 > s_var[band] ? sqrtf(2 / dst2) : sqrtf(2 / s_var[band]);
   }
 }
 
@@ -1270,17 +1425,22 @@ hipError_t launch_keyframe_batch(const KeyFrameJob *jobs, int n, int maxW, int m
   return hipGetLastError();
 }
 hipError_t launch_create_si(const FrameDev *F, const int *list, int n, int maxMB, CostTables ct, hipStream_t s) {
+  // 4x4 tiles of 8x8 blocks: a CIF frame's 11 x 9, more than a QCIF frame's 6 x 5
+  const int tiles = 99;
   hipLaunchKernelGGL(k_forward_me, dim3(maxMB, n), dim3(256), 0, s, F, list, ct);
-  hipLaunchKernelGGL(k_si_chain, dim3(n), dim3(1024), 0, s, F, list, 0);
+  hipLaunchKernelGGL(k_si_sweep, dim3(n), dim3(1024), 0, s, F, list, 0);
+  hipLaunchKernelGGL(k_si_finish, dim3(tiles, n), dim3(256), 0, s, F, list);
   return hipGetLastError();
 }
 hipError_t launch_forward_me(const FrameDev *F, const int *list, int n, int maxMB, CostTables ct, hipStream_t s) {
   hipLaunchKernelGGL(k_forward_me, dim3(maxMB, n), dim3(256), 0, s, F, list, ct);
-  hipLaunchKernelGGL(k_si_chain, dim3(n), dim3(1024), 0, s, F, list, 1);
+  hipLaunchKernelGGL(k_si_sweep, dim3(n), dim3(1024), 0, s, F, list, 1);
   return hipGetLastError();
 }
-hipError_t launch_noise_param(const FrameDev *F, const int *list, int n, int, hipStream_t s) {
-  hipLaunchKernelGGL(k_noise_param, dim3(n), dim3(1024), 0, s, F, list);
+hipError_t launch_noise_param(const FrameDev *F, const int *list, int n, int maxN, hipStream_t s) {
+  hipLaunchKernelGGL(k_residue_transform, dim3((maxN + 255) / 256, n), dim3(256), 0, s, F, list);
+  hipLaunchKernelGGL(k_noise_moments, dim3(16, n), dim3(256), 0, s, F, list);
+  hipLaunchKernelGGL(k_noise_alpha, dim3((maxN + 255) / 256, n), dim3(256), 0, s, F, list);
   return hipGetLastError();
 }
 hipError_t launch_oct(const FrameDev *F, const int *list, int n, int maxPos, int initSideTrans, hipStream_t s) {
