@@ -1047,18 +1047,21 @@ __global__ void k_inverse_transform(const FrameDev *F, const int *list) {
 // sweeps candidate column sL+l down the window, forming each candidate's
 // 4-pixel rows with v_alignbyte and its SAD with v_sad_u8 (exact integer SADs,
 // as the reference's double sums of integer differences are).  A lane keeps
-// its best cost and the row it was found on (the row is wave-uniform, so the
-// select takes it from a scalar register); the rows above the block and the
-// rows from the block down run as two loops, so the cost factor's LDS address
-// steps by a constant.  The 65th column of a full window is spread over the
-// lanes afterwards.  Ties resolve to the first candidate in raster order: the
-// wave's minimum cost first, then the least (row, column) key among the lanes
-// that hold it.
-// A cost (double)sad * fac is formed as fma(2^52 + sad, fac, -2^52 * fac): the
-// double with high word 0x43300000 and low word sad is 2^52 + sad exactly, the
-// fused product-sum is sad * fac before its one rounding, and -2^52 * fac is
-// exact, so the result has the bits of the rounded product (sad = 0 gives +0
-// both ways) without a conversion.
+// its best cost only; the rows above the block and the rows from the block down
+// run as two loops, so the cost factor's LDS address steps by a constant.  The
+// 65th column of a full window is spread over the lanes.  The VALU issue port
+// bounds the loop, so the candidate itself is found afterwards: the wave's
+// least cost, then the columns that hold it (nearly always one), then, a lane
+// per row, the first row of such a column with that cost.  Ties resolve to the
+// first candidate in raster order: the least (row, column) key.
+// A cost (double)sad * fac is the product of two doubles: the one whose bits
+// are the integer sad, which is the subnormal sad * 2^-1074, and fac * 2^1000
+// from the table.  The product is sad * fac * 2^-74, far inside the normal
+// range, so it has the rounded product's mantissa without a conversion, and all
+// costs carry the same scale.
+// Tracking the row of each lane's best and forming a cost as fma(2^52 + sad,
+// fac, -2^52 * fac), the loop took 19.5 VALU instructions per candidate row of
+// both frames, 8 of them SADs; now 14.5 (2421 and 2079 us for 128 CIF frames).
 #define USI_LW 21   // staged words per window row: 20 + one zero word
 #define USI_ROWS 68
 __device__ __forceinline__ uint32_t usi_word(const uint32_t *R, int r, int j, int sh) {
@@ -1077,18 +1080,9 @@ __device__ __forceinline__ double dmin_num(double a, double b) {
   __asm__("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
   return r;
 }
-__device__ __forceinline__ void argmin_take(double c, int i, double &best, int &bi) {
-  if (c < best || (c == best && i < bi)) { best = c; bi = i; }
-}
-// (cost, key) -> the wave's least cost and, among the lanes holding it, the
-// least key; every lane gets both.  Costs are finite or DBL_MAX, never NaN.
-__device__ __forceinline__ void wave_argmin_key(double &cost, int &key) {
-  double m = cost;
+__device__ __forceinline__ double wave_min(double m) {  // numbers only
   for (int o = 32; o > 0; o >>= 1) m = dmin_num(m, __shfl_xor(m, o));
-  int k = cost == m ? key : 0x7fffffff;
-  for (int o = 32; o > 0; o >>= 1) k = imin(k, __shfl_xor(k, o));
-  cost = m;
-  key = k;
+  return m;
 }
 __global__ __launch_bounds__(256) void k_update_si(const FrameDev *F, const int *list, CostTables ct) {
   const FrameDev &f = F[list[blockIdx.y]];
@@ -1097,7 +1091,7 @@ __global__ __launch_bounds__(256) void k_update_si(const FrameDev *F, const int 
   if (b0 >= f.N) return;  // uniform over the workgroup
   const int W = f.W, H = f.H, W2 = 2 * W, H2 = 2 * H, bw = W / 4;
   __shared__ uint32_t s_win[USI_ROWS * 2 * USI_LW];  // [row][past, future][word]
-  __shared__ double s_fac[33 * 33];  // by (|dy|, |dx|)
+  __shared__ double s_fac[33 * 33];  // by (|dy|, |dx|), times 2^1000
   // union window of the 4 blocks: rows [wT, wB], byte columns [cL, cR]
   const int row0 = (b0 / bw) * 4, left0 = (b0 % bw) * 4;
   const int wT = imax(0, row0 - 32), wB = imin(H - 4, row0 + 32) + 3;
@@ -1113,7 +1107,7 @@ __global__ __launch_bounds__(256) void k_update_si(const FrameDev *F, const int 
         dst[r * 2 * USI_LW + w] = w < nw ? *(const uint32_t *)(src + (size_t)(wT + r) * W + cL + 4 * w) : 0u;
     }
     for (int dy = wave; dy < 33; dy += 4)
-      if (lane < 33) s_fac[dy * 33 + lane] = ct.usi[(dy + 32) * 65 + lane + 32];
+      if (lane < 33) s_fac[dy * 33 + lane] = ct.usi[(dy + 32) * 65 + lane + 32] * 0x1p1000;
   }
   __syncthreads();
   const int b = b0 + wave;
@@ -1126,30 +1120,22 @@ __global__ __launch_bounds__(256) void k_update_si(const FrameDev *F, const int 
   for (int m = 0; m < 4; m++) bk[m] = *(const uint32_t *)(f.recons + (size_t)(top + m) * W + left);
   const uint32_t *P = s_win, *Fu = s_win + USI_LW;
   double pBest = DBL_MAX, fBest = DBL_MAX;
-  int pKey = 0x7fffffff, fKey = 0x7fffffff;  // (row - sT) * 128 + column - sL
   if (lane < ww) {
     const int x = sL + lane, xo = x - cL, j = xo >> 2, sh = xo & 3;
     const double *facCol = s_fac + abs(x - left);
-    int r = sT - wT, pRow = 0, fRow = 0;
+    int r = sT - wT;
     uint32_t p0 = usi_word(P, r, j, sh), p1 = usi_word(P, r + 1, j, sh), p2 = usi_word(P, r + 2, j, sh);
     uint32_t f0 = usi_word(Fu, r, j, sh), f1 = usi_word(Fu, r + 1, j, sh), f2 = usi_word(Fu, r + 2, j, sh);
-    // the high words of 2^52 + sad, one register per frame so that each SAD
-    // can land in the low half of its own pair
-    int hiP = 0x43300000, hiF = 0x43300000;
+    // the zero high words of the SADs' doubles, one register per frame so that
+    // each SAD can land in the low half of its own pair
+    int hiP = 0, hiF = 0;
     __asm__ volatile("" : "+v"(hiP));
     __asm__ volatile("" : "+v"(hiF));
-    auto step = [&](int yr, double fac) {
+    auto step = [&](double fac) {
       const uint32_t p3 = usi_word(P, r + 3, j, sh), f3 = usi_word(Fu, r + 3, j, sh);
       const uint32_t ps = sad4(bk, p0, p1, p2, p3), fs = sad4(bk, f0, f1, f2, f3);
-      const double facn = fac * -4503599627370496.0;  // -2^52 fac
-      const double pc = fma(__hiloint2double(hiP, (int)ps), fac, facn);
-      const double fc = fma(__hiloint2double(hiF, (int)fs), fac, facn);
-      // costs are positive and never NaN: the running minimum is a plain
-      // v_min_f64, and only the row needs the strict comparison
-      pRow = pc < pBest ? yr : pRow;
-      fRow = fc < fBest ? yr : fRow;
-      pBest = dmin_num(pBest, pc);
-      fBest = dmin_num(fBest, fc);
+      pBest = dmin_num(pBest, __hiloint2double(hiP, (int)ps) * fac);
+      fBest = dmin_num(fBest, __hiloint2double(hiF, (int)fs) * fac);
       p0 = p1; p1 = p2; p2 = p3;
       f0 = f1; f1 = f2; f2 = f3;
       r++;
@@ -1159,39 +1145,67 @@ __global__ __launch_bounds__(256) void k_update_si(const FrameDev *F, const int 
     // table upwards from the lowest of their entries (LDS offsets are positive)
     const double *lo = facCol + 33 * (top - sT - 3);
     for (; y + 4 <= top; y += 4, lo -= 4 * 33) {
-      step(y - sT, lo[99]);
-      step(y + 1 - sT, lo[66]);
-      step(y + 2 - sT, lo[33]);
-      step(y + 3 - sT, lo[0]);
+      step(lo[99]);
+      step(lo[66]);
+      step(lo[33]);
+      step(lo[0]);
     }
-    for (; y < top; y++) step(y - sT, facCol[33 * (top - y)]);
+    for (; y < top; y++) step(facCol[33 * (top - y)]);
     const double *fp = facCol;  // rows from the block down: |y - top| rises
     for (; y + 4 <= sB + 1; y += 4, fp += 4 * 33) {
-      step(y - sT, fp[0]);
-      step(y + 1 - sT, fp[33]);
-      step(y + 2 - sT, fp[66]);
-      step(y + 3 - sT, fp[99]);
+      step(fp[0]);
+      step(fp[33]);
+      step(fp[66]);
+      step(fp[99]);
     }
-    for (; y <= sB; y++, fp += 33) step(y - sT, *fp);
-    pKey = pRow * 128 + lane;
-    fKey = fRow * 128 + lane;
+    for (; y <= sB; y++, fp += 33) step(*fp);
   }
+  // the cost of candidate (row, column) relative to (sT, sL) on frame R
+  auto cost_at = [&](const uint32_t *R, int row, int col) {
+    const int x = sL + col, xo = x - cL, j = xo >> 2, sh = xo & 3, r = sT + row - wT;
+    const uint32_t sad = sad4(bk, usi_word(R, r, j, sh), usi_word(R, r + 1, j, sh), usi_word(R, r + 2, j, sh),
+                              usi_word(R, r + 3, j, sh));
+    return __hiloint2double(0, (int)sad) * s_fac[33 * abs(sT + row - top) + abs(x - left)];
+  };
+  // column sL+64 of a full window: row `lane`, and row 64 on lane 0
+  double pCol[2] = {DBL_MAX, DBL_MAX}, fCol[2] = {DBL_MAX, DBL_MAX};
   if (ww > 64) {
-    // column sL+64: one candidate row per lane
-    const int x = sL + 64, xo = x - cL, j = xo >> 2, sh = xo & 3;
-    for (int i = lane; i < nr; i += 64) {
-      const int y = sT + i, r = y - wT;
-      const uint32_t ps = sad4(bk, usi_word(P, r, j, sh), usi_word(P, r + 1, j, sh), usi_word(P, r + 2, j, sh),
-                               usi_word(P, r + 3, j, sh));
-      const uint32_t fs = sad4(bk, usi_word(Fu, r, j, sh), usi_word(Fu, r + 1, j, sh), usi_word(Fu, r + 2, j, sh),
-                               usi_word(Fu, r + 3, j, sh));
-      const double fac = s_fac[33 * abs(y - top) + abs(x - left)];
-      argmin_take((double)ps * fac, i * 128 + 64, pBest, pKey);
-      argmin_take((double)fs * fac, i * 128 + 64, fBest, fKey);
-    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      if (lane + 64 * h < nr) {
+        pCol[h] = cost_at(P, lane + 64 * h, 64);
+        fCol[h] = cost_at(Fu, lane + 64 * h, 64);
+      }
   }
-  wave_argmin_key(pBest, pKey);
-  wave_argmin_key(fBest, fKey);
+  // first candidate in raster order of the wave's least cost: (row << 7) + column
+  auto locate = [&](const uint32_t *R, double best, const double *col64) -> int {
+    const double m = wave_min(dmin_num(best, dmin_num(col64[0], col64[1])));
+    int key = 0x7fffffff;
+    const uint64_t e0 = __ballot(col64[0] == m), e1 = __ballot(col64[1] == m);
+    if (e0 | e1) key = ((e0 ? __builtin_ctzll(e0) : 64) << 7) + 64;
+    uint64_t cols = __ballot(best == m);
+    if (__popcll(cols) <= 4) {
+      // a lane per row of each column; row 64 only when no earlier row matches
+      for (; cols; cols &= cols - 1) {
+        const int col = __builtin_ctzll(cols);
+        const uint64_t rows = __ballot(lane < nr && cost_at(R, imin(lane, nr - 1), col) == m);
+        key = imin(key, ((rows ? __builtin_ctzll(rows) : 64) << 7) + col);
+      }
+    } else {
+      // many columns (flat contents): each looks down its own rows, and the
+      // first row that any of them matches holds the least key
+      const bool mine = best == m;
+      for (int row = 0; row < nr && (row << 7) < key; row++) {
+        const uint64_t hit = __ballot(mine && cost_at(R, row, imin(lane, ww - 1)) == m);
+        if (hit) {
+          key = imin(key, (row << 7) + __builtin_ctzll(hit));
+          break;
+        }
+      }
+    }
+    return key;
+  };
+  const int pKey = locate(P, pBest, pCol), fKey = locate(Fu, fBest, fCol);
   const int pbx = sL + (pKey & 127), pby = sT + (pKey >> 7), fbx = sL + (fKey & 127), fby = sT + (fKey >> 7);
   // subPelRefine: lanes 0-8 evaluate the 9 positions of the past frame, 16-24 the future
   const int which = lane >> 4, pos = lane & 15;
