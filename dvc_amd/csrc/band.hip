@@ -147,7 +147,7 @@ extern "C" int dvc_band_frame_init(dvc_ctx *c, int W, int H, int qindex, const u
                oOct = take((size_t)64 * (W - 3) * (H - 3)),
                oOb = take((size_t)4 * (W - 3) * (H - 3)), oSmf = take((size_t)4 * 81 * N),
                oSmfRef = take(sizeof(dvc_smf) * (size_t)N), oLR = take(4 * (size_t)N), oFd = take(sizeof(FrameDev)),
-               oList = take(sizeof(int)), oBlk = take(sizeof(int) * (size_t)N), oMode = take((size_t)n8);
+               oSpan = take(sizeof(int2) * (size_t)N), oList = take(sizeof(int)), oBlk = take(sizeof(int) * (size_t)N), oMode = take((size_t)n8);
   if ((rc = grow(&B->mem, &B->bytes, off))) return rc;
   uint8_t *m = B->mem;
   FrameDev &f = B->fd;
@@ -159,6 +159,7 @@ extern "C" int dvc_band_frame_init(dvc_ctx *c, int W, int H, int qindex, const u
   f.past_half = m + oPh; f.fut_half = m + oFh;
   f.si = m + oSi; f.recons = m + oRec; f.reconsTrans = (int *)(m + oRt); f.alpha = (float *)(m + oAl);
   f.oct = (int *)(m + oOct); f.octBand = (int *)(m + oOb); f.smf = (float *)(m + oSmf); f.LR = (float *)(m + oLR);
+  f.distSpan = (int2 *)(m + oSpan);
   B->smfRef = (dvc_smf *)(m + oSmfRef);
   B->d_blk = (int *)(m + oBlk);
   B->nsir = nsir;
@@ -206,7 +207,7 @@ extern "C" int dvc_noise_distribution(dvc_ctx *c, int range, int index, const fl
   f.index = index; f.range = range; f.distStride = stride; f.dist = B->dist;
   if ((rc = upload_fd(c, B))) return rc;
   DVC_HIP(launch_oct_plane(B->d_fd, B->d_list, 1, (W - 3) * (H - 3), index, s));
-  DVC_HIP(launch_noise_dist(B->d_fd, B->d_list, 1, N, stride, s));
+  DVC_HIP(launch_noise_dist(B->d_fd, B->d_list, 1, N, 1, s));
   if (dist && ns == N) {
     DVC_HIP(hipMemcpyAsync(dist, B->dist, need, hipMemcpyDeviceToHost, s));
   } else if (dist && ns > 0) {  // SIR entries only, in their order

@@ -139,7 +139,7 @@ static size_t job_bytes(const Job &j) {
   size_t t = 0;
   for (size_t b : {(size_t)FS, 4 * (size_t)FS, 4 * (size_t)FS, 4 * (size_t)FS, 4 * (size_t)FS,
                    (size_t)64 * (W - 3) * (H - 3), (size_t)4 * (W - 3) * (H - 3), (size_t)4 * 81 * N, (size_t)4 * N * std::max(maxStride, 1),
-                   4 * (size_t)N, (size_t)N, (size_t)FS, sizeof(MVs) * (size_t)(FS / 64),
+                   sizeof(int2) * (size_t)N, 4 * (size_t)N, (size_t)N, (size_t)FS, sizeof(MVs) * (size_t)(FS / 64),
                    sizeof(MVd) * (size_t)(FS / 256), 16 * (size_t)(FS / 256), np_part_bytes(N), kNpMomBytes,
                    (size_t)j.nbp * (N / 8),
                    sizeof(PlaneState) * (size_t)j.nbp, sizeof(int4) * kMaxCodes * (size_t)j.nbp, 4 * (size_t)N,
@@ -160,7 +160,7 @@ static void carve_job(Job &j, uint8_t *base) {
   const size_t o_si = take(FS), o_res = take(4 * (size_t)FS), o_st = take(4 * (size_t)FS), o_rt = take(4 * (size_t)FS),
                o_al = take(4 * (size_t)FS), o_oct = take((size_t)64 * (W - 3) * (H - 3)),
                o_ob = take((size_t)4 * (W - 3) * (H - 3)), o_smf = take((size_t)4 * 81 * N),
-               o_dist = take((size_t)4 * N * std::max(maxStride, 1)), o_lr = take(4 * (size_t)N), o_dec = take(N),
+               o_dist = take((size_t)4 * N * std::max(maxStride, 1)), o_span = take(sizeof(int2) * (size_t)N), o_lr = take(4 * (size_t)N), o_dec = take(N),
                o_rec = take(FS), o_bmv = take(sizeof(MVs) * (size_t)(FS / 64)),
                o_fwd = take(sizeof(MVd) * (size_t)(FS / 256)), o_holes = take(16 * (size_t)(FS / 256)),
                o_npp = take(np_part_bytes(N)), o_npm = take(kNpMomBytes),
@@ -176,7 +176,7 @@ static void carve_job(Job &j, uint8_t *base) {
   f.si = base + o_si; f.residue = (int *)(base + o_res); f.sideTrans = (int *)(base + o_st);
   f.reconsTrans = (int *)(base + o_rt); f.alpha = (float *)(base + o_al); f.oct = (int *)(base + o_oct);
   f.octBand = (int *)(base + o_ob);
-  f.smf = (float *)(base + o_smf); f.dist = (float *)(base + o_dist); f.LR = (float *)(base + o_lr);
+  f.smf = (float *)(base + o_smf); f.dist = (float *)(base + o_dist); f.distSpan = (int2 *)(base + o_span); f.LR = (float *)(base + o_lr);
   f.decoded = base + o_dec; f.recons = base + o_rec; f.bmv = (MVs *)(base + o_bmv);
   f.fwd = (MVd *)(base + o_fwd); f.holes = (double *)(base + o_holes);
   f.npPart = (uint2 *)(base + o_npp); f.npMom = (float2 *)(base + o_npm);
@@ -729,9 +729,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
   }
   if (!active.empty()) {
     if (!starting.empty()) {
-      int maxStride = 0;
-      for (int i : starting) maxStride = std::max(maxStride, ln.inflight[i]->fd.distStride);
-      TIMED_LAUNCH(c, "noise_dist", s, launch_noise_dist(ln.d_frames, L1, (int)starting.size(), maxN, maxStride, s));
+      TIMED_LAUNCH(c, "noise_dist", s, launch_noise_dist(ln.d_frames, L1, (int)starting.size(), maxN, 0, s));
     }
     // the step's kernels: conditional bit probabilities, LDPCA per code
     // length, bitplane insertion

@@ -53,6 +53,8 @@ struct FrameDev {
                              // whose noise distribution comes next
   float *smf;                // N*81 statistical motion field probabilities
   float *dist;               // N*distStride noise distribution of the current band
+  int2 *distSpan;            // N: [first, end) of a row's values outside which all are +0 (and not stored, see
+                             // launch_noise_dist)
   int distStride;            // range (DC) or 2*range+1 (AC)
   float *LR;                 // N likelihood ratios of the current bitplane
   uint8_t *decoded;          // N decoded bits of the current bitplane
@@ -95,7 +97,8 @@ hipError_t launch_forward_me(const FrameDev *F, const int *list, int n, int maxM
 hipError_t launch_oct_plane(const FrameDev *F, const int *list, int n, int maxPos, int index, hipStream_t s);
 hipError_t launch_noise_param(const FrameDev *F, const int *list, int n, int maxN, hipStream_t s);
 hipError_t launch_oct(const FrameDev *F, const int *list, int n, int maxPos, int initSideTrans, hipStream_t s);
-hipError_t launch_noise_dist(const FrameDev *F, const int *list, int n, int maxN, int maxStride, hipStream_t s);
+// fill: store the zeros outside each block's span as well (readers of whole rows).
+hipError_t launch_noise_dist(const FrameDev *F, const int *list, int n, int maxN, int fill, hipStream_t s);
 hipError_t launch_condbit(const FrameDev *F, const int *list, int n, int maxN, hipStream_t s);
 struct BpFrameLink;
 hipError_t launch_put_bitplane(const FrameDev *F, const int *list, const BpFrameLink *links, int n, int maxN,

@@ -43,6 +43,19 @@ __device__ __forceinline__ double cost_func(double mad, double x, double y) {
   return mad * (1.0 + (double)DVC_K * sqrt(x * x + y * y));
 }
 
+// op over the wave's 64 values, for min, max and the like (op(x, x) = x), by
+// data-parallel moves: within rows of 16 lanes, then across rows to lane 63.
+template <class Op>
+__device__ __forceinline__ int wave_reduce(int v, Op op) {
+  v = op(v, __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, false));   // quad_perm [1, 0, 3, 2]
+  v = op(v, __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, false));   // quad_perm [2, 3, 0, 1]
+  v = op(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, false));  // row_half_mirror
+  v = op(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xf, 0xf, false));  // row_mirror
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1 and 3
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2 and 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // Lexicographic (cost, index) minimum across a wave: the first candidate in
 // scan order among those of least cost, which is what a strict-< raster scan
 // returns.
@@ -751,8 +764,23 @@ __global__ void k_smf_init(const FrameDev *F, const int *list) {
 // per (4x4 block, frame): a block has 2*range+1 <= ~520 values at most
 // Qindex 8, and the small workgroup with a 4 KB table lets a CU hold many
 // blocks at once to hide the LDS and global latencies of each one's phases.
+// A value is +0 where every term's expf underflows, a*d > 104, which for the
+// usual a around 1 leaves most of the range zero (a DC row has 1024 values, an
+// AC row up to about 1000).  The block's span is the interval outside which
+// all values are +0: only it is computed and, for the frame decoder, stored;
+// condBitProb's sums are clipped to it, as adding +0 changes none of them.
+// With every value computed and stored, a band of 256 CIF frames took 2237 us on
+// average (the DC band 3417); now 2124 (2883).  The rest is the sums' products
+// and additions, 8 of the 9 VALU instructions per term and four values.
 #define ND_TAB 1024  // table entries (4 KB of LDS); larger distances call expf directly
 #define ND_T 64      // threads per block distribution (one wave)
+// The least distance from which expf(-a * d) is certainly +0 (it is below
+// -103.98, and the quotient's and product's roundings stay within the slack),
+// or 2^20 where no distance is taken to be.
+__device__ __forceinline__ int nd_reach(float a) {
+  const float q = 104.0f / a;
+  return a > 0.0f && q < 1048000.0f ? (int)q + 2 : 1 << 20;
+}
 // V values k + i*ND_T (i < V) of one block's distribution: sum over the window
 // terms m in order of p_m * tab[value + off_m].  Values at or beyond rmax are
 // computed from the table's padding (never from outside it) and not stored.
@@ -772,55 +800,72 @@ __device__ __forceinline__ void nd_values(const float *tab, const int2 *ps, int 
   for (int i = 0; i < V; i++)
     if (k + i * ND_T < rmax) out[k + i * ND_T] = acc[i];
 }
-__global__ __launch_bounds__(64) void k_noise_dist(const FrameDev *F, const int *list) {
+// fill: also store the zeros outside the span (callers that read whole rows).
+__global__ __launch_bounds__(64) void k_noise_dist(const FrameDev *F, const int *list, int fill) {
   const FrameDev &f = F[list[blockIdx.y]];
   const int b = blockIdx.x;
   if (b >= f.N || !wz_block(f, b)) return;  // only SIR candidates have a distribution
   const int tid = threadIdx.x, T = ND_T;
   const int ow = f.W - 3, index = f.index, range = f.range;
+  const int rmax = index ? 2 * range + 1 : range;  // values of the row
   const SmfWin s = smf_window(f, b);
   const float a = f.alpha[(s.top + (index >> 2)) * f.W + s.left + (index & 3)];
   float *out = f.dist + (size_t)b * f.distStride;
+  int reach = nd_reach(a);
+  auto put_span = [&](int lo, int hi) {  // [lo, hi) within [0, rmax], possibly empty
+    if (tid == 0) f.distSpan[b] = make_int2(lo, hi);
+    if (!fill) return;
+    for (int k = tid; k < lo; k += T) out[k] = 0.0f;
+    for (int k = hi + tid; k < rmax; k += T) out[k] = 0.0f;
+  };
   if (index == 0) {
     const int side = f.octBand[s.top * ow + s.left];
-    for (int k = tid; k < range; k += T) out[k] = dvc_expf(-a * (float)abs(k - side));
+    const int lo = imin(rmax, imax(0, side - reach + 1)), hi = imax(lo, imin(rmax, side + reach));
+    put_span(lo, hi);
+    for (int k = lo + tid; k < hi; k += T) out[k] = dvc_expf(-a * (float)abs(k - side));
     return;
   }
   __shared__ int2 s_ps[81];  // (probability bits, SI coefficient) of the kept window terms
-  __shared__ int s_n, s_maxabs;
   // table entries [0, 2D] with 2D + 1 <= ND_TAB, and 3 * ND_T of padding that a
-  // lane's values beyond rmax (at most 3 * ND_T further on) may read
+  // lane's values beyond the span (at most 3 * ND_T further on) may read
   __shared__ float s_tab[ND_TAB + 3 * ND_T];
-  if (tid < 64) {
-    // wave 0 compacts the window's non-zero terms in raster order
-    const bool fin = isfinite(a);
-    int n = 0, mx = 0;
-    for (int base = 0; base < s.len; base += 64) {
-      const int p = base + tid;
-      float pr = 0.0f;
-      bool keep = false;
-      if (p < s.len) {
-        pr = f.smf[(size_t)81 * b + p];
-        keep = !(fin && pr == 0.0f);
-      }
-      const unsigned long long mask = __ballot(keep);
-      if (keep) {
-        const int pos = n + __popcll(mask & ((1ull << tid) - 1ull));
-        const int m = s.sT + p / s.w, q = s.sL + p % s.w;
-        const int sd = f.octBand[m * ow + q];
-        s_ps[pos] = make_int2(__float_as_int(pr), sd);
-        mx = imax(mx, abs(sd));
-      }
-      n += __popcll(mask);
+  // compact the window's non-zero terms in raster order
+  const bool fin = isfinite(a);
+  const float rw = __builtin_amdgcn_rcpf((float)s.w);
+  int n = 0, mn = 0x7fffffff, mx = -0x7fffffff;
+  bool odd = false;  // some kept probability is not finite: it makes NaN of the zeros
+  for (int base = 0; base < s.len; base += 64) {
+    const int p = base + tid;
+    float pr = 0.0f;
+    bool keep = false;
+    if (p < s.len) {
+      pr = f.smf[(size_t)81 * b + p];
+      keep = !(fin && pr == 0.0f);
     }
-    for (int o = 32; o > 0; o >>= 1) mx = imax(mx, __shfl_xor(mx, o));
-    if (tid == 0) { s_n = n; s_maxabs = mx; }
+    const unsigned long long mask = __ballot(keep);
+    if (keep) {
+      const int pos = n + __popcll(mask & ((1ull << tid) - 1ull));
+      const int m = (int)(((float)p + 0.5f) * rw);  // p / s.w, at least 0.5 / 9 from rounding over
+      const int sd = f.octBand[(s.sT + m) * ow + s.sL + p - m * s.w];
+      s_ps[pos] = make_int2(__float_as_int(pr), sd);
+      mn = imin(mn, sd);
+      mx = imax(mx, sd);
+      odd |= !isfinite(pr);
+    }
+    n += __popcll(mask);
   }
-  __syncthreads();
-  const int n = s_n;
-  // |k - range - SI_m| <= range + max|SI_m| = D for k in [0, 2*range]
-  const int D = range + s_maxabs;
-  const int rmax = 2 * range + 1;
+  mn = wave_reduce(mn, [](int x, int y) { return imin(x, y); });
+  mx = wave_reduce(mx, [](int x, int y) { return imax(x, y); });
+  if (n == 0) {
+    put_span(0, 0);
+    return;
+  }
+  if (__ballot(odd)) reach = 1 << 20;
+  const int lo = imin(rmax, imax(0, range + mn - reach + 1)), hi = imax(lo, imin(rmax, range + mx + reach));
+  put_span(lo, hi);
+  // |k - range - SI_m| for k in the span: within it by reach + (mx - mn), and in
+  // any case by range + max|SI_m|
+  const int D = imin(range + imax(abs(mn), abs(mx)), reach + mx - mn);
   if (2 * D + 1 <= ND_TAB) {
     // two-sided table s_tab[D + t] = expf(-a*|t|), t in [-D, D]: term m of
     // value k reads s_tab[k + off_m] with off_m = D - range - SI_m
@@ -829,22 +874,23 @@ __global__ __launch_bounds__(64) void k_noise_dist(const FrameDev *F, const int 
       s_tab[D + d] = v;
       s_tab[D - d] = v;
     }
+    __syncthreads();
     for (int m = tid; m < n; m += T) s_ps[m].y = D - range - s_ps[m].y;
     __syncthreads();
     // a lane's values k, k + T, ... share each term's offset and carry
     // independent sums; each value still adds its terms in window order.  The
     // number of values per lane is the same on every lane (groups of up to 4).
-    int k = tid, left = (rmax + T - 1) / T;
-    for (; left >= 4; left -= 4, k += 4 * T) nd_values<4>(s_tab, s_ps, n, k, rmax, out);
-    if (left == 3) nd_values<3>(s_tab, s_ps, n, k, rmax, out);
-    else if (left == 2) nd_values<2>(s_tab, s_ps, n, k, rmax, out);
-    else if (left == 1) nd_values<1>(s_tab, s_ps, n, k, rmax, out);
+    int k = lo + tid, left = (hi - lo + T - 1) / T;
+    for (; left >= 4; left -= 4, k += 4 * T) nd_values<4>(s_tab, s_ps, n, k, hi, out);
+    if (left == 3) nd_values<3>(s_tab, s_ps, n, k, hi, out);
+    else if (left == 2) nd_values<2>(s_tab, s_ps, n, k, hi, out);
+    else if (left == 1) nd_values<1>(s_tab, s_ps, n, k, hi, out);
   } else {
     const int need = D + 1;
     const int tl = imin(need, ND_TAB);
     for (int d = tid; d < tl; d += T) s_tab[d] = dvc_expf(-a * (float)d);
     __syncthreads();
-    for (int k = tid; k < rmax; k += T) {
+    for (int k = lo + tid; k < hi; k += T) {
       const int pc = k - range;
       float sum = 0.0f;
       for (int m = 0; m < n; m++) {
@@ -860,96 +906,99 @@ __global__ __launch_bounds__(64) void k_noise_dist(const FrameDev *F, const int 
 
 // ------------------------------------------------------------ conditional bit probability
 // condBitProb (noiseModel.cpp:191-310): interval sums in ascending k, p0/(p0+p1),
-// clipped likelihood ratio.  One wave per 64 blocks: the wave stages the span
-// of each block's two intervals through LDS in chunks of 32 values (each load
-// a coalesced 128-byte piece of one block's distribution row), and each lane
-// then adds its own block's values in ascending k, as the reference's loops do.
+// clipped likelihood ratio.  Two lanes per block, one per interval, each adding
+// its own interval's values in ascending k, as the reference's loops do, clipped
+// to the block's span (the values outside are +0).  The wave stages the 64
+// intervals through LDS in chunks of C values (each load a contiguous piece of
+// two intervals), the next chunk's loads issued before this chunk is summed.
+// HBM bounds a large batch, the chain of chunks a single frame: with a lane per
+// block adding both intervals of the whole row, a launch for one CIF frame took
+// 21 us on average and up to 128, for 256 frames 199; now 9.5, 37 and 172.
+template <int C>
+__device__ __forceinline__ float interval_sum(const float *dist, size_t stride, const int2 *iv, float *v, int lane,
+                                              int span) {
+  constexpr int R = 64 / C, LD = C + 4;  // rows per load; row length in LDS, 16-byte aligned
+  const int i = lane % C, jr = lane / C;
+  float nxt[C];
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int l = 0; l < C; l++) {
+      const int j = l * R + jr;
+      const int2 r = iv[j];
+      const int k = r.x + c0 + i;
+      nxt[l] = k < r.y ? dist[(size_t)(j >> 1) * stride + k] : 0.0f;
+    }
+  };
+  float sum = 0.0f;
+  if (span > 0) fetch(0);
+  for (int c0 = 0; c0 < span; c0 += C) {
+#pragma unroll
+    for (int l = 0; l < C; l++) v[(l * R + jr) * LD + i] = nxt[l];
+    __syncthreads();
+    if (c0 + C < span) fetch(c0 + C);
+    const float4 *q = (const float4 *)(v + lane * LD);
+#pragma unroll
+    for (int t = 0; t < C / 4; t++) {
+      // past the interval's end the values are +0, which changes no sum
+      const float4 x = q[t];
+      sum += x.x;
+      sum += x.y;
+      sum += x.z;
+      sum += x.w;
+    }
+    __syncthreads();
+  }
+  return sum;
+}
 __global__ __launch_bounds__(64) void k_condbit(const FrameDev *F, const int *list) {
   const FrameDev &f = F[list[blockIdx.y]];
   const int lane = threadIdx.x;
-  const int b0 = blockIdx.x * 64;
+  const int b0 = blockIdx.x * 32;
   if (b0 >= f.N) return;  // uniform over the wave
-  __shared__ float s_v[64 * 33];
-  __shared__ int s_lo[64], s_hi[64];
-  const int b = b0 + lane;
+  __shared__ __align__(16) float s_v[64 * 36];
+  __shared__ int2 s_iv[64];
+  const int b = b0 + (lane >> 1), one = lane & 1;
   const bool valid = b < f.N;
   const bool wz = valid && wz_block(f, b);  // condBitProb walks the SIR's WZ blocks
-  int v0l = 0, v0u = 0, v1l = 0, v1u = 0;
+  int lo = 0, hi = 0;
   if (wz) {
     const int bw = f.W / 4, top = (b / bw) * 4, left = (b % bw) * 4;
     const int index = f.index, bit = f.bit, step = f.step, range = f.range;
     const int iq = (1 << (bit - 1)) - 1;
     const int rc = f.reconsTrans[(top + (index >> 2)) * f.W + left + (index & 3)];
-    int lim;
+    // the quantisation indices of bit value `one`
+    int ql = one ? ((rc << 1) + 1) << (bit - 1) : rc << bit;
     if (index == 0) {
-      const int q0l = rc << bit, q1l = ((rc << 1) + 1) << (bit - 1);
-      const int q0u = q0l + iq, q1u = q1l + iq;
-      v0l = q0l * step; v1l = q1l * step; v0u = (q0u + 1) * step; v1u = (q1u + 1) * step;
-      lim = range;
+      lo = ql * step;
+      hi = (ql + iq + 1) * step;
     } else {
       const int ls = f.levelShift;
-      const int q0l = (rc << bit) - ls, q1l = (((rc << 1) + 1) << (bit - 1)) - ls;
-      const int q0u = q0l + iq;
-      int q1u = q1l + iq;
-      if (q1u > ls) q1u = ls;
-      v0l = (q0l <= 0) ? (q0l - 1) * step + 1 : q0l * step;
-      v1l = (q1l <= 0) ? (q1l - 1) * step + 1 : q1l * step;
-      v0u = (q0u < 0) ? q0u * step + 1 : (q0u + 1) * step;
-      v1u = (q1u < 0) ? q1u * step + 1 : (q1u + 1) * step;
-      v0l += range; v0u += range; v1l += range; v1u += range;
-      lim = 2 * range + 1;
+      ql -= ls;
+      int qu = ql + iq;
+      if (one && qu > ls) qu = ls;
+      lo = ((ql <= 0) ? (ql - 1) * step + 1 : ql * step) + range;
+      hi = ((qu < 0) ? qu * step + 1 : (qu + 1) * step) + range;
     }
-    v0l = imax(v0l, 0); v1l = imax(v1l, 0); v0u = imin(v0u, lim); v1u = imin(v1u, lim);
+    const int2 sp = f.distSpan[b];  // within [0, values of the row]
+    lo = imax(lo, sp.x);
+    hi = imin(hi, sp.y);
   }
-  // the span read for this block: [lo, hi) covers both (non-empty) intervals
-  int lo = 0, hi = 0;
-  if (v0u > v0l) { lo = v0l; hi = v0u; }
-  if (v1u > v1l) {
-    lo = hi > lo ? imin(lo, v1l) : v1l;
-    hi = imax(hi, v1u);
-  }
-  s_lo[lane] = lo;
-  s_hi[lane] = hi;
-  int span = hi - lo;
-  for (int o = 32; o > 0; o >>= 1) span = imax(span, __shfl_xor(span, o));
+  s_iv[lane] = make_int2(lo, hi);
+  const int span = wave_reduce(imax(0, hi - lo), [](int x, int y) { return imax(x, y); });
   __syncthreads();
-  const size_t stride = f.distStride;
-  float p0 = 0.0f, p1 = 0.0f;
-  // chunk c0 of every block's span, 32 values per block: lane (j parity,
-  // i) fetches value i of blocks jj + (lane >> 5); the next chunk's loads are
-  // issued before this chunk is summed
-  float nxt[32];
-  auto fetch = [&](int c0) {
-#pragma unroll
-    for (int jj = 0; jj < 64; jj += 2) {
-      const int j = jj + (lane >> 5), i = lane & 31;
-      const int k = s_lo[j] + c0 + i;
-      nxt[jj >> 1] = (b0 + j < f.N && k < s_hi[j]) ? f.dist[(size_t)(b0 + j) * stride + k] : 0.0f;
-    }
-  };
-  if (span > 0) fetch(0);
-  for (int c0 = 0; c0 < span; c0 += 32) {
-#pragma unroll
-    for (int jj = 0; jj < 64; jj += 2) s_v[(jj + (lane >> 5)) * 33 + (lane & 31)] = nxt[jj >> 1];
-    __syncthreads();
-    if (c0 + 32 < span) fetch(c0 + 32);
-    for (int i = 0; i < 32; i++) {
-      const int k = lo + c0 + i;
-      const float v = s_v[lane * 33 + i];
-      if (k >= v0l && k < v0u) p0 += v;
-      if (k >= v1l && k < v1u) p1 += v;
-    }
-    __syncthreads();
-  }
-  if (!valid) return;
+  const float *dist = f.dist + (size_t)b0 * f.distStride;
+  // short intervals (the lower bits) load in pieces of 16 values
+  const float mine = span <= 16 ? interval_sum<16>(dist, f.distStride, s_iv, s_v, lane, span)
+                                : interval_sum<32>(dist, f.distStride, s_iv, s_v, lane, span);
+  const float other = __shfl_xor(mine, 1);
+  if (!valid || one) return;
   if (!wz) {
     // the frame's LR are first set to 0.9999f / 0.0001f when it has skip or
     // intra blocks (DVC_Decoder.cpp:203-207); WZ blocks overwrite theirs
     f.LR[b] = 0.9999f / 0.0001f;
     return;
   }
-  p0 = p0 / (p0 + p1);
-  p1 = 1 - p0;
+  const float p0 = mine / (mine + other), p1 = 1 - p0;
   float lr;
   if ((double)p0 <= 0.0001) lr = (float)(0.0001 / 0.9999);
   else if ((double)p0 >= 0.9999) lr = (float)(0.9999 / 0.0001);
@@ -1482,13 +1531,12 @@ hipError_t launch_oct_plane(const FrameDev *F, const int *list, int n, int maxPo
   hipLaunchKernelGGL(k_oct_plane, dim3((maxPos + 255) / 256, n), dim3(256), 0, s, F, list, index);
   return hipGetLastError();
 }
-hipError_t launch_noise_dist(const FrameDev *F, const int *list, int n, int maxN, int maxStride, hipStream_t s) {
-  (void)maxStride;  // one wave per block whatever the band's value count
-  hipLaunchKernelGGL(k_noise_dist, dim3(maxN, n), dim3(ND_T), 0, s, F, list);
+hipError_t launch_noise_dist(const FrameDev *F, const int *list, int n, int maxN, int fill, hipStream_t s) {
+  hipLaunchKernelGGL(k_noise_dist, dim3(maxN, n), dim3(ND_T), 0, s, F, list, fill);
   return hipGetLastError();
 }
 hipError_t launch_condbit(const FrameDev *F, const int *list, int n, int maxN, hipStream_t s) {
-  hipLaunchKernelGGL(k_condbit, dim3((maxN + 63) / 64, n), dim3(64), 0, s, F, list);
+  hipLaunchKernelGGL(k_condbit, dim3((maxN + 31) / 32, n), dim3(64), 0, s, F, list);
   return hipGetLastError();
 }
 hipError_t launch_put_bitplane(const FrameDev *F, const int *list, const BpFrameLink *links, int n, int maxN,
