@@ -1387,7 +1387,6 @@ __global__ __launch_bounds__(256) void k_update_smf(const FrameDev *F, const int
 // already decoded are summed too but not stored.  A window row's weights are
 // loaded three per lane by the four lanes of a block column and passed
 // between them with quad permutes.
-#define ML_ROWS 8
 #define ML_COLS 16  // block columns per wave
 template <int L>
 __device__ __forceinline__ float quad_bcast(float v) {
@@ -1402,6 +1401,7 @@ __device__ __forceinline__ float quad_bcast(float v, int l) {  // l is a constan
     default: return quad_bcast<3>(v);
   }
 }
+template <int ML_ROWS>
 __global__ __launch_bounds__(256) void k_update_si_ml(const FrameDev *F, const int *list) {
   const FrameDev &f = F[list[blockIdx.y]];
   const int bandStart = f.band + 1;  // update_si_ML(..., band+1, ...) (DVC_Decoder.cpp:369)
@@ -1564,9 +1564,22 @@ hipError_t launch_update_smf(const FrameDev *F, const int *list, int n, int maxN
   hipLaunchKernelGGL(k_update_smf, dim3((maxN + 3) / 4, n), dim3(256), 0, s, F, list);
   return hipGetLastError();
 }
+template <int ML_ROWS>
+static void launch_ml(const FrameDev *F, const int *list, int n, int colTiles, int maxBh, hipStream_t s) {
+  const int tiles = colTiles * ((maxBh + ML_ROWS - 1) / ML_ROWS);
+  hipLaunchKernelGGL((k_update_si_ml<ML_ROWS>), dim3((tiles + 3) / 4, n), dim3(256), 0, s, F, list);
+}
 hipError_t launch_update_si_ml(const FrameDev *F, const int *list, int n, int maxBw, int maxBh, hipStream_t s) {
-  const int tiles = (maxBw + ML_COLS - 1) / ML_COLS * ((maxBh + ML_ROWS - 1) / ML_ROWS);
-  hipLaunchKernelGGL(k_update_si_ml, dim3((tiles + 3) / 4, n), dim3(256), 0, s, F, list);
+  // Block rows per wave: eight read the least (4.6 position rows per block row,
+  // against 5.3 for four and 9 for one), but a wave walks its 37 rows one after
+  // another, so while eight-row waves do not fill the chip's 1024 SIMDs shorter
+  // walks win.  us for 1, 8, 24, 64 and 128 CIF frames (54 eight-row waves each):
+  // one row 24, 35, 111, 307, 596; four 59, 62, 95, 257, 490; eight 105, 108,
+  // 143, 238, 463.
+  const int colTiles = (maxBw + ML_COLS - 1) / ML_COLS, waves8 = n * colTiles * ((maxBh + 7) / 8);
+  if (waves8 <= 1024) launch_ml<1>(F, list, n, colTiles, maxBh, s);
+  else if (waves8 <= 2560) launch_ml<4>(F, list, n, colTiles, maxBh, s);
+  else launch_ml<8>(F, list, n, colTiles, maxBh, s);
   return hipGetLastError();
 }
 
