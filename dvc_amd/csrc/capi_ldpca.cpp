@@ -250,18 +250,21 @@ static int ldpca_workspace(dvc_ctx *c, size_t devBytes, size_t hostBytes) {
 }
 
 // Shared driver for one group of bitplanes with the same code length.
-// sequential != 0: one code per launch in increasing order (the plain path,
-// which mirrors the reference's per-code beliefPropagation_CUDA call).
+// sequential != 0 (n = 1): the codes one after another in increasing order, the
+// plain search.  In ParallelMode 0 that is one launch of a single workgroup,
+// which takes the codes in order and stops at the first accepted one; with a
+// launch and a read-back per code, a QCIF bitplane of 4 codes took 10% longer (1.8
+// against 1.63 ms), a CIF one of 9 codes 5%.  ParallelMode 1
+// launches each code by itself with the decisions the one before it left.
 // ParallelMode 1: items[i].decoded holds the decisions carried into the
 // bitplane's first code on entry (the reference's in/out decoded buffer).
 static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int sequential, hipStream_t s) {
   Ladder *L = c->ladder(N);
   const int C = L->numCodes, nb = N / 8;
   const bool mode1 = c->bp_mode == 1;
-  // slots: each (bitplane, code) accepts at most once; ParallelMode 1 keeps
-  // every run code's decisions and its repeat-case decisions as well
-  const int slotCap = sequential ? (mode1 ? 2 * C + 2 : 2) : (mode1 ? 2 * C * n + 1 : C * n + 1);
-  const LdpcaLayout o = ldpca_layout(n, N, C, slotCap, mode1);
+  const bool perCode = sequential && mode1;
+  const SlotPlan slots = slot_plan(n, C, c->bp_mode);
+  const LdpcaLayout o = ldpca_layout(n, N, C, slots.total, mode1);
   int rc = ldpca_workspace(c, o.total, o.outEnd);
   if (rc) return rc;
   uint8_t *dev = (uint8_t *)c->ld_dev, *host = (uint8_t *)c->ld_host;
@@ -289,11 +292,10 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     hState[i] = PlaneState{st0 >= 0 ? st0 : -1, C - 1, 0.0f, 0, 0};
     for (int l = 0; l < C; l++) hRec[(size_t)i * C + l] = make_int4(0, REC_NOT_RUN, -1, 0);
   }
-  hCounters[0] = hCounters[1] = hCounters[2] = 0;
   DVC_HIP(hipMemcpyAsync(dev, host, o.inEnd, hipMemcpyHostToDevice, s));
-  TIMED(c, "ce_llr", s, launch_ce_llr(dPlanes, n, 1, c->lad1584, c->lad6336, s));
+  TIMED(c, "ce_llr", s, launch_ce_llr(dPlanes, n, 1, c->lad1584, c->lad6336, dCounters, s));
   std::vector<PlaneState> state(n);
-  if (sequential) {
+  if (perCode) {
     DVC_HIP(hipMemcpyAsync(state.data(), dState, sizeof(PlaneState) * n, hipMemcpyDeviceToHost, s));
     DVC_HIP(hipStreamSynchronize(s));
   }
@@ -301,19 +303,17 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
   const int threads = bp_threads(c, N);
   LadderDev ld = ladder_dev(*L);
   std::vector<int4> rec((size_t)n * C);
-  if (sequential) {
-    // Plain path: bitplane by bitplane, one code per launch, each with the
-    // decisions the previous code left (ParallelMode 1).
+  if (perCode) {
+    // one code per launch, each with the decisions the previous code left
     for (int i = 0; i < n; i++) {
       int level = state[i].start;
       int4 r;
-      for (; level < C - 1;
-           level = c->rate_step ? std::min(C - 1, state[i].start + dynstep_next(level - state[i].start)) : level + 1) {
+      for (; level < C - 1; level++) {
         PlaneState ps{state[i].start, C - 1, state[i].entropy, level, state[i].taint};
         int zero[3] = {0, 0, 0};
         DVC_HIP(hipMemcpyAsync(dState + i, &ps, sizeof(ps), hipMemcpyHostToDevice, s));
         DVC_HIP(hipMemcpyAsync(dCounters, zero, sizeof(zero), hipMemcpyHostToDevice, s));
-        BpArgs a{ld, dPlanes + i, 1, dCounters, 1, 1, c->max_iter, dSlots, dCounters + 1, slotCap, c->bp_poll,
+        BpArgs a{ld, dPlanes + i, 1, dCounters, 1, 1, c->max_iter, dSlots, dCounters + 1, slots.bp, c->bp_poll,
                  c->bp_mode, c->rate_step};
         TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, 1, s));
         DVC_HIP(hipMemcpyAsync(&r, dRec + (size_t)i * C + level, sizeof(r), hipMemcpyDeviceToHost, s));
@@ -322,17 +322,13 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
           DVC_HIP(hipMemcpy(items[i].decoded, dSlots + (size_t)r.z * N, N, hipMemcpyDeviceToHost));
           break;
         }
-        if (mode1) {
-          DVC_CHECK(r.z >= 0 && r.z < slotCap, DVC_ESTATE, "dvc_ldpca: missing decisions of a failed code");
-          DVC_HIP(hipMemcpyAsync(dCarry + (size_t)i * N, dSlots + (size_t)r.z * N, N, hipMemcpyDeviceToDevice, s));
-        }
+        DVC_CHECK(r.z >= 0 && r.z < slots.bp, DVC_ESTATE, "dvc_ldpca: missing decisions of a failed code");
+        DVC_HIP(hipMemcpyAsync(dCarry + (size_t)i * N, dSlots + (size_t)r.z * N, N, hipMemcpyDeviceToDevice, s));
       }
       if (level == C - 1) {
         PlaneState ps{state[i].start, C - 1, state[i].entropy, C, state[i].taint};
-        int zero[3] = {0, 0, 0};
         DVC_HIP(hipMemcpyAsync(dState + i, &ps, sizeof(ps), hipMemcpyHostToDevice, s));
-        DVC_HIP(hipMemcpyAsync(dCounters, zero, sizeof(zero), hipMemcpyHostToDevice, s));
-        TIMED(c, "invh", s, launch_invh(dPlanes + i, 1, ld, dSlots, dCounters + 1, slotCap, s));
+        TIMED(c, "invh", s, launch_invh(dPlanes + i, 1, ld, dSlots, slots.bp, s));
         DVC_HIP(hipMemcpyAsync(&r, dRec + (size_t)i * C + (C - 1), sizeof(r), hipMemcpyDeviceToHost, s));
         DVC_HIP(hipStreamSynchronize(s));
         DVC_HIP(hipMemcpy(items[i].decoded, dSlots + (size_t)r.z * N, N, hipMemcpyDeviceToHost));
@@ -341,38 +337,38 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     DVC_HIP(hipMemcpy(rec.data(), dRec, sizeof(int4) * rec.size(), hipMemcpyDeviceToHost));
   } else {
     const int maxOff = C - 1;
-    BpArgs a{ld, dPlanes, n, dCounters, n * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, slotCap,
+    BpArgs a{ld, dPlanes, n, dCounters, n * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, slots.bp,
              c->bp_poll, c->bp_mode, c->rate_step};
-    const int grid = bp_grid(c, N, n * maxOff);
+    const int grid = sequential ? 1 : bp_grid(c, N, n * maxOff);
     TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, grid, s));
     for (int round = 0; mode1; round++) {
       // ParallelMode 1: resolve with the carried decisions; resume the
       // bitplanes that reach a code this launch did not finish
       DVC_CHECK(round <= C, DVC_ESTATE, "dvc_ldpca: ParallelMode 1 resolution does not settle");
       DVC_HIP(launch_zero_ints(dCounters + 2, 1, s));
-      DVC_HIP(launch_mode1_resolve(dPlanes, n, C, N, dSlots, slotCap, dCounters + 2, s));
+      DVC_HIP(launch_mode1_resolve(dPlanes, n, C, N, dSlots, slots.bp, dCounters + 2, s));
       int resume = 0;
       DVC_HIP(hipMemcpyAsync(&resume, dCounters + 2, sizeof(int), hipMemcpyDeviceToHost, s));
       DVC_HIP(hipStreamSynchronize(s));
       DVC_CHECK(resume < (1 << 20), DVC_ENOMEM, "ParallelMode 1: decision slots exhausted");
-    if (!resume) break;
+      if (!resume) break;
       DVC_HIP(launch_zero_ints(dCounters, 1, s));
       TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, grid, s));
     }
-    TIMED(c, "invh", s, launch_invh(dPlanes, n, ld, dSlots, dCounters + 1, slotCap, s));
+    TIMED(c, "invh", s, launch_invh(dPlanes, n, ld, dSlots, slots.bp, s));
     // every bitplane's accepted decisions to dOut, then states, records,
     // counters and decisions back in one copy
-    DVC_HIP(launch_gather_accepted(dPlanes, n, N, dSlots, slotCap, dOut, s));
+    DVC_HIP(launch_gather_accepted(dPlanes, n, N, dSlots, slots.total, dOut, s));
     DVC_HIP(hipMemcpyAsync(host + o.state, dev + o.state, o.outEnd - o.state, hipMemcpyDeviceToHost, s));
     DVC_HIP(hipStreamSynchronize(s));
-    DVC_CHECK(hCounters[1] <= slotCap, DVC_ENOMEM, "dvc_ldpca_decode_batch: decision slots exhausted");
+    DVC_CHECK(hCounters[1] <= slots.bp, DVC_ENOMEM, "dvc_ldpca_decode_batch: decision slots exhausted");
     memcpy(state.data(), hState, sizeof(PlaneState) * n);
     memcpy(rec.data(), hRec, sizeof(int4) * rec.size());
     for (int i = 0; i < n; i++) {
       const int best = state[i].best;
       DVC_CHECK(best >= 0 && best < C, DVC_ESTATE, "dvc_ldpca_decode_batch: bad accepted code");
       const int4 r = rec[(size_t)i * C + best];
-      DVC_CHECK(r.y == REC_ACCEPTED && r.z >= 0 && r.z < slotCap, DVC_ESTATE,
+      DVC_CHECK(r.y == REC_ACCEPTED && r.z >= 0 && r.z < slots.total, DVC_ESTATE,
                 "dvc_ldpca_decode_batch: missing accepted record");
       memcpy(items[i].decoded, host + o.out + (size_t)i * N, N);
     }

@@ -224,62 +224,69 @@ int ensure_cost_tables(dvc_ctx *c) {
     (c)->timer_end(slot_, ev_, s);                               \
   } while (0)
 
-// One bitplane step of LDPCA decoding for the planes of one code length.
-int bp_step(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, bool sequential, uint8_t *d_slots, int slotCap,
-            int *d_counters, PlaneDesc *d_planes, hipStream_t s);
-// The speculative step's launches alone (the plane descriptors already in
-// d_planes): entropy and LLR, counters, the persistent BP launch and the
-// full-rate inverse.  Kernel launches only, so a stream capture of it replays.
-int bp_step_launch(dvc_ctx *c, int N, int n, uint8_t *d_slots, int slotCap, int *d_counters, PlaneDesc *d_planes,
-                   hipStream_t s);
+// One bitplane step of LDPCA decoding for the n planes of one code length (their
+// descriptors in d_planes): entropy and LLR, the persistent BP launch and the
+// full-rate inverse.  In ParallelMode 0 these are kernel launches only, so a
+// stream capture of them replays.  sequential: the plain search, a launch of one
+// workgroup per bitplane, which takes the codes one after another.
+int bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, uint8_t *d_slots, const SlotPlan &slots,
+                   int *d_counters, PlaneDesc *d_planes, hipStream_t s);
+// The plain search in ParallelMode 1: a launch per code, each with the decisions
+// the code before it left.
+int bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, uint8_t *d_slots, const SlotPlan &slots,
+                  int *d_counters, PlaneDesc *d_planes, hipStream_t s);
 }  // namespace dvc
 
-int dvc::bp_step_launch(dvc_ctx *c, int N, int n, uint8_t *d_slots, int slotCap, int *d_counters, PlaneDesc *d_planes,
-                        hipStream_t s) {
+int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, uint8_t *d_slots, const SlotPlan &slots,
+                        int *d_counters, PlaneDesc *d_planes, hipStream_t s) {
   Ladder *L = c->ladder(N);
   const int C = L->numCodes;
   LadderDev ld = ladder_dev(*L);
   const int threads = bp_threads(c, N);
   const int maxOff = C - 1;
-  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, s));
-  DVC_HIP(launch_zero_ints(d_counters, 3, s));
-  BpArgs a{ld, d_planes, n, d_counters, n * maxOff, maxOff, c->max_iter, d_slots, d_counters + 1, slotCap, c->bp_poll,
+  const char *name = N == 6336 ? "bp_6336" : "bp_1584";
+  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
+  BpArgs a{ld, d_planes, n, d_counters, n * maxOff, maxOff, c->max_iter, d_slots, d_counters + 1, slots.bp, c->bp_poll,
            c->bp_mode, c->rate_step};
-  const int grid = bp_grid(c, N, n * maxOff);
-  TIMED_LAUNCH(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, grid, s));
-  for (int round = 0; c->bp_mode == 1; round++) {
-    // ParallelMode 1: resolve with the carried decisions and resume the
-    // bitplanes that reach a code the launch did not finish (host-synchronous)
-    DVC_CHECK(round <= C, DVC_ESTATE, "ParallelMode 1 resolution does not settle");
-    DVC_HIP(launch_zero_ints(d_counters + 2, 1, s));
-    DVC_HIP(launch_mode1_resolve(d_planes, n, C, N, d_slots, slotCap, d_counters + 2, s));
-    int resume = 0;
-    DVC_HIP(hipMemcpyAsync(&resume, d_counters + 2, sizeof(int), hipMemcpyDeviceToHost, s));
-    DVC_HIP(hipStreamSynchronize(s));
-    DVC_CHECK(resume < (1 << 20), DVC_ENOMEM, "ParallelMode 1: decision slots exhausted");
-    if (!resume) break;
-    DVC_HIP(launch_zero_ints(d_counters, 1, s));
-    TIMED_LAUNCH(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, grid, s));
+  if (sequential) {
+    a.nplanes = 1;
+    a.total = maxOff;
+    for (int i = 0; i < n; i++) {
+      if (i) DVC_HIP(launch_zero_ints(d_counters, 1, s));  // queue head only: the step's slots accumulate
+      a.planes = d_planes + i;
+      TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, 1, s));
+    }
+  } else {
+    const int grid = bp_grid(c, N, n * maxOff);
+    TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, grid, s));
+    for (int round = 0; c->bp_mode == 1; round++) {
+      // ParallelMode 1: resolve with the carried decisions and resume the
+      // bitplanes that reach a code the launch did not finish (host-synchronous)
+      DVC_CHECK(round <= C, DVC_ESTATE, "ParallelMode 1 resolution does not settle");
+      DVC_HIP(launch_zero_ints(d_counters + 2, 1, s));
+      DVC_HIP(launch_mode1_resolve(d_planes, n, C, N, d_slots, slots.bp, d_counters + 2, s));
+      int resume = 0;
+      DVC_HIP(hipMemcpyAsync(&resume, d_counters + 2, sizeof(int), hipMemcpyDeviceToHost, s));
+      DVC_HIP(hipStreamSynchronize(s));
+      DVC_CHECK(resume < (1 << 20), DVC_ENOMEM, "ParallelMode 1: decision slots exhausted");
+      if (!resume) break;
+      DVC_HIP(launch_zero_ints(d_counters, 1, s));
+      TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, grid, s));
+    }
   }
-  TIMED_LAUNCH(c, "invh", s, launch_invh(d_planes, n, ld, d_slots, d_counters + 1, slotCap, s));
+  TIMED_LAUNCH(c, "invh", s, launch_invh(d_planes, n, ld, d_slots, slots.bp, s));
   return DVC_OK;
 }
 
-int dvc::bp_step(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, bool sequential, uint8_t *d_slots,
-                 int slotCap, int *d_counters, PlaneDesc *d_planes, hipStream_t s) {
+int dvc::bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, uint8_t *d_slots,
+                       const SlotPlan &slots, int *d_counters, PlaneDesc *d_planes, hipStream_t s) {
   Ladder *L = c->ladder(N);
   const int n = (int)planes.size(), C = L->numCodes;
-  if (n == 0) return DVC_OK;
   LadderDev ld = ladder_dev(*L);
   const int threads = bp_threads(c, N);
-  DVC_HIP(hipMemcpyAsync(d_planes, planes.data(), sizeof(PlaneDesc) * n, hipMemcpyHostToDevice, s));
-  if (!sequential) return bp_step_launch(c, N, n, d_slots, slotCap, d_counters, d_planes, s);
-  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, s));
-  // Plain path: per bitplane, one code per launch in increasing order, with
-  // the host deciding the next code (the reference's beliefPropagation_CUDA loop).
+  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
   // Every host-side source below stays alive until the stream is drained.
   std::vector<PlaneState> st(n);
-  DVC_HIP(hipMemsetAsync(d_counters, 0, 2 * sizeof(int), s));
   for (int i = 0; i < n; i++)
     DVC_HIP(hipMemcpyAsync(&st[i], planes[i].state, sizeof(PlaneState), hipMemcpyDeviceToHost, s));
   DVC_HIP(hipStreamSynchronize(s));
@@ -288,31 +295,27 @@ int dvc::bp_step(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, bool s
     bool ok = false;
     PlaneState ps;
     int4 r;
-    for (; level < C - 1;
-         level = c->rate_step ? std::min(C - 1, st[i].start + dynstep_next(level - st[i].start)) : level + 1) {
+    for (; level < C - 1; level++) {
       ps = PlaneState{st[i].start, C - 1, st[i].entropy, level, st[i].taint};
       DVC_HIP(hipMemcpyAsync(planes[i].state, &ps, sizeof(ps), hipMemcpyHostToDevice, s));
-      DVC_HIP(hipMemsetAsync(d_counters, 0, sizeof(int), s));  // queue head only: the step's slots accumulate
-      BpArgs a{ld, d_planes + i, 1, d_counters, 1, 1, c->max_iter, d_slots, d_counters + 1, slotCap, c->bp_poll,
+      DVC_HIP(launch_zero_ints(d_counters, 1, s));  // queue head only: the step's slots accumulate
+      BpArgs a{ld, d_planes + i, 1, d_counters, 1, 1, c->max_iter, d_slots, d_counters + 1, slots.bp, c->bp_poll,
                c->bp_mode, c->rate_step};
       TIMED_LAUNCH(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, 1, s));
       DVC_HIP(hipMemcpyAsync(&r, planes[i].rec + level, sizeof(r), hipMemcpyDeviceToHost, s));
       DVC_HIP(hipStreamSynchronize(s));
       if (r.y == REC_ACCEPTED) { ok = true; break; }
-      if (c->bp_mode == 1) {
-        // the failed code's decisions are carried into the next code
-        DVC_CHECK(r.z >= 0 && r.z < slotCap, DVC_ESTATE, "missing decisions of a failed code");
-        DVC_HIP(hipMemcpyAsync(planes[i].carry, d_slots + (size_t)r.z * N, N, hipMemcpyDeviceToDevice, s));
-      }
+      // the failed code's decisions are carried into the next code
+      DVC_CHECK(r.z >= 0 && r.z < slots.bp, DVC_ESTATE, "missing decisions of a failed code");
+      DVC_HIP(hipMemcpyAsync(planes[i].carry, d_slots + (size_t)r.z * N, N, hipMemcpyDeviceToDevice, s));
     }
     ps = PlaneState{st[i].start, ok ? level : C - 1, st[i].entropy, C, st[i].taint};
     DVC_HIP(hipMemcpyAsync(planes[i].state, &ps, sizeof(ps), hipMemcpyHostToDevice, s));
-    if (!ok) TIMED_LAUNCH(c, "invh", s, launch_invh(d_planes + i, 1, ld, d_slots, d_counters + 1, slotCap, s));
+    if (!ok) TIMED_LAUNCH(c, "invh", s, launch_invh(d_planes + i, 1, ld, d_slots, slots.bp + i, s));
     DVC_HIP(hipStreamSynchronize(s));
   }
   return DVC_OK;
 }
-
 
 // ---------------------------------------------------------------- engine
 namespace dvc {
@@ -331,7 +334,8 @@ struct KeyEntry {
 // lanes' kernels.
 struct Lane {
   hipStream_t s = nullptr;
-  int cap = 0, groupCap = 0;
+  int cap = 0;
+  SlotPlan slots{};  // decision slots of each code length
   std::vector<Job *> inflight;
   std::vector<Job *> finished;  // retired by the engine after the step
   // A step's descriptors, written to one pinned host block and uploaded to
@@ -676,7 +680,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
                  m1 ? j.d_bcase + (size_t)kMaxCodes * j.bp : nullptr};
     ln.groups[j.N == 6336].push_back(pd);
     ln.h_links[a] = BpFrameLink{j.d_state + j.bp, j.d_rec + (size_t)kMaxCodes * j.bp,
-                                ln.d_slots + (size_t)(j.N == 6336 ? ln.groupCap : 0) * 6336, ln.groupCap,
+                                ln.d_slots + (size_t)(j.N == 6336 ? ln.slots.total : 0) * 6336, ln.slots.total,
                                 m1 ? j.d_carry : nullptr};
   }
   const int na = (int)active.size(), n0 = (int)ln.groups[0].size(), n1 = (int)ln.groups[1].size();
@@ -739,12 +743,12 @@ static int lane_step(dvc_engine *e, Lane &ln) {
       for (int g = 0; g < 2; g++) {
         const int ng = g ? n1 : n0;
         if (!ng) continue;
-        uint8_t *slots = ln.d_slots + (size_t)(g ? ln.groupCap : 0) * 6336;
-        const int r = e->sequentialBp
-                          ? bp_step(c, g ? 6336 : 1584, ln.groups[g], true, slots, ln.groupCap, ln.d_counters + 3 * g,
-                                    ln.d_planes + off, s)
-                          : bp_step_launch(c, g ? 6336 : 1584, ng, slots, ln.groupCap, ln.d_counters + 3 * g,
-                                           ln.d_planes + off, s);
+        uint8_t *slots = ln.d_slots + (size_t)(g ? ln.slots.total : 0) * 6336;
+        const int r = e->sequentialBp && c->bp_mode == 1
+                          ? bp_step_codes(c, g ? 6336 : 1584, ln.groups[g], slots, ln.slots, ln.d_counters + 3 * g,
+                                          ln.d_planes + off, s)
+                          : bp_step_launch(c, g ? 6336 : 1584, ng, e->sequentialBp, slots, ln.slots,
+                                           ln.d_counters + 3 * g, ln.d_planes + off, s);
         if (r) return r;
         off += ng;
       }
@@ -752,7 +756,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
       return DVC_OK;
     };
     // (ParallelMode 1 steps read a resolution count back, so they are not captured)
-    const bool steady = e->graphs && !e->sequentialBp && !c->profiling && c->bp_mode == 0 && setup.empty() &&
+    const bool steady = e->graphs && !c->profiling && c->bp_mode == 0 && setup.empty() &&
                         starting.empty() && ending.empty();
     if (steady) {
       const auto key = std::make_tuple(na, n0, n1, maxN);
@@ -822,7 +826,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
     for (size_t k = 0; k < fin.size(); k++) {
       Job &j = *ln.inflight[fin[k]];
       DVC_CHECK(j.setup && j.done(), DVC_ESTATE, "engine: a finishing frame has bands left");
-      if ((rc = finish_job(e, j, ln.h_out + outOff[k], ln.groupCap))) return rc;
+      if ((rc = finish_job(e, j, ln.h_out + outOff[k], ln.slots.total))) return rc;
     }
     std::vector<Job *> keep;
     for (int i = 0; i < n; i++) {
@@ -990,7 +994,7 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
   for (int k = 0; k < nl && err == hipSuccess; k++) {
     Lane &l = e->lanes[k];
     l.cap = (e->maxInflight + nl - 1) / nl;
-    l.groupCap = (c->bp_mode == 1 ? 2 * kMaxCodes : kMaxCodes) * l.cap + 1;  // ParallelMode 1 keeps two decision sets per code
+    l.slots = slot_plan(l.cap, kMaxCodes, c->bp_mode);
     const size_t M = l.cap;
     const size_t oFrames = 0, oLists = align_up(oFrames + sizeof(FrameDev) * M), oLinks = align_up(oLists + sizeof(int) * 5 * M),
                  oPlanes = align_up(oLinks + sizeof(BpFrameLink) * M), oSegs = align_up(oPlanes + sizeof(PlaneDesc) * M),
@@ -1007,7 +1011,7 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
       l.h_planes = (PlaneDesc *)(l.h_stage + oPlanes); l.d_planes = (PlaneDesc *)(l.d_stage + oPlanes);
       l.h_segs = (CopySeg *)(l.h_stage + oSegs); l.d_segs = (CopySeg *)(l.d_stage + oSegs);
     }
-    if (err == hipSuccess) err = hipMalloc((void **)&l.d_slots, (size_t)2 * l.groupCap * 6336);
+    if (err == hipSuccess) err = hipMalloc((void **)&l.d_slots, (size_t)2 * l.slots.total * 6336);
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_counters, 6 * sizeof(int));
   }
   if (err != hipSuccess) {

@@ -92,14 +92,17 @@ __device__ __forceinline__ uint32_t acc_bit(gbyte_t *acc, int i) {
 // and 8.7 (sums of 16 terms with the next 16 read meanwhile: 34 and 12).
 #define DVC_LOG2 (0.693147181f)
 constexpr int CE_T = 1024, CE_CHUNK = CE_T - 64;  // a multiple of 64
+// It also clears the step's launch counters (a kernel's store, so that a captured
+// step holds no memset).
 __global__ __launch_bounds__(CE_T) void ce_llr_kernel(const PlaneDesc *planes, int nplanes, int fixed_start,
                                                       const float *codeRate1584, const float *codeRate6336,
-                                                      int numCodes1584, int numCodes6336) {
+                                                      int numCodes1584, int numCodes6336, int *counters) {
   __shared__ __align__(16) float terms[6336 + 64];  // spare: the last group of 64
   const int p = blockIdx.x;
   if (p >= nplanes) return;
   const PlaneDesc d = planes[p];
   const int N = d.N, tid = threadIdx.x;
+  if (p == 0 && tid < 3) counters[tid] = 0;
   int nan = 0;
   float rlb = 0.0f;
   if (tid < 64) terms[N + tid] = 0.0f;
@@ -562,17 +565,9 @@ __global__ __launch_bounds__(64) void mode1_resolve_kernel(const PlaneDesc *plan
 
 // ------------------------------------------------------------------ full rate
 // invH_mul (LdpcaDecoder.cpp:624-643) for every bitplane whose BP codes all
-// failed, in two launches: invh_slot_kernel gives each such bitplane its
-// decision slot (one thread per bitplane), then invh_kernel multiplies.
-
-__global__ void invh_slot_kernel(const PlaneDesc *planes, int nplanes, int numCodes, int *slot_count) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nplanes) return;
-  const PlaneDesc d = planes[p];
-  if (d.state->best < numCodes - 1) return;
-  d.rec[numCodes - 1] = make_int4(0, REC_ACCEPTED, atomicAdd(slot_count, 1), 1);
-}
-
+// failed.  Bitplane p's product goes to decision slot slot0 + p, a range the BP
+// launches do not hand out, so the bitplanes that need one are not counted first
+// (that took a launch of its own, 4.6 us in every bitplane step).
 // Grid (ceil(N / INVH_ROWS), INVH_COLS).  Every wave finds the bitplanes that
 // need the inverse with a ballot over the plane list; column y takes the
 // k-th of them for k = y, y + INVH_COLS, ...  Workgroup x computes rows
@@ -585,7 +580,7 @@ constexpr int INVH_ROWS = 64, INVH_COLS = 8, INVH_THREADS = 256;
 constexpr int INVH_MAX_WORDS = (6336 + 31) / 32;  // <= 4 words per lane
 
 __global__ __launch_bounds__(INVH_THREADS) void invh_kernel(const PlaneDesc *planes, int nplanes, LadderDev L,
-                                                            uint8_t *slots, int slot_capacity) {
+                                                            uint8_t *slots, int slot0) {
   __shared__ uint32_t sw[INVH_MAX_WORDS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int N = L.N, nw = (N + 31) / 32, C = L.numCodes;
@@ -620,8 +615,8 @@ __global__ __launch_bounds__(INVH_THREADS) void invh_kernel(const PlaneDesc *pla
       uint32_t w[4];
 #pragma unroll
       for (int q = 0; q < 4; q++) w[q] = lane + 64 * q < nw ? sw[lane + 64 * q] : 0u;
-      const int slot = d.rec[C - 1].z;
-      uint8_t *dst = slot >= 0 && slot < slot_capacity ? slots + (size_t)slot * N : nullptr;
+      if (blockIdx.x == 0 && tid == 0) d.rec[C - 1] = make_int4(0, REC_ACCEPTED, slot0 + b, 1);
+      uint8_t *dst = slots + (size_t)(slot0 + b) * N;
       uint32_t mine = 0;  // parity of row row0 + lane (lane < INVH_ROWS / 4)
 #pragma unroll 4
       for (int i = 0; i < INVH_ROWS / 4; i++) {
@@ -635,7 +630,7 @@ __global__ __launch_bounds__(INVH_THREADS) void invh_kernel(const PlaneDesc *pla
         const uint32_t par = __popcll(__ballot(__popc(x) & 1u)) & 1u;
         if (lane == i) mine = par;
       }
-      if (dst && lane < INVH_ROWS / 4 && row0 + lane < N) dst[row0 + lane] = (uint8_t)mine;
+      if (lane < INVH_ROWS / 4 && row0 + lane < N) dst[row0 + lane] = (uint8_t)mine;
     }
   }
 }
@@ -656,8 +651,8 @@ __global__ void gather_accepted_kernel(const PlaneDesc *planes, int nplanes, int
   for (int i = threadIdx.x; i < N / 16; i += blockDim.x) dst[i] = src[i];
 }
 
-// Clears n ints.  Used instead of hipMemsetAsync for the launch counters so a
-// captured step graph holds kernel nodes only.
+// Clears n ints (instead of hipMemsetAsync, so that a captured step holds kernel
+// nodes only).
 __global__ void zero_ints_kernel(int *p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
@@ -695,20 +690,17 @@ hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStrea
 }
 
 hipError_t launch_ce_llr(const PlaneDesc *d_planes, int n, int fixed_start, const Ladder &l1584,
-                         const Ladder &l6336, hipStream_t s) {
+                         const Ladder &l6336, int *counters, hipStream_t s) {
   hipLaunchKernelGGL(ce_llr_kernel, dim3(n), dim3(CE_T), 0, s, d_planes, n, fixed_start, l1584.d_codeRate,
-                     l6336.d_codeRate, l1584.numCodes, l6336.numCodes);
+                     l6336.d_codeRate, l1584.numCodes, l6336.numCodes, counters);
   return hipGetLastError();
 }
 
-hipError_t launch_invh(const PlaneDesc *d_planes, int n, const LadderDev &L, uint8_t *slots, int *slot_count,
-                       int slot_capacity, hipStream_t s) {
+hipError_t launch_invh(const PlaneDesc *d_planes, int n, const LadderDev &L, uint8_t *slots, int slot0,
+                       hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(invh_slot_kernel, dim3((n + 63) / 64), dim3(64), 0, s, d_planes, n, L.numCodes, slot_count);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(invh_kernel, dim3((L.N + INVH_ROWS - 1) / INVH_ROWS, INVH_COLS), dim3(INVH_THREADS), 0, s,
-                     d_planes, n, L, slots, slot_capacity);
+                     d_planes, n, L, slots, slot0);
   return hipGetLastError();
 }
 

@@ -93,6 +93,16 @@ __host__ __device__ inline int dynstep_next(int off) {
   return off < 1 ? 1 : off < 3 ? 3 : off < 6 ? 6 : off < 10 ? 10 : off + 4;
 }
 
+// Decision slots of a launch of n bitplanes over C codes.  The BP kernel hands
+// out the first `bp` of them: ParallelMode 0 accepts each (bitplane, code) at
+// most once, and a bitplane that accepts code C - 1 does so through the inverse;
+// ParallelMode 1 keeps every run code's decisions and its repeat-case decisions.
+// The n after them are the bitplanes' inverse slots.
+struct SlotPlan { int bp, total; };
+inline SlotPlan slot_plan(int n, int C, int mode) {
+  return mode == 1 ? SlotPlan{2 * C * n + 1, 2 * C * n + 1 + n} : SlotPlan{(C - 1) * n + 1, C * n + 1};
+}
+
 // record.y status values
 enum { REC_FAILED = 0, REC_CRC_MISMATCH = 1, REC_ACCEPTED = 2, REC_CANCELLED = 3, REC_NOT_RUN = -1 };
 
@@ -101,12 +111,16 @@ hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStrea
 hipError_t launch_zero_ints(int *p, int n, hipStream_t s);
 hipError_t launch_mode1_resolve(const PlaneDesc *planes, int n, int numCodes, int N, const uint8_t *slots,
                                 int slot_capacity, int *rerun_count, hipStream_t s);
+// Entropy, LLRs and start codes of n bitplanes; also clears the three launch
+// counters (queue head, decision slots handed out, bitplanes to resume).
 hipError_t launch_ce_llr(const PlaneDesc *d_planes, int n, int fixed_start, const Ladder &l1584,
-                         const Ladder &l6336, hipStream_t s);
+                         const Ladder &l6336, int *counters, hipStream_t s);
 // BP on an irregular ladder (bp_irregular_kernel, kIrregThreads per workgroup).
 hipError_t launch_bp_irregular(const BpArgs &a, int grid, hipStream_t s);
-hipError_t launch_invh(const PlaneDesc *d_planes, int n, const LadderDev &L, uint8_t *slots, int *slot_count,
-                       int slot_capacity, hipStream_t s);
+// Full-rate inverse of the bitplanes whose BP codes all failed, bitplane p's
+// into decision slot slot0 + p.
+hipError_t launch_invh(const PlaneDesc *d_planes, int n, const LadderDev &L, uint8_t *slots, int slot0,
+                       hipStream_t s);
 // Copies bitplane p's accepted decisions (N bytes, N a multiple of 16) to
 // out + p * N for every p < n; one with no accepted record in range is skipped.
 hipError_t launch_gather_accepted(const PlaneDesc *d_planes, int n, int N, const uint8_t *slots, int slot_capacity,

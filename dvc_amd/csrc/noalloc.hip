@@ -70,19 +70,17 @@ static NoallocLayout noalloc_layout(int nTotal, int n, int N, int C) {
   return o;
 }
 
-// One workgroup: lists the items of code length N (in item order), builds
-// their plane descriptors, rate-search states and run records, and clears
-// the launch counters.
+// One workgroup: lists the items of code length N (in item order) and builds
+// their plane descriptors, rate-search states and run records.
 __global__ __launch_bounds__(256) void noalloc_setup_kernel(const dvc_ldpca_item *items, int nTotal, int N, int C,
                                                            int *index, PlaneDesc *planes, PlaneState *state,
-                                                           int4 *rec, float *llr, int *counters) {
+                                                           int4 *rec, float *llr) {
   __shared__ int s_n;
   if (threadIdx.x == 0) {
     int k = 0;
     for (int i = 0; i < nTotal; i++)
       if (items[i].N == N) index[k++] = i;
     s_n = k;
-    counters[0] = counters[1] = counters[2] = 0;
   }
   __syncthreads();
   const int n = s_n;
@@ -188,7 +186,8 @@ extern "C" int dvc_ldpca_decode_batch_noalloc(dvc_ctx *c, int n, dvc_ldpca_item 
     if (!ng) continue;
     const int N = g ? 6336 : 1584;
     Ladder *L = c->ladder(N);
-    const int C = L->numCodes, maxOff = C - 1, slotCap = C * ng + 1;
+    const int C = L->numCodes, maxOff = C - 1;
+    const SlotPlan sp = slot_plan(ng, C, 0);
     const NoallocLayout o = noalloc_layout(n, ng, N, C);
     int *dIndex = (int *)(base + o.index), *dCounters = (int *)(base + o.counters);
     PlaneDesc *dPlanes = (PlaneDesc *)(base + o.planes);
@@ -197,15 +196,15 @@ extern "C" int dvc_ldpca_decode_batch_noalloc(dvc_ctx *c, int n, dvc_ldpca_item 
     float *dLLR = (float *)(base + o.llr);
     uint8_t *dSlots = base + o.slots;
     hipLaunchKernelGGL(noalloc_setup_kernel, dim3(1), dim3(256), 0, s, dItems, n, N, C, dIndex, dPlanes, dState, dRec,
-                       dLLR, dCounters);
+                       dLLR);
     DVC_HIP(hipGetLastError());
-    DVC_HIP(launch_ce_llr(dPlanes, ng, 1, c->lad1584, c->lad6336, s));
+    DVC_HIP(launch_ce_llr(dPlanes, ng, 1, c->lad1584, c->lad6336, dCounters, s));
     const LadderDev ld = ladder_dev(*L);
-    BpArgs a{ld, dPlanes, ng, dCounters, ng * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, slotCap,
+    BpArgs a{ld, dPlanes, ng, dCounters, ng * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, sp.bp,
              c->bp_poll, c->bp_mode, c->rate_step};
     DVC_HIP(launch_bp_any(N, bp_threads(c, N), a, bp_grid(c, N, ng * maxOff), s));
-    DVC_HIP(launch_invh(dPlanes, ng, ld, dSlots, dCounters + 1, slotCap, s));
-    hipLaunchKernelGGL(noalloc_finish_kernel, dim3(ng), dim3(128), 0, s, dItems, dIndex, dState, dRec, dSlots, slotCap,
+    DVC_HIP(launch_invh(dPlanes, ng, ld, dSlots, sp.bp, s));
+    hipLaunchKernelGGL(noalloc_finish_kernel, dim3(ng), dim3(128), 0, s, dItems, dIndex, dState, dRec, dSlots, sp.total,
                        N, C, L->d_syndLength, c->rate_step, dErr);
     DVC_HIP(hipGetLastError());
   }
