@@ -369,9 +369,9 @@ class Context:
             past = np.ascontiguousarray(d["past"], np.uint8)
             fut = np.ascontiguousarray(d["fut"], np.uint8)
             h, w = past.shape
-            si = np.zeros((h, w), np.uint8)
-            res = np.zeros((h, w), np.int32)
-            al = np.zeros((h, w), np.float32)
+            si = np.empty((h, w), np.uint8)
+            res = np.empty((h, w), np.int32)
+            al = np.empty((h, w), np.float32)
             keep += [past, fut]
             outs.append((si, res, al))
             pi, ci, fi = d.get("idx", (0, 1, 2))
@@ -429,14 +429,14 @@ class BandSession:
         oct_ = np.ascontiguousarray(oct_, np.int32)
         n = smf.size
         per = 2 * rng + 1 if index else rng
-        out = np.zeros((n, per), np.float32) if want else None
+        out = np.empty((n, per), np.float32) if want else None
         _check(lib.dvc_noise_distribution(self.ctx.h, rng, index, alpha.ctypes.data, smf.ctypes.data, oct_.ctypes.data,
                                           None if out is None else out.ctypes.data), "dvc_noise_distribution")
         return out
 
     def cond_bit_prob(self, index, bit, step, recons_trans, rng):
         rt = np.ascontiguousarray(recons_trans, np.int32)
-        lr = np.zeros(self.w * self.h // 16, np.float32)
+        lr = np.empty(self.w * self.h // 16, np.float32)
         _check(lib.dvc_cond_bit_prob(self.ctx.h, lr.ctypes.data, index, bit, step, rt.ctypes.data, rng),
                "dvc_cond_bit_prob")
         return lr

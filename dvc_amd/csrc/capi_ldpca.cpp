@@ -141,6 +141,8 @@ int dvc_ctx_destroy(dvc_ctx *c) {
   if (c->d_costFme) (void)hipFree(c->d_costFme);
   if (c->d_costUsi) (void)hipFree(c->d_costUsi);
   if (c->si_scratch) (void)hipFree(c->si_scratch);
+  if (c->si_host) (void)hipHostFree(c->si_host);
+  host_pool_free(c);
   if (c->ld_dev) (void)hipFree(c->ld_dev);
   if (c->ld_host) (void)hipHostFree(c->ld_host);
   band_free(c);

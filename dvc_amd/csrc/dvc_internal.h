@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -95,6 +96,18 @@ void band_free(dvc_ctx *c);
 // (current) device, once per device (noalloc.hip).
 int noalloc_attach(dvc_ctx *c);
 void free_ladder(Ladder &L);
+// Host copies of the entry points that take host buffers, on up to eight threads
+// (host_pool.cpp), and pinned staging kept between calls.
+struct HostPool;
+struct HostCopy { void *dst; const void *src; size_t bytes; };
+void host_parallel(dvc_ctx *c, size_t n, size_t bytes, const std::function<void(size_t)> &fn);
+void host_copy(dvc_ctx *c, const std::vector<HostCopy> &list);
+void host_pool_free(dvc_ctx *c);
+// Device memory to a caller's buffer through pinned memory of the same size,
+// the copies out overlapping the transfers; returns when all is there.
+int copy_back(dvc_ctx *c, hipStream_t s, void *user, const void *dev, uint8_t *pinned, size_t bytes);
+// Pinned host block of at least `bytes` in *p (grown, contents dropped).
+int pinned_grow(uint8_t **p, size_t *have, size_t bytes);
 
 }  // namespace dvc
 
@@ -134,6 +147,9 @@ struct dvc_ctx {
   hipStream_t stream = nullptr;
   void *si_scratch = nullptr;  // dvc_side_info_batch's device buffers, kept between calls
   size_t si_scratch_bytes = 0;
+  uint8_t *si_host = nullptr;  // its pinned host staging, and the per-band entry points'
+  size_t si_host_bytes = 0;
+  dvc::HostPool *pool = nullptr;  // host copy threads (made on first use)
   void *ld_dev = nullptr;      // the LDPCA entry points' device workspace, kept between calls
   size_t ld_dev_bytes = 0;
   void *ld_host = nullptr;     // its pinned host staging (inputs up, results back)

@@ -92,9 +92,6 @@ hipError_t launch_keyframe_filters(const uint8_t *in, uint8_t *lp, uint8_t *half
 hipError_t launch_create_si(const FrameDev *F, const int *list, int n, int maxMB, CostTables ct, hipStream_t s);
 // forwardME alone (sideInfoCreation.cpp:61-145): macroblock MVs (mbmv, unscaled) from past_lp/fut_lp.
 hipError_t launch_forward_me(const FrameDev *F, const int *list, int n, int maxMB, CostTables ct, hipStream_t s);
-// Writes octBand from oct for coefficient `index` (the per-band entry points,
-// whose over-complete transform comes from the caller).
-hipError_t launch_oct_plane(const FrameDev *F, const int *list, int n, int maxPos, int index, hipStream_t s);
 hipError_t launch_noise_param(const FrameDev *F, const int *list, int n, int maxN, hipStream_t s);
 hipError_t launch_oct(const FrameDev *F, const int *list, int n, int maxPos, int initSideTrans, hipStream_t s);
 // fill: store the zeros outside each block's span as well (readers of whole rows).

@@ -639,7 +639,8 @@ __global__ __launch_bounds__(256) void k_noise_moments(const FrameDev *F, const 
     f.npMom[index] = make_float2(mean, var / (float)N - mean * mean);
   }
 }
-// alpha of every block at the frame's bands, a thread per 4x4 block.
+// alpha of every block at the frame's bands, 0 at the other coefficients; a
+// thread per 4x4 block.
 __global__ __launch_bounds__(256) void k_noise_alpha(const FrameDev *F, const int *list) {
   const FrameDev &f = F[list[blockIdx.y]];
   const int b = blockIdx.x * 256 + threadIdx.x, W = f.W, bw = W / 4;
@@ -650,14 +651,17 @@ __global__ __launch_bounds__(256) void k_noise_alpha(const FrameDev *F, const in
     const size_t o = (size_t)(top + m) * W + left;
     const int4 v = *(const int4 *)(f.sideTrans + o);
     const int c4[4] = {v.x, v.y, v.z, v.w};
+    float a4[4];
 #pragma unroll
     for (int n = 0; n < 4; n++) {
+      a4[n] = 0.0f;
       if (c_qbits[f.qindex][4 * m + n] <= 0) continue;  // uniform
       const float2 mom = f.npMom[4 * m + n];
       const float dst = (float)abs(c4[n]) - mom.x;
       const float dst2 = dst * dst;
-      f.alpha[o + n] = dst2 > mom.y ? sqrtf(2 / dst2) : sqrtf(2 / mom.y);
+      a4[n] = dst2 > mom.y ? sqrtf(2 / dst2) : sqrtf(2 / mom.y);
     }
+    *(float4 *)(f.alpha + o) = make_float4(a4[0], a4[1], a4[2], a4[3]);
   }
 }
 
@@ -721,14 +725,6 @@ __global__ __launch_bounds__(256) void k_oct(const FrameDev *F, const int *list,
     const int piece = 256 * i + threadIdx.x;
     if (p0 + (piece >> 2) < npos) dst[piece] = s_rec[piece];
   }
-}
-
-// octBand from a complete over-complete transform (coefficient `index`).
-__global__ __launch_bounds__(256) void k_oct_plane(const FrameDev *F, const int *list, int index) {
-  const FrameDev &f = F[list[blockIdx.y]];
-  const int npos = (f.W - 3) * (f.H - 3);
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < npos) f.octBand[p] = f.oct[(size_t)16 * p + index];
 }
 
 // SMF window of WZ block b (initSMF, motionLearning.cpp:6-47).
@@ -1525,10 +1521,6 @@ __global__ void k_skip_copy(const FrameDev *F, const int *list) {
 }
 hipError_t launch_skip_copy(const FrameDev *F, const int *list, int n, int maxBlk88, hipStream_t s) {
   hipLaunchKernelGGL(k_skip_copy, dim3((maxBlk88 + 255) / 256, n), dim3(256), 0, s, F, list);
-  return hipGetLastError();
-}
-hipError_t launch_oct_plane(const FrameDev *F, const int *list, int n, int maxPos, int index, hipStream_t s) {
-  hipLaunchKernelGGL(k_oct_plane, dim3((maxPos + 255) / 256, n), dim3(256), 0, s, F, list, index);
   return hipGetLastError();
 }
 hipError_t launch_noise_dist(const FrameDev *F, const int *list, int n, int maxN, int fill, hipStream_t s) {
