@@ -328,6 +328,8 @@ struct KeyEntry {
   size_t bytes = 0;
 };
 
+constexpr int kStageRing = 4;
+
 // One lane of the engine: a stream, the frames it advances in lockstep and
 // its device scratch.  Lanes step concurrently from host threads, so the tail
 // of one lane's LDPCA launch and its host round trips overlap the other
@@ -338,12 +340,17 @@ struct Lane {
   SlotPlan slots{};  // decision slots of each code length
   std::vector<Job *> inflight;
   std::vector<Job *> finished;  // retired by the engine after the step
-  // A step's descriptors, written to one pinned host block and uploaded to
-  // its device mirror with one copy: frame descriptors, five frame lists of
+  // A step's descriptors, written to one of kStageRing pinned host blocks in turn
+  // and uploaded to the one device mirror with one copy: frame descriptors, five frame lists of
   // cap entries (stepped, starting a band, ending a band, set up, finishing),
   // BP frame links, plane descriptors, result copy segments (3 per frame).
-  uint8_t *h_stage = nullptr, *d_stage = nullptr;
-  size_t stageBytes = 0;
+  // The copy is ordered behind the previous step's kernels, so only the host
+  // block has to wait for it, and the host prepares and queues the next steps
+  // while this one runs: nothing in a step depends on its predecessors' results.
+  uint8_t *h_stage = nullptr, *d_stage = nullptr;  // h_stage: kStageRing blocks
+  size_t stageBytes = 0, oLists = 0, oLinks = 0, oPlanes = 0, oSegs = 0;
+  hipEvent_t staged[kStageRing] = {};  // block k's last upload
+  unsigned steps = 0;
   FrameDev *h_frames = nullptr, *d_frames = nullptr;
   int *h_lists = nullptr, *d_lists = nullptr;
   BpFrameLink *h_links = nullptr, *d_links = nullptr;
@@ -625,6 +632,17 @@ static int lane_step(dvc_engine *e, Lane &ln) {
   int rc;
   const int n = (int)ln.inflight.size();
   if (n == 0) return DVC_OK;
+  // the staging block used kStageRing steps ago, once its upload is done.  (With
+  // the stream drained after every step, a CIF frame decoded alone left the GPU
+  // idle for 40 us of each of its 63 steps.)
+  const int slot = (int)(ln.steps++ % kStageRing);
+  uint8_t *stage = ln.h_stage + slot * ln.stageBytes;
+  DVC_HIP(hipEventSynchronize(ln.staged[slot]));
+  ln.h_frames = (FrameDev *)stage;
+  ln.h_lists = (int *)(stage + ln.oLists);
+  ln.h_links = (BpFrameLink *)(stage + ln.oLinks);
+  ln.h_planes = (PlaneDesc *)(stage + ln.oPlanes);
+  ln.h_segs = (CopySeg *)(stage + ln.oSegs);
   int maxN = 0, maxMB = 0, maxPos = 0, maxBw = 0, maxBh = 0;
   for (int i = 0; i < n; i++) {
     Job *j = ln.inflight[i];
@@ -695,7 +713,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
     outUsed += job_out_bytes(e, *ln.inflight[fin[k]]);
   }
   if (outUsed > ln.outBytes) {
-    // the lane's stream is idle here (synchronised at the end of every step)
+    DVC_HIP(hipStreamSynchronize(s));  // the last gather into the blocks is done
     if (ln.d_out) (void)hipFree(ln.d_out);
     if (ln.h_out) (void)hipHostFree(ln.h_out);
     ln.d_out = ln.h_out = nullptr;
@@ -716,7 +734,8 @@ static int lane_step(dvc_engine *e, Lane &ln) {
     if (e->deviceBuffers) ln.h_segs[nseg++] = CopySeg{j.fd.recons, j.spec.recons, FS};
   }
   // ---- one upload of the step's descriptors
-  DVC_HIP(hipMemcpyAsync(ln.d_stage, ln.h_stage, ln.stageBytes, hipMemcpyHostToDevice, s));
+  DVC_HIP(hipMemcpyAsync(ln.d_stage, stage, ln.stageBytes, hipMemcpyHostToDevice, s));
+  DVC_HIP(hipEventRecord(ln.staged[slot], s));
   // ---- setup of newly admitted frames: SI, noise parameters, OCT, SMF
   if (!setup.empty()) {
     const int nf = (int)setup.size();
@@ -836,7 +855,6 @@ static int lane_step(dvc_engine *e, Lane &ln) {
     }
     ln.inflight.swap(keep);
   }
-  DVC_HIP(hipStreamSynchronize(s));  // the step's host staging is reused next step
   return DVC_OK;
 }
 
@@ -996,20 +1014,22 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
     l.cap = (e->maxInflight + nl - 1) / nl;
     l.slots = slot_plan(l.cap, kMaxCodes, c->bp_mode);
     const size_t M = l.cap;
-    const size_t oFrames = 0, oLists = align_up(oFrames + sizeof(FrameDev) * M), oLinks = align_up(oLists + sizeof(int) * 5 * M),
-                 oPlanes = align_up(oLinks + sizeof(BpFrameLink) * M), oSegs = align_up(oPlanes + sizeof(PlaneDesc) * M),
-                 total = align_up(oSegs + sizeof(CopySeg) * 4 * M);
+    l.oLists = align_up(sizeof(FrameDev) * M);
+    l.oLinks = align_up(l.oLists + sizeof(int) * 5 * M);
+    l.oPlanes = align_up(l.oLinks + sizeof(BpFrameLink) * M);
+    l.oSegs = align_up(l.oPlanes + sizeof(PlaneDesc) * M);
+    l.stageBytes = align_up(l.oSegs + sizeof(CopySeg) * 4 * M);
     err = hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking);
-    if (err == hipSuccess) err = hipHostMalloc((void **)&l.h_stage, total, hipHostMallocDefault);
-    if (err == hipSuccess) err = hipMalloc((void **)&l.d_stage, total);
+    if (err == hipSuccess) err = hipHostMalloc((void **)&l.h_stage, l.stageBytes * kStageRing, hipHostMallocDefault);
+    if (err == hipSuccess) err = hipMalloc((void **)&l.d_stage, l.stageBytes);
+    for (int r = 0; r < kStageRing && err == hipSuccess; r++) err = hipEventCreateWithFlags(&l.staged[r], hipEventDisableTiming);
     if (err == hipSuccess) {
-      l.stageBytes = total;
-      memset(l.h_stage, 0, total);
-      l.h_frames = (FrameDev *)(l.h_stage + oFrames); l.d_frames = (FrameDev *)(l.d_stage + oFrames);
-      l.h_lists = (int *)(l.h_stage + oLists); l.d_lists = (int *)(l.d_stage + oLists);
-      l.h_links = (BpFrameLink *)(l.h_stage + oLinks); l.d_links = (BpFrameLink *)(l.d_stage + oLinks);
-      l.h_planes = (PlaneDesc *)(l.h_stage + oPlanes); l.d_planes = (PlaneDesc *)(l.d_stage + oPlanes);
-      l.h_segs = (CopySeg *)(l.h_stage + oSegs); l.d_segs = (CopySeg *)(l.d_stage + oSegs);
+      memset(l.h_stage, 0, l.stageBytes * kStageRing);
+      l.d_frames = (FrameDev *)l.d_stage;
+      l.d_lists = (int *)(l.d_stage + l.oLists);
+      l.d_links = (BpFrameLink *)(l.d_stage + l.oLinks);
+      l.d_planes = (PlaneDesc *)(l.d_stage + l.oPlanes);
+      l.d_segs = (CopySeg *)(l.d_stage + l.oSegs);
     }
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_slots, (size_t)2 * l.slots.total * 6336);
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_counters, 6 * sizeof(int));
@@ -1038,6 +1058,8 @@ static void engine_destroy(dvc_engine *e) {
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
     if (l.h_stage) (void)hipHostFree(l.h_stage);
+    for (hipEvent_t e : l.staged)
+      if (e) (void)hipEventDestroy(e);
     if (l.h_out) (void)hipHostFree(l.h_out);
     if (l.s) (void)hipStreamDestroy(l.s);
   }
