@@ -29,8 +29,9 @@ static std::string default_data_dir() {
 int bp_threads(const dvc_ctx *c, int N) { return N == 1584 ? c->bp_threads_qcif : c->bp_threads_cif; }
 
 int bp_grid(const dvc_ctx *c, int N, int items) {
-  // a CIF codeword takes 118 KB of a CU's 160 KB LDS; QCIF codewords (30 KB) share one
-  const int perCU = N == 6336 ? 1 : c->bp_wg_per_cu_qcif;
+  // a CIF codeword takes 126 KB of a CU's 160 KB LDS, an irregular QCIF codeword's
+  // 16 waves its registers; regular QCIF codewords (38 KB, 8 waves) share one
+  const int perCU = N == 6336 || !c->lad1584.regular ? 1 : c->bp_wg_per_cu_qcif;
   return std::max(1, std::min(c->sm_count * perCU, items));
 }
 

@@ -30,10 +30,6 @@ void set_error(const std::string &msg);
     if (!(cond)) { dvc::set_error(msg); return (code); }                               \
   } while (0)
 
-// The BP kernels' threads per workgroup on an irregular ladder (its
-// column-to-thread table is built for this count).
-constexpr int kIrregThreads = 256;
-
 // Host copy of one ladder (all codes of one code length) and its device image.
 struct Ladder {
   int N = 0, E = 0, period = 0, numCodes = 0;
@@ -59,16 +55,12 @@ struct Ladder {
   //   d_tx[c*N + k]            accumulated-syndrome position of syndrome bit k
   ColEdges *d_colRows = nullptr;
   // Irregular ladders (column degrees differ) instead of d_colRows:
-  //   d_colEdges[c*E + l]   edge l (column order) as row | rank << 16
+  //   d_slotEdges[c*E + s]  message slot s (row order) as row | column << 13
   //   d_jc[k]               column pointers (N+1)
-  //   d_colSlots[t*S + i]   the i-th column thread t of a kIrregThreads
-  //                         workgroup updates (-1: none), S = colSlotsPerThread,
-  //                         columns dealt to threads so each thread's edge
-  //                         count is nearly equal
-  uint32_t *d_colEdges = nullptr;
+  //   d_colSlots[c*E + l]   edge l's message slot (l in column order)
+  uint32_t *d_slotEdges = nullptr;
   int *d_jc = nullptr;
-  int16_t *d_colSlots = nullptr;
-  int colSlotsPerThread = 0;
+  uint16_t *d_colSlots = nullptr;
   uint16_t *d_rowPtr = nullptr, *d_tx = nullptr;
   int *d_syndLength = nullptr;
   float *d_codeRate = nullptr;

@@ -145,32 +145,10 @@ int load_ladder(const std::string &dir, const char *kind, int N, Ladder &L) {
   return DVC_OK;
 }
 
-// Deals the columns of an irregular ladder to kIrregThreads threads: by
-// decreasing degree, each to the thread with the fewest edges so far, so the
-// threads of a workgroup carry nearly equal variable-node work.
-static void column_slots(const Ladder &L, std::vector<int16_t> &slots, int &perThread) {
-  const int T = kIrregThreads, N = L.N;
-  std::vector<int> order(N), load(T, 0), cnt(T, 0), owner(N);
-  for (int k = 0; k < N; k++) order[k] = k;
-  std::stable_sort(order.begin(), order.end(),
-                   [&L](int a, int b) { return L.jc[a + 1] - L.jc[a] > L.jc[b + 1] - L.jc[b]; });
-  for (int k : order) {
-    int t = 0;
-    for (int u = 1; u < T; u++)
-      if (load[u] < load[t]) t = u;
-    owner[k] = t;
-    load[t] += L.jc[k + 1] - L.jc[k];
-    cnt[t]++;
-  }
-  perThread = *std::max_element(cnt.begin(), cnt.end());
-  slots.assign((size_t)T * perThread, (int16_t)-1);
-  std::fill(cnt.begin(), cnt.end(), 0);
-  for (int k = 0; k < N; k++) slots[(size_t)owner[k] * perThread + cnt[owner[k]]++] = (int16_t)k;
-}
-
 int upload_ladder(Ladder &L) {
   const int N = L.N, E = L.E, C = L.numCodes;
-  std::vector<uint32_t> colRows(L.regular ? (size_t)C * N * 3 : 0), colEdges(L.regular ? 0 : (size_t)C * E);
+  std::vector<uint32_t> colRows(L.regular ? (size_t)C * N * 3 : 0), slotEdges(L.regular ? 0 : (size_t)C * E);
+  std::vector<uint16_t> colSlots(L.regular ? 0 : (size_t)C * E);
   std::vector<uint16_t> rowPtr((size_t)C * (N + 1)), tx((size_t)C * N);
   DVC_CHECK(E <= 0xffff && N <= 0x2000, DVC_EIO, "ladder: more than 65535 edges or 8192 checks");
   for (int c = 0; c < C; c++) {
@@ -183,13 +161,15 @@ int upload_ladder(Ladder &L) {
     // rank of each edge within its row, rows listing edges in ascending order
     std::vector<int> fill(cnt.begin(), cnt.end() - 1);
     std::vector<uint32_t> field(E);
-    for (int e = 0; e < E; e++) {
-      const int rank = fill[dir[e]]++ - cnt[dir[e]];
+    for (int k = 0, e = 0; e < E; e++) {
+      while (e >= L.jc[k + 1]) k++;  // edge e belongs to column k
+      const int slot = fill[dir[e]]++;
       if (!L.regular) {
-        colEdges[(size_t)c * E + e] = (uint32_t)dir[e] | ((uint32_t)rank << 16);
+        slotEdges[(size_t)c * E + slot] = (uint32_t)dir[e] | ((uint32_t)k << 13);
+        colSlots[(size_t)c * E + e] = (uint16_t)slot;
         continue;
       }
-      field[e] = (uint32_t)dir[e] | ((uint32_t)(cnt[dir[e]] + rank) << 15);  // row | message slot << 15
+      field[e] = (uint32_t)dir[e] | ((uint32_t)slot << 15);  // row | message slot << 15
     }
     for (int k = 0; L.regular && k < N; k++)  // every column has degree 3: edges 3k..3k+2
       for (int q = 0; q < 3; q++) colRows[((size_t)c * N + k) * 3 + q] = field[3 * k + q];
@@ -199,14 +179,12 @@ int upload_ladder(Ladder &L) {
   if (L.regular) {
     DVC_HIP(hipMalloc(&L.d_colRows, colRows.size() * 4));
     } else {
-    std::vector<int16_t> slots;
-    column_slots(L, slots, L.colSlotsPerThread);
-    DVC_HIP(hipMalloc(&L.d_colEdges, colEdges.size() * 4));
+    DVC_HIP(hipMalloc(&L.d_slotEdges, slotEdges.size() * 4));
     DVC_HIP(hipMalloc(&L.d_jc, (N + 1) * sizeof(int)));
-    DVC_HIP(hipMalloc(&L.d_colSlots, slots.size() * sizeof(int16_t)));
-    DVC_HIP(hipMemcpy(L.d_colEdges, colEdges.data(), colEdges.size() * 4, hipMemcpyHostToDevice));
+    DVC_HIP(hipMalloc(&L.d_colSlots, colSlots.size() * 2));
+    DVC_HIP(hipMemcpy(L.d_slotEdges, slotEdges.data(), slotEdges.size() * 4, hipMemcpyHostToDevice));
     DVC_HIP(hipMemcpy(L.d_jc, L.jc.data(), (N + 1) * sizeof(int), hipMemcpyHostToDevice));
-    DVC_HIP(hipMemcpy(L.d_colSlots, slots.data(), slots.size() * sizeof(int16_t), hipMemcpyHostToDevice));
+    DVC_HIP(hipMemcpy(L.d_colSlots, colSlots.data(), colSlots.size() * 2, hipMemcpyHostToDevice));
   }
   DVC_HIP(hipMalloc(&L.d_rowPtr, rowPtr.size() * 2));
   DVC_HIP(hipMalloc(&L.d_tx, tx.size() * 2));
@@ -225,12 +203,12 @@ int upload_ladder(Ladder &L) {
 }
 
 void free_ladder(Ladder &L) {
-  void *ptrs[] = {L.d_colRows, L.d_colEdges, L.d_jc, L.d_colSlots, L.d_rowPtr,  L.d_tx,
+  void *ptrs[] = {L.d_colRows, L.d_slotEdges, L.d_jc, L.d_colSlots, L.d_rowPtr,  L.d_tx,
                   L.d_syndLength, L.d_codeRate, L.d_invH, L.d_crcBasis};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   L.d_colRows = nullptr;
-  L.d_colEdges = nullptr; L.d_jc = nullptr; L.d_colSlots = nullptr;
+  L.d_slotEdges = nullptr; L.d_jc = nullptr; L.d_colSlots = nullptr;
   L.d_rowPtr = L.d_tx = nullptr;
   L.d_syndLength = nullptr; L.d_codeRate = nullptr; L.d_invH = L.d_crcBasis = nullptr;
 }

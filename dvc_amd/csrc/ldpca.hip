@@ -716,7 +716,7 @@ LadderDev ladder_dev(const Ladder &L) {
   d.N = L.N; d.E = L.E; d.numCodes = L.numCodes;
   d.regular = L.regular ? 1 : 0;
   d.colRows = L.d_colRows; d.rowPtr = L.d_rowPtr; d.tx = L.d_tx;
-  d.colEdges = L.d_colEdges; d.jc = L.d_jc; d.colSlots = L.d_colSlots; d.colSlotsPerThread = L.colSlotsPerThread;
+  d.slotEdges = L.d_slotEdges; d.jc = L.d_jc; d.colSlots = L.d_colSlots;
   d.syndLength = L.d_syndLength; d.invH = L.d_invH; d.crcBasis = L.d_crcBasis;
   return d;
 }

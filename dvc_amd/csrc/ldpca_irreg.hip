@@ -8,19 +8,24 @@
 // (ldpca.hip) evaluates it: phi(x) = -logf(tanhf((x + 1e-9f)/2)) by
 // dvc_bp_phi_fast, check sums in ascending edge order, variable sums
 // LLR + c2v of the column's edges in jc order, the same decision, parity and
-// CRC rules, and the same handling of NaN likelihood ratios.  What differs
-// is the column walk: a column's edges come from the ladder's column pointers
-// (jc) and per-edge (row, rank in row) words, and the variable pass runs in
-// two sweeps over them -- the first forms each c2v and the column total and
-// parks the c2v in the edge's message slot, the second turns the slot into
-// the next v2c's phi -- because a degree-21 column's messages do not fit in
-// registers.  Columns are dealt to the workgroup's threads by the ladder
-// upload so that each thread carries nearly the same number of edges.
+// CRC rules, and the same handling of NaN likelihood ratios.  What differs is
+// the variable pass.  Its two phi per edge bound the kernel, and a column has 2
+// to 21 edges, so it runs in three sweeps with a barrier between: a lane per
+// message slot turns the slot's message into its c2v; a lane per column adds
+// the column's c2v in jc order; a lane per slot turns the c2v into the next
+// v2c's phi.  Slots are in row order, so a sweep's messages, rows and stores are
+// those of consecutive lanes, and only the column totals and the column sums'
+// reads are scattered.  The decisions go out as ballots, one bit per slot, and
+// the check pass counts a row's bits, so nothing is XORed by atomics.
+// With a lane walking all edges of its columns twice (columns dealt to 256
+// threads by edge count) the search of one bitplane took 3.28 ms, of 64 4.2 and
+// of 256 8.2; now 0.58, 1.30 and 3.46 (with 512 threads and two workgroups per
+// CU 0.76, 1.42 and 3.47).
 //
 // Batched form and cancellation are those of bp_persistent_kernel: a
 // persistent grid walks (bitplane, code offset) items in offset-major order,
 // skips codes above the lowest accepted one and stops running ones once a
-// lower code is accepted.  LDS: 42 KB per codeword (3 per CU).
+// lower code is accepted.  One codeword per CU (60 KB of LDS, 16 waves).
 #include <stdio.h>
 #include "dvc_internal.h"
 #include "dvc_math.h"
@@ -30,7 +35,8 @@
 
 namespace dvc {
 
-constexpr int IR_NMAX = 1584, IR_EMAX = 8192;
+constexpr int IR_T = 1024;  // threads per workgroup
+constexpr int IR_NMAX = 1584, IR_EMAX = 8192;  // edges: a multiple of 64 with room for the last wave's slots
 
 __device__ __forceinline__ uint32_t ir_f2u(float f) { return __float_as_uint(f); }
 __device__ __forceinline__ float ir_u2f(uint32_t u) { return __uint_as_float(u); }
@@ -41,8 +47,8 @@ __device__ __forceinline__ uint32_t ir_acc_bit(const uint8_t *acc, int i) {
 }
 
 template <bool MODE1>
-__global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
-  constexpr int T = kIrregThreads;
+__global__ __launch_bounds__(IR_T) void bp_irregular_kernel(BpArgs a) {
+  constexpr int T = IR_T;
   // phi's logf table: (invc * 2^-k, k*ln2 + logc) for each (k, i) that phi's
   // arguments reach, read with per-lane indices
   __shared__ __align__(16) double s_phitab[2 * DVC_PHI_LOGTAB];
@@ -50,18 +56,18 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
   // the end, so that the check pass may read a row's last slots unconditionally
   __shared__ float phi[IR_EMAX + 3];
   __shared__ float rowTot[IR_NMAX];
+  __shared__ float colTot[IR_NMAX];
+  __shared__ uint64_t slotDec[IR_EMAX / 64 + 1];  // each slot's column's decision
   __shared__ uint16_t rowPtr[IR_NMAX + 2];
   __shared__ uint8_t dec[IR_NMAX];
   __shared__ uint32_t synBits[(IR_NMAX + 31) / 32];
-  __shared__ uint32_t parBits[2][(IR_NMAX + 31) / 32];
   __shared__ int s_item, s_cancel;
   __shared__ uint32_t s_crc[T / 64];
   __shared__ int s_changed[2];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const LadderDev L = a.lad;
-  const int N = L.N, E = L.E, S = L.colSlotsPerThread, synWords = (N + 31) / 32;
-  const int16_t *mySlots = L.colSlots + (size_t)tid * S;
+  const int N = L.N, E = L.E, synWords = (N + 31) / 32;
   for (int e = tid; e < DVC_PHI_LOGTAB; e += T) dvc_phi_logtab_entry(e, s_phitab);
 
   for (;;) {
@@ -102,7 +108,8 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
     };
     const bool mode1 = MODE1, exact = level == run;
     const int m = L.syndLength[level];
-    const uint32_t *gedge = L.colEdges + (size_t)level * E;
+    const uint32_t *gslot = L.slotEdges + (size_t)level * E;   // per slot: row | column << 13
+    const uint16_t *gcolSlot = L.colSlots + (size_t)level * E;  // per edge in column order: its slot
     const uint16_t *growPtr = L.rowPtr + (size_t)level * (N + 1);
     const float *gLLR = pd.LLR;
 
@@ -122,18 +129,14 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
       synBits[wd] = bits;
     }
     // ---- variable-to-check messages start at the channel LLR (:478-481)
-    for (int i = 0; i < S; i++) {
-      const int k = mySlots[i];
-      if (k < 0) break;
+    for (int k = tid; k < N; k += T) {
       const float v = gLLR[k];
       const uint32_t s = ir_f2u(v) >> 31;
       const float mag = (s ? -1.0f : 1.0f) * v;
-      const float f = ir_u2f((ir_f2u(phi_of(mag)) & 0x7fffffffu) | (s << 31));
-      for (int l = L.jc[k]; l < L.jc[k + 1]; l++) {
-        const uint32_t e = gedge[l];
-        phi[growPtr[e & 0xffffu] + (e >> 16)] = f;
-      }
+      colTot[k] = ir_u2f((ir_f2u(phi_of(mag)) & 0x7fffffffu) | (s << 31));
     }
+    __syncthreads();
+    for (int l = tid; l < E; l += T) phi[l] = colTot[gslot[l] >> 13];
     __syncthreads();
 
     int status = 0, iters = 0;
@@ -142,7 +145,6 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
       // ---- check pass: |phi| sums and sign products; parity of the previous
       // decisions (:495-515, :551-568)
       int fail = 0;
-      const uint32_t *parPrev = parBits[(t + 1) & 1];
       for (int r = tid; r < m; r += T) {
         const int e0 = rowPtr[r], e1 = rowPtr[r + 1];
         const uint32_t syn = (synBits[r >> 5] >> (r & 31)) & 1u;
@@ -173,9 +175,21 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
         }
         const uint32_t sgn = syn ^ (sx >> 31);
         rowTot[r] = ir_u2f(ir_f2u(sum) | (sgn << 31));
-        if (t > 0 && (syn ^ ((parPrev[r >> 5] >> (r & 31)) & 1u))) fail = 1;
+        if (t > 0) {
+          // parity of the decisions on slots [e0, e1)
+          uint32_t par = 0;
+          if (e1 > e0) {
+            const int w0 = e0 >> 6, w1 = (e1 - 1) >> 6;
+            uint64_t bits = slotDec[w0] & (~0ull << (e0 & 63));
+            for (int q = w0; q < w1; q++) {
+              par ^= (uint32_t)__popcll(bits);
+              bits = slotDec[q + 1];
+            }
+            par ^= (uint32_t)__popcll(bits & (~0ull >> (63 - ((e1 - 1) & 63))));
+          }
+          fail |= (int)((syn ^ par) & 1u);
+        }
       }
-      for (int wd = tid; wd < synWords; wd += T) parBits[t & 1][wd] = 0u;
       if (mode1 && t > 0) sameCount = s_changed[(t - 1) & 1] ? 0 : sameCount + 1;
       if (tid == 0) {
         s_changed[t & 1] = 0;
@@ -200,24 +214,34 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
       if (s_cancel) { status = 3; iters = t; break; }
       if (t == a.max_iter) { status = 0; iters = t; break; }
 
-      // ---- variable pass (:512-548): c2v of every edge and the column total
-      // in jc order, the decision, then each edge's next v2c
+      // ---- variable pass (:512-548).  c2v of every slot
+      uint32_t eNext = tid < E ? gslot[tid] : 0u;
+      for (int l = tid; l < E; l += T) {
+        const uint32_t e = eNext;
+        if (l + T < E) eNext = gslot[l + T];
+        const uint32_t R = ir_f2u(rowTot[e & 0x1fffu]), ph = ir_f2u(phi[l]);
+        const float v = phi_of(ir_u2f(R & 0x7fffffffu) - ir_u2f(ph & 0x7fffffffu));
+        // times -1 or 1 by the sign product; with no NaN (ParallelMode 0 never
+        // runs a NaN bitplane) that is the sign bit flipped
+        phi[l] = MODE1 ? (((R ^ ph) >> 31) ? v * -1.0f : v * 1.0f)
+                       : ir_u2f((ir_f2u(v) & 0x7fffffffu) | ((ir_f2u(v) ^ R ^ ph) & 0x80000000u));
+      }
+      __syncthreads();
+      // column totals in jc order and decisions
       bool changed = false;
-      for (int i = 0; i < S; i++) {
-        const int k = mySlots[i];
-        if (k < 0) break;
+      for (int k = tid; k < N; k += T) {
         const int l0 = L.jc[k], l1 = L.jc[k + 1];
         float tmp = gLLR[k];
-        for (int l = l0; l < l1; l++) {
-          const uint32_t e = gedge[l];
-          const int row = e & 0xffffu, pos = rowPtr[row] + (e >> 16);
-          const uint32_t R = ir_f2u(rowTot[row]), ph = ir_f2u(phi[pos]);
-          const float x = ir_u2f(R & 0x7fffffffu) - ir_u2f(ph & 0x7fffffffu);
-          const float v = phi_of(x);
-          const float c2v = ((R ^ ph) >> 31) ? v * -1.0f : v * 1.0f;
-          tmp += c2v;
-          phi[pos] = c2v;
+        int l = l0;
+        for (; l + 4 <= l1; l += 4) {
+          float c[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) c[i] = phi[gcolSlot[l + i]];
+#pragma unroll
+          for (int i = 0; i < 4; i++) tmp += c[i];
         }
+        for (; l < l1; l++) tmp += phi[gcolSlot[l]];
+        colTot[k] = tmp;
         uint32_t d;
         if (!mode1) {
           d = ir_f2u(tmp) >> 31;
@@ -227,17 +251,23 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
           else changed |= dec[k] != (uint8_t)d;
         }
         dec[k] = (uint8_t)d;
-        for (int l = l0; l < l1; l++) {
-          const uint32_t e = gedge[l];
-          const int row = e & 0xffffu, pos = rowPtr[row] + (e >> 16);
-          const float v2c = tmp - phi[pos];
-          const uint32_t sg = ir_f2u(v2c) >> 31;
-          const float v = phi_of((sg ? -1.0f : 1.0f) * v2c);
-          phi[pos] = ir_u2f((ir_f2u(v) & 0x7fffffffu) | (sg << 31));
-          if (d) atomicXor(&parBits[t & 1][row >> 5], 1u << (row & 31));
-        }
       }
       if (changed) s_changed[t & 1] = 1;
+      __syncthreads();
+      // each slot's next v2c
+      eNext = tid < E ? gslot[tid] : 0u;
+      for (int l = tid; l < E; l += T) {
+        const uint32_t e = eNext;
+        if (l + T < E) eNext = gslot[l + T];
+        const float tot = colTot[e >> 13];
+        const float v2c = tot - phi[l];
+        const uint32_t sg = ir_f2u(v2c) >> 31;
+        const float v = phi_of((sg ? -1.0f : 1.0f) * v2c);
+        phi[l] = ir_u2f((ir_f2u(v) & 0x7fffffffu) | (sg << 31));
+        // lanes of a wave hold 64 consecutive slots, those past E inactive (0)
+        const uint64_t bal = __ballot(mode1 ? tot < 0.0f : ir_f2u(tot) >> 31 != 0u);
+        if (lane == 0) slotDec[l >> 6] = bal;
+      }
       __syncthreads();
     }
 
@@ -287,11 +317,9 @@ __global__ __launch_bounds__(kIrregThreads) void bp_irregular_kernel(BpArgs a) {
 }
 
 hipError_t launch_bp_irregular(const BpArgs &a, int grid, hipStream_t s) {
-  if (a.lad.N > IR_NMAX || a.lad.E > IR_EMAX || !a.lad.colSlots) return hipErrorInvalidValue;
-  if (a.mode == 1)
-    hipLaunchKernelGGL(bp_irregular_kernel<true>, dim3(grid), dim3(kIrregThreads), 0, s, a);
-  else
-    hipLaunchKernelGGL(bp_irregular_kernel<false>, dim3(grid), dim3(kIrregThreads), 0, s, a);
+  if (a.lad.N > IR_NMAX || a.lad.E > IR_EMAX || !a.lad.slotEdges) return hipErrorInvalidValue;
+  if (a.mode == 1) hipLaunchKernelGGL((bp_irregular_kernel<true>), dim3(grid), dim3(IR_T), 0, s, a);
+  else hipLaunchKernelGGL((bp_irregular_kernel<false>), dim3(grid), dim3(IR_T), 0, s, a);
   return hipGetLastError();
 }
 

@@ -54,12 +54,11 @@ struct ColEdges {
 
 struct LadderDev {
   int N, E, numCodes;
-  int regular;           // every column has degree 3 (colRows), else colEdges/jc/colSlots
+  int regular;           // every column has degree 3 (colRows), else slotEdges/jc/colSlots
   const ColEdges *colRows;  // per code and column: its three edges as row | message slot << 15
-  const uint32_t *colEdges;  // irregular: per code and edge (column order) row | rank << 16
-  const int *jc;             // irregular: column pointers
-  const int16_t *colSlots;   // irregular: columns of each of kIrregThreads threads (-1: none)
-  int colSlotsPerThread;
+  const uint32_t *slotEdges;  // irregular: per code and message slot (row order) row | column << 13
+  const int *jc;              // irregular: column pointers
+  const uint16_t *colSlots;   // irregular: per code and edge (column order) its message slot
   const uint16_t *rowPtr, *tx;
   const int *syndLength;
   const uint8_t *invH, *crcBasis;
@@ -115,7 +114,7 @@ hipError_t launch_mode1_resolve(const PlaneDesc *planes, int n, int numCodes, in
 // counters (queue head, decision slots handed out, bitplanes to resume).
 hipError_t launch_ce_llr(const PlaneDesc *d_planes, int n, int fixed_start, const Ladder &l1584,
                          const Ladder &l6336, int *counters, hipStream_t s);
-// BP on an irregular ladder (bp_irregular_kernel, kIrregThreads per workgroup).
+// BP on an irregular ladder (bp_irregular_kernel).
 hipError_t launch_bp_irregular(const BpArgs &a, int grid, hipStream_t s);
 // Full-rate inverse of the bitplanes whose BP codes all failed, bitplane p's
 // into decision slot slot0 + p.
