@@ -26,7 +26,17 @@ static std::string default_data_dir() {
   return "data";
 }
 
-int bp_threads(const dvc_ctx *c, int N) { return N == 1584 ? c->bp_threads_qcif : c->bp_threads_cif; }
+int bp_threads(const dvc_ctx *c, int N, int planes) {
+  if (N != 1584) return c->bp_threads_cif;
+  // A QCIF launch whose bitplanes need fewer codewords than there are CUs (about
+  // eight codes each; the searches try 5 on average, rarely more than 12) is bound
+  // by one codeword's latency, which 16 waves cut by a tenth; more bitplanes run
+  // faster with several smaller workgroups per CU.  ms with 512 and 1024 threads:
+  // 1 bitplane 0.307 and 0.276, 8 0.399 and 0.373, 32 0.56 and 0.48, 64 0.776 and
+  // 0.804, 128 1.30 and 1.37, 256 2.33 and 2.50.
+  if (8 * planes <= c->sm_count) return 1024;
+  return c->bp_threads_qcif;
+}
 
 int bp_grid(const dvc_ctx *c, int N, int items) {
   // a CIF codeword takes 126 KB of a CU's 160 KB LDS, an irregular QCIF codeword's
@@ -303,7 +313,7 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     DVC_HIP(hipStreamSynchronize(s));
   }
 
-  const int threads = bp_threads(c, N);
+  const int threads = bp_threads(c, N, n);
   LadderDev ld = ladder_dev(*L);
   std::vector<int4> rec((size_t)n * C);
   if (perCode) {

@@ -69,9 +69,10 @@ struct Ladder {
 
 // Loads dir/<kind><N>.ladder (kind "reg" or "irreg") and its cached inverse.
 int load_ladder(const std::string &dir, const char *kind, int N, Ladder &L);
-// BP launch shape of the context's tuning: threads per workgroup and the
-// persistent grid for `items` queued (bitplane, code) items.
-int bp_threads(const dvc_ctx *c, int N);
+// BP launch shape: threads per workgroup for a launch of `planes` bitplanes, and
+// the persistent grid for `items` queued (bitplane, code) items (the context's
+// tuning, but for small QCIF launches).
+int bp_threads(const dvc_ctx *c, int N, int planes);
 int bp_grid(const dvc_ctx *c, int N, int items);
 int upload_ladder(Ladder &L);
 // Quantisation table entry Qtable[q][index] (reconstruction.cpp:9-78), 0 outside 1..8 x 0..15.

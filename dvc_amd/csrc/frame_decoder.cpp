@@ -242,7 +242,7 @@ int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, uint8_t *d_sl
   Ladder *L = c->ladder(N);
   const int C = L->numCodes;
   LadderDev ld = ladder_dev(*L);
-  const int threads = bp_threads(c, N);
+  const int threads = bp_threads(c, N, sequential ? 1 : n);
   const int maxOff = C - 1;
   const char *name = N == 6336 ? "bp_6336" : "bp_1584";
   TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
@@ -283,7 +283,7 @@ int dvc::bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, 
   Ladder *L = c->ladder(N);
   const int n = (int)planes.size(), C = L->numCodes;
   LadderDev ld = ladder_dev(*L);
-  const int threads = bp_threads(c, N);
+  const int threads = bp_threads(c, N, 1);
   TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
   // Every host-side source below stays alive until the stream is drained.
   std::vector<PlaneState> st(n);

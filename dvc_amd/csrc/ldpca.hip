@@ -685,6 +685,7 @@ hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStrea
     if (threads == 512) return launch_bp<6336, 512>(a, grid, s);
     return launch_bp<6336, 1024>(a, grid, s);
   }
+  if (threads == 1024) return launch_bp<1584, 1024>(a, grid, s);
   if (threads == 512) return launch_bp<1584, 512>(a, grid, s);
   return launch_bp<1584, 256>(a, grid, s);
 }

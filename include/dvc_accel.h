@@ -146,7 +146,8 @@ int dvc_ldpca_decode_batch_noalloc(dvc_ctx *ctx, int n, dvc_ldpca_item *items);
  * returns it.  The choice changes time only, never results. */
 typedef struct {
   int cif_threads;      /* threads per workgroup for N = 6336: 512, 704 or 1024 */
-  int qcif_threads;     /* threads per workgroup for N = 1584: 256 or 512 */
+  int qcif_threads;     /* threads per workgroup for N = 1584: 256 or 512 (launches of few
+                           bitplanes use 1024 whatever is set) */
   int qcif_wg_per_cu;   /* QCIF codewords (workgroups) per CU in the persistent grid: 1..4 */
   int poll;             /* BP iterations between a speculative item's cancellation polls: 1..8 */
   double cif_ms, qcif_ms;  /* dvc_autotune: calibration time of the chosen variant */
