@@ -5,6 +5,7 @@
 #include <string.h>
 #include <dlfcn.h>
 #include <string>
+#include <thread>
 #include <vector>
 #include <algorithm>
 #include "dvc_internal.h"
@@ -38,11 +39,25 @@ int bp_threads(const dvc_ctx *c, int N, int planes) {
   return c->bp_threads_qcif;
 }
 
-int bp_grid(const dvc_ctx *c, int N, int items) {
+int bp_grid(const dvc_ctx *c, int N, int items, int planes, int other) {
   // a CIF codeword takes 126 KB of a CU's 160 KB LDS, an irregular QCIF codeword's
   // 16 waves its registers; regular QCIF codewords (38 KB, 8 waves) share one
   const int perCU = N == 6336 || !c->lad1584.regular ? 1 : c->bp_wg_per_cu_qcif;
-  return std::max(1, std::min(c->sm_count * perCU, items));
+  // Two launches at once that fill the chip for a round or two of codes (eight per
+  // bitplane) share its CUs by their work: a CIF codeword's iteration takes four
+  // times a QCIF one's, 2.5 times an irregular one's.  Either would take all CUs
+  // for its speculative codes and the other wait for the last of them (60 mixed
+  // bitplanes 2.20 ms, shared 1.65).  Larger pairs keep full grids: the second
+  // fills the CUs that the first one's tail leaves, where a share would idle (512
+  // bitplanes 19.0 ms shared, 15.4 so, 16.1 one after the other).
+  int cus = c->sm_count;
+  if (other > 0) {
+    const double cif = N == 6336 ? planes : other, qcif = N == 6336 ? other : planes;
+    const double wq = qcif * (c->lad1584.regular ? 0.25 : 0.4), part = (N == 6336 ? cif : wq) / (cif + wq);
+    if (8 * (cif + wq) <= 2 * c->sm_count)
+      cus = std::max(1, std::min(c->sm_count - 1, (int)(c->sm_count * part + 0.5)));
+  }
+  return std::max(1, std::min(cus * perCU, items));
 }
 
 }  // namespace dvc
@@ -135,6 +150,7 @@ int dvc_ctx_create(const dvc_params *params, dvc_ctx **out) {
     return rc;
   }
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking);
   if (e != hipSuccess) { dvc_ctx_destroy(c); set_error("hipStreamCreate failed"); return DVC_EDEVICE; }
   if ((rc = noalloc_attach(c))) {
     dvc_ctx_destroy(c);
@@ -154,10 +170,13 @@ int dvc_ctx_destroy(dvc_ctx *c) {
   if (c->si_scratch) (void)hipFree(c->si_scratch);
   if (c->si_host) (void)hipHostFree(c->si_host);
   host_pool_free(c);
-  if (c->ld_dev) (void)hipFree(c->ld_dev);
-  if (c->ld_host) (void)hipHostFree(c->ld_host);
+  for (auto &w : c->ld) {
+    if (w.dev) (void)hipFree(w.dev);
+    if (w.host) (void)hipHostFree(w.host);
+  }
   band_free(c);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  if (c->stream2) (void)hipStreamDestroy(c->stream2);
   delete c;
   return DVC_OK;
 }
@@ -242,22 +261,22 @@ static LdpcaLayout ldpca_layout(size_t n, size_t N, size_t C, size_t slotCap, bo
   return o;
 }
 
-// Grows the context's LDPCA workspace (device) and its pinned staging (host);
+// Grows a code length's LDPCA workspace (device) and its pinned staging (host);
 // both are kept between calls and freed by dvc_ctx_destroy.
-static int ldpca_workspace(dvc_ctx *c, size_t devBytes, size_t hostBytes) {
-  if (c->ld_dev_bytes < devBytes) {
-    if (c->ld_dev) DVC_HIP(hipFree(c->ld_dev));
-    c->ld_dev = nullptr;
-    c->ld_dev_bytes = 0;
-    DVC_HIP(hipMalloc(&c->ld_dev, devBytes));
-    c->ld_dev_bytes = devBytes;
+static int ldpca_workspace(dvc_ctx::LdWork &w, size_t devBytes, size_t hostBytes) {
+  if (w.devBytes < devBytes) {
+    if (w.dev) DVC_HIP(hipFree(w.dev));
+    w.dev = nullptr;
+    w.devBytes = 0;
+    DVC_HIP(hipMalloc(&w.dev, devBytes));
+    w.devBytes = devBytes;
   }
-  if (c->ld_host_bytes < hostBytes) {
-    if (c->ld_host) DVC_HIP(hipHostFree(c->ld_host));
-    c->ld_host = nullptr;
-    c->ld_host_bytes = 0;
-    DVC_HIP(hipHostMalloc(&c->ld_host, hostBytes, hipHostMallocDefault));
-    c->ld_host_bytes = hostBytes;
+  if (w.hostBytes < hostBytes) {
+    if (w.host) DVC_HIP(hipHostFree(w.host));
+    w.host = nullptr;
+    w.hostBytes = 0;
+    DVC_HIP(hipHostMalloc(&w.host, hostBytes, hipHostMallocDefault));
+    w.hostBytes = hostBytes;
   }
   return DVC_OK;
 }
@@ -271,16 +290,18 @@ static int ldpca_workspace(dvc_ctx *c, size_t devBytes, size_t hostBytes) {
 // launches each code by itself with the decisions the one before it left.
 // ParallelMode 1: items[i].decoded holds the decisions carried into the
 // bitplane's first code on entry (the reference's in/out decoded buffer).
-static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int sequential, hipStream_t s) {
+// other: bitplanes of the other code length decoded at the same time.
+static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int sequential, int other, hipStream_t s) {
   Ladder *L = c->ladder(N);
   const int C = L->numCodes, nb = N / 8;
   const bool mode1 = c->bp_mode == 1;
   const bool perCode = sequential && mode1;
   const SlotPlan slots = slot_plan(n, C, c->bp_mode);
   const LdpcaLayout o = ldpca_layout(n, N, C, slots.total, mode1);
-  int rc = ldpca_workspace(c, o.total, o.outEnd);
+  dvc_ctx::LdWork &work = c->ld[N == 6336];
+  int rc = ldpca_workspace(work, o.total, o.outEnd);
   if (rc) return rc;
-  uint8_t *dev = (uint8_t *)c->ld_dev, *host = (uint8_t *)c->ld_host;
+  uint8_t *dev = (uint8_t *)work.dev, *host = (uint8_t *)work.host;
   float *dLR = (float *)(dev + o.lr), *dLLR = (float *)(dev + o.llr);
   uint8_t *dAcc = dev + o.acc, *dCarry = dev + o.carry, *dSlots = dev + o.slots, *dOut = dev + o.out;
   PlaneDesc *dPlanes = (PlaneDesc *)(dev + o.planes);
@@ -352,7 +373,7 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     const int maxOff = C - 1;
     BpArgs a{ld, dPlanes, n, dCounters, n * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, slots.bp,
              c->bp_poll, c->bp_mode, c->rate_step};
-    const int grid = sequential ? 1 : bp_grid(c, N, n * maxOff);
+    const int grid = sequential ? 1 : bp_grid(c, N, n * maxOff, n, other);
     TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, grid, s));
     for (int round = 0; mode1; round++) {
       // ParallelMode 1: resolve with the carried decisions; resume the
@@ -423,7 +444,7 @@ int dvc_ldpca_decode(dvc_ctx *c, int N, const float *LR, const uint8_t *acc, uin
   DVC_CHECK(c->ladder(N), DVC_EINVAL, "dvc_ldpca_decode: N must be 1584 or 6336");
   DVC_HIP(hipSetDevice(c->device));
   dvc_ldpca_item it{N, LR, acc, crc, start_level, decoded, {}};
-  int rc = decode_group(c, N, 1, &it, 1, c->stream);
+  int rc = decode_group(c, N, 1, &it, 1, 0, c->stream);
   if (rc == DVC_OK && stats) *stats = it.stats;
   return rc;
 }
@@ -440,10 +461,37 @@ int dvc_ldpca_decode_batch(dvc_ctx *c, int n, dvc_ldpca_item *items) {
     g[k].push_back(items[i]);
     gi[k].push_back(i);
   }
+  // both code lengths at once, each on its own stream and host thread: one after
+  // the other, the second waited for the last codes of the first (see bp_grid)
+  int rcs[2] = {DVC_OK, DVC_OK};
+  std::string err[2];
+  auto run = [&](int k, hipStream_t s) {
+    if (hipSetDevice(c->device) != hipSuccess) {
+      rcs[k] = DVC_EDEVICE;
+      err[k] = "hipSetDevice failed";
+      return;
+    }
+    rcs[k] = decode_group(c, k ? 6336 : 1584, (int)g[k].size(), g[k].data(), 0, (int)g[1 - k].size(), s);
+    if (rcs[k]) err[k] = dvc_last_error();
+  };
+  if (!g[0].empty() && !g[1].empty()) {
+    std::thread th;
+    try {
+      th = std::thread(run, 0, c->stream2);
+    } catch (...) {  // no thread to be had: on this one, first
+    }
+    if (!th.joinable()) run(0, c->stream2);
+    run(1, c->stream);
+    if (th.joinable()) th.join();
+  } else {
+    for (int k = 0; k < 2; k++)
+      if (!g[k].empty()) run(k, c->stream);
+  }
   for (int k = 0; k < 2; k++) {
-    if (g[k].empty()) continue;
-    int rc = decode_group(c, k ? 6336 : 1584, (int)g[k].size(), g[k].data(), 0, c->stream);
-    if (rc) return rc;
+    if (rcs[k]) {
+      set_error(err[k]);
+      return rcs[k];
+    }
     for (size_t j = 0; j < g[k].size(); j++) items[gi[k][j]].stats = g[k][j].stats;
   }
   return DVC_OK;

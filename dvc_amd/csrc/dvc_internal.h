@@ -70,10 +70,11 @@ struct Ladder {
 // Loads dir/<kind><N>.ladder (kind "reg" or "irreg") and its cached inverse.
 int load_ladder(const std::string &dir, const char *kind, int N, Ladder &L);
 // BP launch shape: threads per workgroup for a launch of `planes` bitplanes, and
-// the persistent grid for `items` queued (bitplane, code) items (the context's
+// the persistent grid for its `items` queued (bitplane, code) items beside a
+// concurrent launch of `other` bitplanes of the other code length (the context's
 // tuning, but for small QCIF launches).
 int bp_threads(const dvc_ctx *c, int N, int planes);
-int bp_grid(const dvc_ctx *c, int N, int items);
+int bp_grid(const dvc_ctx *c, int N, int items, int planes, int other);
 int upload_ladder(Ladder &L);
 // Quantisation table entry Qtable[q][index] (reconstruction.cpp:9-78), 0 outside 1..8 x 0..15.
 int qtable_entry(int q, int index);
@@ -143,10 +144,13 @@ struct dvc_ctx {
   uint8_t *si_host = nullptr;  // its pinned host staging, and the per-band entry points'
   size_t si_host_bytes = 0;
   dvc::HostPool *pool = nullptr;  // host copy threads (made on first use)
-  void *ld_dev = nullptr;      // the LDPCA entry points' device workspace, kept between calls
-  size_t ld_dev_bytes = 0;
-  void *ld_host = nullptr;     // its pinned host staging (inputs up, results back)
-  size_t ld_host_bytes = 0;
+  // the LDPCA entry points' workspaces, one per code length (1584, 6336), kept
+  // between calls: device memory and pinned staging (inputs up, results back)
+  struct LdWork {
+    void *dev = nullptr, *host = nullptr;
+    size_t devBytes = 0, hostBytes = 0;
+  } ld[2];
+  hipStream_t stream2 = nullptr;  // the second code length of a mixed batch
   void *noalloc_scratch = nullptr;  // device address of noalloc.hip's scratch array on this device
   dvc::BandState *band = nullptr;   // per-band entry points' frame state (dvc_band_frame_init)
   dvc::Ladder *ladder(int N) { return N == 1584 ? &lad1584 : (N == 6336 ? &lad6336 : nullptr); }

@@ -228,8 +228,9 @@ int ensure_cost_tables(dvc_ctx *c) {
 // descriptors in d_planes): entropy and LLR, the persistent BP launch and the
 // full-rate inverse.  In ParallelMode 0 these are kernel launches only, so a
 // stream capture of them replays.  sequential: the plain search, a launch of one
-// workgroup per bitplane, which takes the codes one after another.
-int bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, uint8_t *d_slots, const SlotPlan &slots,
+// workgroup per bitplane, which takes the codes one after another.  other:
+// bitplanes of the other code length that a concurrent step decodes.
+int bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, uint8_t *d_slots, const SlotPlan &slots,
                    int *d_counters, PlaneDesc *d_planes, hipStream_t s);
 // The plain search in ParallelMode 1: a launch per code, each with the decisions
 // the code before it left.
@@ -237,8 +238,8 @@ int bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, uint8
                   int *d_counters, PlaneDesc *d_planes, hipStream_t s);
 }  // namespace dvc
 
-int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, uint8_t *d_slots, const SlotPlan &slots,
-                        int *d_counters, PlaneDesc *d_planes, hipStream_t s) {
+int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, uint8_t *d_slots,
+                        const SlotPlan &slots, int *d_counters, PlaneDesc *d_planes, hipStream_t s) {
   Ladder *L = c->ladder(N);
   const int C = L->numCodes;
   LadderDev ld = ladder_dev(*L);
@@ -257,7 +258,7 @@ int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, uint8_t *d_sl
       TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, 1, s));
     }
   } else {
-    const int grid = bp_grid(c, N, n * maxOff);
+    const int grid = bp_grid(c, N, n * maxOff, n, other);
     TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, grid, s));
     for (int round = 0; c->bp_mode == 1; round++) {
       // ParallelMode 1: resolve with the carried decisions and resume the
@@ -335,7 +336,8 @@ constexpr int kStageRing = 4;
 // of one lane's LDPCA launch and its host round trips overlap the other
 // lanes' kernels.
 struct Lane {
-  hipStream_t s = nullptr;
+  hipStream_t s = nullptr, s2 = nullptr;  // s2: QCIF bitplanes beside CIF ones
+  hipEvent_t fork = nullptr, join = nullptr;
   int cap = 0;
   SlotPlan slots{};  // decision slots of each code length
   std::vector<Job *> inflight;
@@ -758,18 +760,30 @@ static int lane_step(dvc_engine *e, Lane &ln) {
     // length, bitplane insertion
     auto launches = [&]() -> int {
       TIMED_LAUNCH(c, "condbit", s, launch_condbit(ln.d_frames, L0, na, maxN, s));
+      // both code lengths' bitplanes at once, QCIF's on the lane's second stream
+      // (ParallelMode 1 and the plain search wait for one another on the host)
+      const bool both = n0 && n1 && !e->sequentialBp && c->bp_mode == 0;
+      if (both) {
+        DVC_HIP(hipEventRecord(ln.fork, s));
+        DVC_HIP(hipStreamWaitEvent(ln.s2, ln.fork, 0));
+      }
       int off = 0;
       for (int g = 0; g < 2; g++) {
         const int ng = g ? n1 : n0;
         if (!ng) continue;
+        hipStream_t gs = both && g == 0 ? ln.s2 : s;
         uint8_t *slots = ln.d_slots + (size_t)(g ? ln.slots.total : 0) * 6336;
         const int r = e->sequentialBp && c->bp_mode == 1
                           ? bp_step_codes(c, g ? 6336 : 1584, ln.groups[g], slots, ln.slots, ln.d_counters + 3 * g,
-                                          ln.d_planes + off, s)
-                          : bp_step_launch(c, g ? 6336 : 1584, ng, e->sequentialBp, slots, ln.slots,
-                                           ln.d_counters + 3 * g, ln.d_planes + off, s);
+                                          ln.d_planes + off, gs)
+                          : bp_step_launch(c, g ? 6336 : 1584, ng, e->sequentialBp, both ? (g ? n0 : n1) : 0, slots,
+                                           ln.slots, ln.d_counters + 3 * g, ln.d_planes + off, gs);
         if (r) return r;
         off += ng;
+      }
+      if (both) {
+        DVC_HIP(hipEventRecord(ln.join, ln.s2));
+        DVC_HIP(hipStreamWaitEvent(s, ln.join, 0));
       }
       TIMED_LAUNCH(c, "put_bitplane", s, launch_put_bitplane(ln.d_frames, L0, ln.d_links, na, maxN, s));
       return DVC_OK;
@@ -1020,6 +1034,9 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
     l.oSegs = align_up(l.oPlanes + sizeof(PlaneDesc) * M);
     l.stageBytes = align_up(l.oSegs + sizeof(CopySeg) * 4 * M);
     err = hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking);
+    if (err == hipSuccess) err = hipStreamCreateWithFlags(&l.s2, hipStreamNonBlocking);
+    for (hipEvent_t *ev : {&l.fork, &l.join})
+      if (err == hipSuccess) err = hipEventCreateWithFlags(ev, hipEventDisableTiming);
     if (err == hipSuccess) err = hipHostMalloc((void **)&l.h_stage, l.stageBytes * kStageRing, hipHostMallocDefault);
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_stage, l.stageBytes);
     for (int r = 0; r < kStageRing && err == hipSuccess; r++) err = hipEventCreateWithFlags(&l.staged[r], hipEventDisableTiming);
@@ -1048,7 +1065,8 @@ static void engine_destroy(dvc_engine *e) {
   (void)hipSetDevice(e->c->device);
   (void)hipStreamSynchronize(e->c->stream);
   for (auto &l : e->lanes)
-    if (l.s) (void)hipStreamSynchronize(l.s);
+    for (hipStream_t s : {l.s, l.s2})
+      if (s) (void)hipStreamSynchronize(s);
   for (Job *j : e->pending) delete j;
   for (auto &l : e->lanes) {
     for (Job *j : l.inflight) { if (j->mem) (void)hipFree(j->mem); delete j; }
@@ -1061,7 +1079,10 @@ static void engine_destroy(dvc_engine *e) {
     for (hipEvent_t e : l.staged)
       if (e) (void)hipEventDestroy(e);
     if (l.h_out) (void)hipHostFree(l.h_out);
+    for (hipEvent_t ev : {l.fork, l.join})
+      if (ev) (void)hipEventDestroy(ev);
     if (l.s) (void)hipStreamDestroy(l.s);
+    if (l.s2) (void)hipStreamDestroy(l.s2);
   }
   for (auto &kv : e->keys) (void)hipFree(kv.second.k.full);
   for (auto &kv : e->pool) (void)hipFree(kv.second);

@@ -202,7 +202,7 @@ extern "C" int dvc_ldpca_decode_batch_noalloc(dvc_ctx *c, int n, dvc_ldpca_item 
     const LadderDev ld = ladder_dev(*L);
     BpArgs a{ld, dPlanes, ng, dCounters, ng * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, sp.bp,
              c->bp_poll, c->bp_mode, c->rate_step};
-    DVC_HIP(launch_bp_any(N, bp_threads(c, N, ng), a, bp_grid(c, N, ng * maxOff), s));
+    DVC_HIP(launch_bp_any(N, bp_threads(c, N, ng), a, bp_grid(c, N, ng * maxOff, ng, 0), s));
     DVC_HIP(launch_invh(dPlanes, ng, ld, dSlots, sp.bp, s));
     hipLaunchKernelGGL(noalloc_finish_kernel, dim3(ng), dim3(128), 0, s, dItems, dIndex, dState, dRec, dSlots, sp.total,
                        N, C, L->d_syndLength, c->rate_step, dErr);
