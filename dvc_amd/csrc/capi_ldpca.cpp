@@ -39,25 +39,55 @@ int bp_threads(const dvc_ctx *c, int N, int planes) {
   return c->bp_threads_qcif;
 }
 
+// CUs of a launch beside a concurrent one of `other` bitplanes of the other code
+// length.  Two launches at once that fill the chip for a round or two of codes
+// (eight per bitplane) share its CUs by their work: a CIF codeword's iteration
+// takes four times a QCIF one's, 2.5 times an irregular one's.  Either would take
+// all CUs for its speculative codes and the other wait for the last of them (60
+// mixed bitplanes 2.20 ms, shared 1.65).  Larger pairs keep full grids: the second
+// fills the CUs that the first one's tail leaves, where a share would idle (512
+// bitplanes 19.0 ms shared, 15.4 so, 16.1 one after the other).
+static int launch_cus(const dvc_ctx *c, int N, int planes, int other) {
+  if (other <= 0) return c->sm_count;
+  const double cif = N == 6336 ? planes : other, qcif = N == 6336 ? other : planes;
+  const double wq = qcif * (c->lad1584.regular ? 0.25 : 0.4), part = (N == 6336 ? cif : wq) / (cif + wq);
+  if (8 * (cif + wq) > 2 * c->sm_count) return c->sm_count;
+  return std::max(1, std::min(c->sm_count - 1, (int)(c->sm_count * part + 0.5)));
+}
+
 int bp_grid(const dvc_ctx *c, int N, int items, int planes, int other) {
   // a CIF codeword takes 126 KB of a CU's 160 KB LDS, an irregular QCIF codeword's
   // 16 waves its registers; regular QCIF codewords (38 KB, 8 waves) share one
   const int perCU = N == 6336 || !c->lad1584.regular ? 1 : c->bp_wg_per_cu_qcif;
-  // Two launches at once that fill the chip for a round or two of codes (eight per
-  // bitplane) share its CUs by their work: a CIF codeword's iteration takes four
-  // times a QCIF one's, 2.5 times an irregular one's.  Either would take all CUs
-  // for its speculative codes and the other wait for the last of them (60 mixed
-  // bitplanes 2.20 ms, shared 1.65).  Larger pairs keep full grids: the second
-  // fills the CUs that the first one's tail leaves, where a share would idle (512
-  // bitplanes 19.0 ms shared, 15.4 so, 16.1 one after the other).
-  int cus = c->sm_count;
-  if (other > 0) {
-    const double cif = N == 6336 ? planes : other, qcif = N == 6336 ? other : planes;
-    const double wq = qcif * (c->lad1584.regular ? 0.25 : 0.4), part = (N == 6336 ? cif : wq) / (cif + wq);
-    if (8 * (cif + wq) <= 2 * c->sm_count)
-      cus = std::max(1, std::min(c->sm_count - 1, (int)(c->sm_count * part + 0.5)));
+  return std::max(1, std::min(launch_cus(c, N, planes, other) * perCU, items));
+}
+
+// Workgroups per CIF codeword (1: the persistent kernel).  A launch's CUs are
+// shared among the codewords its bitplanes need (about eight each), up to the
+// eight that a codeword can use.  Four per codeword still pay when a quarter of
+// the codes has to wait for a cluster (10 bitplanes, unsplit 0.93 ms a batch: 4
+// workgroups 0.66, 3 0.74, 2 0.86); with more than that waiting the gain is gone or
+// hangs on how many codes the bitplanes need (16: 0.91 against 0.99, 20: 1.12
+// against 1.02).  One bitplane: 0.84 unsplit, 0.48 with 4, 0.42 with 8.  A QCIF
+// codeword's iteration is shorter than an exchange between workgroups: never.
+static int bp_split(const dvc_ctx *c, int N, int planes, int other, int lanes, bool sequential, const BpArgs &a) {
+  if (!a.area || N != 6336 || !a.lad.regular || a.max_iter < 1) return 1;
+  const int cus = launch_cus(c, N, planes, other) / lanes, codewords = sequential ? 1 : 8 * planes;
+  if (3 * codewords > cus) return 1;
+  return std::max(4, std::min(kSplitMax, cus / codewords));
+}
+
+hipError_t launch_bp(const dvc_ctx *c, int N, int planes, int other, int lanes, bool sequential, const BpArgs &a,
+                     hipStream_t s) {
+  const int split = bp_split(c, N, planes, other, lanes, sequential, a);
+  if (split > 1) {
+    BpArgs b = a;
+    b.split = split;
+    const int fit = launch_cus(c, N, planes, other) / lanes / split;
+    return launch_bp_split(N, b, sequential ? 1 : std::max(1, std::min({kSplitClusters, fit, a.total})), s);
   }
-  return std::max(1, std::min(cus * perCU, items));
+  return launch_bp_any(N, bp_threads(c, N, sequential ? 1 : planes), a,
+                       sequential ? 1 : bp_grid(c, N, a.total, planes, other), s);
 }
 
 }  // namespace dvc
@@ -233,7 +263,7 @@ int dvc_ladder_export(dvc_ctx *c, int N, int code, int *ir_out, uint8_t *inv_out
 // The input region [lr, inEnd) is filled in pinned host memory at the same
 // offsets and uploaded in one copy; [state, outEnd) comes back in one copy.
 struct LdpcaLayout {
-  size_t lr, acc, carry, planes, state, rec, counters, inEnd, out, outEnd, llr, slots, bcase, total;
+  size_t lr, acc, carry, planes, state, rec, counters, inEnd, out, outEnd, llr, slots, bcase, area, total;
 };
 
 static LdpcaLayout ldpca_layout(size_t n, size_t N, size_t C, size_t slotCap, bool mode1) {
@@ -257,6 +287,7 @@ static LdpcaLayout ldpca_layout(size_t n, size_t N, size_t C, size_t slotCap, bo
   o.llr = take(sizeof(float) * n * N);
   o.slots = take(slotCap * N);
   o.bcase = take(mode1 ? sizeof(int) * n * C : 0);
+  o.area = take(N == 6336 ? sizeof(uint32_t) * split_area_words((int)N) : 0);
   o.total = at;
   return o;
 }
@@ -334,7 +365,6 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     DVC_HIP(hipStreamSynchronize(s));
   }
 
-  const int threads = bp_threads(c, N, n);
   LadderDev ld = ladder_dev(*L);
   std::vector<int4> rec((size_t)n * C);
   if (perCode) {
@@ -349,7 +379,8 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
         DVC_HIP(hipMemcpyAsync(dCounters, zero, sizeof(zero), hipMemcpyHostToDevice, s));
         BpArgs a{ld, dPlanes + i, 1, dCounters, 1, 1, c->max_iter, dSlots, dCounters + 1, slots.bp, c->bp_poll,
                  c->bp_mode, c->rate_step};
-        TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, 1, s));
+        a.area = (uint32_t *)(dev + o.area);
+        TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp(c, N, 1, 0, 1, true, a, s));
         DVC_HIP(hipMemcpyAsync(&r, dRec + (size_t)i * C + level, sizeof(r), hipMemcpyDeviceToHost, s));
         DVC_HIP(hipStreamSynchronize(s));
         if (r.y == REC_ACCEPTED) {
@@ -373,8 +404,8 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     const int maxOff = C - 1;
     BpArgs a{ld, dPlanes, n, dCounters, n * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, slots.bp,
              c->bp_poll, c->bp_mode, c->rate_step};
-    const int grid = sequential ? 1 : bp_grid(c, N, n * maxOff, n, other);
-    TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, grid, s));
+    a.area = (uint32_t *)(dev + o.area);
+    TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp(c, N, n, other, 1, sequential, a, s));
     for (int round = 0; mode1; round++) {
       // ParallelMode 1: resolve with the carried decisions; resume the
       // bitplanes that reach a code this launch did not finish
@@ -387,7 +418,7 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
       DVC_CHECK(resume < (1 << 20), DVC_ENOMEM, "ParallelMode 1: decision slots exhausted");
       if (!resume) break;
       DVC_HIP(launch_zero_ints(dCounters, 1, s));
-      TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, grid, s));
+      TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp(c, N, n, other, 1, sequential, a, s));
     }
     TIMED(c, "invh", s, launch_invh(dPlanes, n, ld, dSlots, slots.bp, s));
     // every bitplane's accepted decisions to dOut, then states, records,

@@ -75,6 +75,13 @@ int load_ladder(const std::string &dir, const char *kind, int N, Ladder &L);
 // tuning, but for small QCIF launches).
 int bp_threads(const dvc_ctx *c, int N, int planes);
 int bp_grid(const dvc_ctx *c, int N, int items, int planes, int other);
+// The BP launch of `planes` bitplanes' queued items (a.total of them): persistent,
+// or split over several workgroups per codeword when a.area is given and the
+// launch would leave most CUs idle.  lanes: launches like it that other streams
+// issue at the same time.  sequential: codes one after another.
+struct BpArgs;
+hipError_t launch_bp(const dvc_ctx *c, int N, int planes, int other, int lanes, bool sequential, const BpArgs &a,
+                     hipStream_t s);
 int upload_ladder(Ladder &L);
 // Quantisation table entry Qtable[q][index] (reconstruction.cpp:9-78), 0 outside 1..8 x 0..15.
 int qtable_entry(int q, int index);

@@ -228,38 +228,38 @@ int ensure_cost_tables(dvc_ctx *c) {
 // descriptors in d_planes): entropy and LLR, the persistent BP launch and the
 // full-rate inverse.  In ParallelMode 0 these are kernel launches only, so a
 // stream capture of them replays.  sequential: the plain search, a launch of one
-// workgroup per bitplane, which takes the codes one after another.  other:
-// bitplanes of the other code length that a concurrent step decodes.
-int bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, uint8_t *d_slots, const SlotPlan &slots,
-                   int *d_counters, PlaneDesc *d_planes, hipStream_t s);
+// codeword's workgroups per bitplane, which takes the codes one after another.  other:
+// bitplanes of the other code length that a concurrent step decodes, lanes those
+// that step at the same time.
+int bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, int lanes, uint8_t *d_slots,
+                   const SlotPlan &slots, int *d_counters, uint32_t *d_area, PlaneDesc *d_planes, hipStream_t s);
 // The plain search in ParallelMode 1: a launch per code, each with the decisions
 // the code before it left.
-int bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, uint8_t *d_slots, const SlotPlan &slots,
-                  int *d_counters, PlaneDesc *d_planes, hipStream_t s);
+int bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, int lanes, uint8_t *d_slots,
+                  const SlotPlan &slots, int *d_counters, uint32_t *d_area, PlaneDesc *d_planes, hipStream_t s);
 }  // namespace dvc
 
-int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, uint8_t *d_slots,
-                        const SlotPlan &slots, int *d_counters, PlaneDesc *d_planes, hipStream_t s) {
+int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, int lanes, uint8_t *d_slots,
+                        const SlotPlan &slots, int *d_counters, uint32_t *d_area, PlaneDesc *d_planes, hipStream_t s) {
   Ladder *L = c->ladder(N);
   const int C = L->numCodes;
   LadderDev ld = ladder_dev(*L);
-  const int threads = bp_threads(c, N, sequential ? 1 : n);
   const int maxOff = C - 1;
   const char *name = N == 6336 ? "bp_6336" : "bp_1584";
   TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
   BpArgs a{ld, d_planes, n, d_counters, n * maxOff, maxOff, c->max_iter, d_slots, d_counters + 1, slots.bp, c->bp_poll,
            c->bp_mode, c->rate_step};
+  a.area = d_area;
   if (sequential) {
     a.nplanes = 1;
     a.total = maxOff;
     for (int i = 0; i < n; i++) {
       if (i) DVC_HIP(launch_zero_ints(d_counters, 1, s));  // queue head only: the step's slots accumulate
       a.planes = d_planes + i;
-      TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, 1, s));
+      TIMED_LAUNCH(c, name, s, launch_bp(c, N, 1, 0, lanes, true, a, s));
     }
   } else {
-    const int grid = bp_grid(c, N, n * maxOff, n, other);
-    TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, grid, s));
+    TIMED_LAUNCH(c, name, s, launch_bp(c, N, n, other, lanes, false, a, s));
     for (int round = 0; c->bp_mode == 1; round++) {
       // ParallelMode 1: resolve with the carried decisions and resume the
       // bitplanes that reach a code the launch did not finish (host-synchronous)
@@ -272,19 +272,19 @@ int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, ui
       DVC_CHECK(resume < (1 << 20), DVC_ENOMEM, "ParallelMode 1: decision slots exhausted");
       if (!resume) break;
       DVC_HIP(launch_zero_ints(d_counters, 1, s));
-      TIMED_LAUNCH(c, name, s, launch_bp_any(N, threads, a, grid, s));
+      TIMED_LAUNCH(c, name, s, launch_bp(c, N, n, other, lanes, false, a, s));
     }
   }
   TIMED_LAUNCH(c, "invh", s, launch_invh(d_planes, n, ld, d_slots, slots.bp, s));
   return DVC_OK;
 }
 
-int dvc::bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, uint8_t *d_slots,
-                       const SlotPlan &slots, int *d_counters, PlaneDesc *d_planes, hipStream_t s) {
+int dvc::bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, int lanes, uint8_t *d_slots,
+                       const SlotPlan &slots, int *d_counters, uint32_t *d_area, PlaneDesc *d_planes,
+                       hipStream_t s) {
   Ladder *L = c->ladder(N);
   const int n = (int)planes.size(), C = L->numCodes;
   LadderDev ld = ladder_dev(*L);
-  const int threads = bp_threads(c, N, 1);
   TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
   // Every host-side source below stays alive until the stream is drained.
   std::vector<PlaneState> st(n);
@@ -302,7 +302,8 @@ int dvc::bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, 
       DVC_HIP(launch_zero_ints(d_counters, 1, s));  // queue head only: the step's slots accumulate
       BpArgs a{ld, d_planes + i, 1, d_counters, 1, 1, c->max_iter, d_slots, d_counters + 1, slots.bp, c->bp_poll,
                c->bp_mode, c->rate_step};
-      TIMED_LAUNCH(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp_any(N, threads, a, 1, s));
+      a.area = d_area;
+      TIMED_LAUNCH(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp(c, N, 1, 0, lanes, true, a, s));
       DVC_HIP(hipMemcpyAsync(&r, planes[i].rec + level, sizeof(r), hipMemcpyDeviceToHost, s));
       DVC_HIP(hipStreamSynchronize(s));
       if (r.y == REC_ACCEPTED) { ok = true; break; }
@@ -365,6 +366,7 @@ struct Lane {
   size_t outBytes = 0;
   uint8_t *d_slots = nullptr;
   int *d_counters = nullptr;
+  uint32_t *d_area = nullptr;  // split CIF BP launches meet here
   int rc = 0;
   std::string err;
   // host-side lists of one step
@@ -372,10 +374,11 @@ struct Lane {
   std::vector<PlaneDesc> groups[2];
   // Captured launch sequences of steady steps (no frame starts or ends a
   // band), keyed by their launch shape: frames stepped, planes of each code
-  // length, largest code length.  Their kernels read the step's frame list,
+  // length, largest code length, lanes stepping (which the BP launches share the
+  // CUs with).  Their kernels read the step's frame list,
   // frame descriptors and plane descriptors from this lane's buffers, which
   // are uploaded before each replay.
-  std::map<std::tuple<int, int, int, int>, hipGraphExec_t> graphs;
+  std::map<std::tuple<int, int, int, int, int>, hipGraphExec_t> graphs;
 };
 }  // namespace dvc
 
@@ -390,6 +393,7 @@ struct dvc_engine {
   uint64_t nextTicket = 1, clock = 0;
   std::deque<dvc::Job *> pending;
   std::vector<dvc::Lane> lanes;
+  int busyLanes = 1;  // lanes with frames in the current dvc_engine_step
   std::map<uint64_t, int> doneTickets;  // ticket -> 1
   std::map<uint64_t, dvc::KeyEntry> keys;
   // device blocks of retired frames and dropped key frames, kept for reuse
@@ -774,10 +778,11 @@ static int lane_step(dvc_engine *e, Lane &ln) {
         hipStream_t gs = both && g == 0 ? ln.s2 : s;
         uint8_t *slots = ln.d_slots + (size_t)(g ? ln.slots.total : 0) * 6336;
         const int r = e->sequentialBp && c->bp_mode == 1
-                          ? bp_step_codes(c, g ? 6336 : 1584, ln.groups[g], slots, ln.slots, ln.d_counters + 3 * g,
-                                          ln.d_planes + off, gs)
-                          : bp_step_launch(c, g ? 6336 : 1584, ng, e->sequentialBp, both ? (g ? n0 : n1) : 0, slots,
-                                           ln.slots, ln.d_counters + 3 * g, ln.d_planes + off, gs);
+                          ? bp_step_codes(c, g ? 6336 : 1584, ln.groups[g], e->busyLanes, slots, ln.slots,
+                                          ln.d_counters + 3 * g, g ? ln.d_area : nullptr, ln.d_planes + off, gs)
+                          : bp_step_launch(c, g ? 6336 : 1584, ng, e->sequentialBp, both ? (g ? n0 : n1) : 0, e->busyLanes,
+                                           slots, ln.slots, ln.d_counters + 3 * g, g ? ln.d_area : nullptr,
+                                           ln.d_planes + off, gs);
         if (r) return r;
         off += ng;
       }
@@ -792,7 +797,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
     const bool steady = e->graphs && !c->profiling && c->bp_mode == 0 && setup.empty() &&
                         starting.empty() && ending.empty();
     if (steady) {
-      const auto key = std::make_tuple(na, n0, n1, maxN);
+      const auto key = std::make_tuple(na, n0, n1, maxN, e->busyLanes);
       auto it = ln.graphs.find(key);
       if (it == ln.graphs.end()) {
         DVC_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -919,6 +924,7 @@ static int engine_step(dvc_engine *e, int *completed) {
   for (auto &l : e->lanes)
     if (!l.inflight.empty()) busy.push_back(&l);
   if (busy.empty()) return DVC_OK;
+  e->busyLanes = (int)busy.size();
   // a lane keeps stepping without waiting for the others until one of its
   // frames completes or lane_steps steps are done; one step while frames
   // wait for admission (the pending queue cannot change during the call)
@@ -1050,6 +1056,7 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
     }
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_slots, (size_t)2 * l.slots.total * 6336);
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_counters, 6 * sizeof(int));
+    if (err == hipSuccess) err = hipMalloc((void **)&l.d_area, sizeof(uint32_t) * split_area_words(6336));
   }
   if (err != hipSuccess) {
     set_error(std::string("dvc_engine_create: ") + hipGetErrorString(err));
@@ -1072,7 +1079,7 @@ static void engine_destroy(dvc_engine *e) {
     for (Job *j : l.inflight) { if (j->mem) (void)hipFree(j->mem); delete j; }
     for (Job *j : l.finished) { if (j->mem) (void)hipFree(j->mem); delete j; }
     for (auto &g : l.graphs) (void)hipGraphExecDestroy(g.second);
-    void *ptrs[] = {l.d_stage, l.d_out, l.d_slots, l.d_counters};
+    void *ptrs[] = {l.d_stage, l.d_out, l.d_slots, l.d_counters, l.d_area};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
     if (l.h_stage) (void)hipHostFree(l.h_stage);

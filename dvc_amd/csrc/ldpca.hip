@@ -173,6 +173,94 @@ struct BpShape {
   static constexpr int SYN_WORDS = (N + 31) / 32;
 };
 
+// One check's row of messages, slots e0 .. e1-1 of phi: |phi| summed in
+// ascending edge order (:514-515) and the messages' sign product; returns the
+// row's total with syn times that product in the sign bit.
+__device__ __forceinline__ float check_row(const float *phi, int e0, int e1, uint32_t syn) {
+  uint32_t sx = 0u;  // XOR of the row's message words: the sign product in bit 31
+  float sum = 0.0f;
+  // groups of four loads without conditions, then the last 1..3 slots
+  // read unconditionally too (the rows are contiguous and phi has spare
+  // slots at its end) with those past the row's end taken as +0: sum +
+  // 0.0f is sum bit for bit (sum is never -0)
+  int j = e0;
+  for (; j + 4 <= e1; j += 4) {
+    uint32_t f[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) f[i] = f2u(phi[j + i]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) sum += u2f(f[i] & 0x7fffffffu);
+    sx ^= f[0] ^ f[1] ^ f[2] ^ f[3];
+  }
+  if (j < e1) {
+    uint32_t f[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) f[i] = f2u(phi[j + i]);
+    f[1] = j + 1 < e1 ? f[1] : 0u;
+    f[2] = j + 2 < e1 ? f[2] : 0u;
+#pragma unroll
+    for (int i = 0; i < 3; i++) sum += u2f(f[i] & 0x7fffffffu);
+    sx ^= f[0] ^ f[1] ^ f[2];
+  }
+  return u2f(f2u(sum) | ((syn ^ (sx >> 31)) << 31));
+}
+
+// c2v of a column's three edges and its overall LLR (:512-539).
+template <bool MODE1, class Phi>
+__device__ __forceinline__ float column_total(const int row[3], const uint32_t pos[3], float llr, const float *rowTot,
+                                              float *phi, const Phi &phi_of, float c2v[3]) {
+  uint32_t R[3], ph[3];
+  float x[3], v[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    R[q] = f2u(rowTot[row[q]]);
+    ph[q] = f2u(at_byte(phi, pos[q]));
+  }
+#pragma unroll
+  for (int q = 0; q < 3; q++) x[q] = u2f(R[q] & 0x7fffffffu) - u2f(ph[q] & 0x7fffffffu);
+#pragma unroll
+  for (int q = 0; q < 3; q++) v[q] = phi_of(x[q]);
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+    // times -1 or 1 by the sign product; with no NaN (ParallelMode 0
+    // never runs a NaN bitplane) that is the sign bit flipped
+    c2v[q] = MODE1 ? (((R[q] ^ ph[q]) >> 31) ? v[q] * -1.0f : v[q] * 1.0f)
+                   : u2f((f2u(v[q]) & 0x7fffffffu) | ((f2u(v[q]) ^ R[q] ^ ph[q]) & 0x80000000u));
+  float tmp = llr;
+  tmp += c2v[0];
+  tmp += c2v[1];
+  tmp += c2v[2];
+  return tmp;
+}
+// The next v2c of the edges as messages: phi of the magnitude with the sign.
+template <class Phi>
+__device__ __forceinline__ void column_messages(float tmp, const float c2v[3], const Phi &phi_of, float f[3]) {
+  uint32_t sg[3];
+  float x[3], v[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    const float v2c = tmp - c2v[q];
+    sg[q] = f2u(v2c) >> 31;
+    x[q] = (sg[q] ? -1.0f : 1.0f) * v2c;
+  }
+#pragma unroll
+  for (int q = 0; q < 3; q++) v[q] = phi_of(x[q]);
+#pragma unroll
+  for (int q = 0; q < 3; q++) f[q] = copysignf(v[q], u2f(sg[q] << 31));
+}
+// A column's decision 1 XORed into its three checks' parity bits.
+__device__ __forceinline__ void column_parity(const ColEdges &rows, const int row[3], uint32_t *par) {
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    // word row >> 5 = bits 5..12 of the column word, extracted by one
+    // v_bfe_u32 (kept as written, so that the word's address is one
+    // shift-and-add); the bit's shift takes the row's low 5 bits
+    uint32_t w;
+    __asm__("v_bfe_u32 %0, %1, 5, 8" : "=v"(w) : "v"(rows.e[q]));
+    atomicXor(&par[w], 1u << (row[q] & 31));
+  }
+}
+
 // MODE1: beliefPropagation_OpenMP's semantics (ParallelMode 1), else
 // beliefPropagation's (ParallelMode 0).
 //
@@ -299,33 +387,7 @@ __global__ __launch_bounds__(T) void bp_persistent_kernel(BpArgs a) {
       for (int r = tid; r < m; r += T) {
         const int e0 = rowPtr[r], e1 = rowPtr[r + 1];
         const uint32_t syn = (synBits[r >> 5] >> (r & 31)) & 1u;
-        uint32_t sx = 0u;  // XOR of the row's message words: the sign product in bit 31
-        float sum = 0.0f;
-        // groups of four loads without conditions, then the last 1..3 slots
-        // read unconditionally too (the rows are contiguous and phi has spare
-        // slots at its end) with those past the row's end taken as +0: sum +
-        // 0.0f is sum bit for bit (sum is never -0)
-        int j = e0;
-        for (; j + 4 <= e1; j += 4) {
-          uint32_t f[4];
-#pragma unroll
-          for (int i = 0; i < 4; i++) f[i] = f2u(phi[j + i]);
-#pragma unroll
-          for (int i = 0; i < 4; i++) sum += u2f(f[i] & 0x7fffffffu);
-          sx ^= f[0] ^ f[1] ^ f[2] ^ f[3];
-        }
-        if (j < e1) {
-          uint32_t f[3];
-#pragma unroll
-          for (int i = 0; i < 3; i++) f[i] = f2u(phi[j + i]);
-          f[1] = j + 1 < e1 ? f[1] : 0u;
-          f[2] = j + 2 < e1 ? f[2] : 0u;
-#pragma unroll
-          for (int i = 0; i < 3; i++) sum += u2f(f[i] & 0x7fffffffu);
-          sx ^= f[0] ^ f[1] ^ f[2];
-        }
-        const uint32_t sgn = syn ^ (sx >> 31);
-        rowTot[r] = u2f(f2u(sum) | (sgn << 31));
+        rowTot[r] = check_row(phi, e0, e1, syn);
         if (t > 0 && (syn ^ ((parPrev[r >> 5] >> (r & 31)) & 1u))) fail = 1;
       }
       for (int wd = tid; wd < S::SYN_WORDS; wd += T) parBits[t & 1][wd] = 0u;
@@ -380,31 +442,10 @@ __global__ __launch_bounds__(T) void bp_persistent_kernel(BpArgs a) {
         uint32_t dec = 0;
         if (k < N) {
           float c2v[3];
-          uint32_t ph[3];
           int row[3];
           uint32_t pos[3];
           col_edges(rows, row, pos);
-          uint32_t R[3];
-          float x[3], v[3];
-#pragma unroll
-          for (int q = 0; q < 3; q++) {
-            R[q] = f2u(rowTot[row[q]]);
-            ph[q] = f2u(at_byte(phi, pos[q]));
-          }
-#pragma unroll
-          for (int q = 0; q < 3; q++) x[q] = u2f(R[q] & 0x7fffffffu) - u2f(ph[q] & 0x7fffffffu);
-#pragma unroll
-          for (int q = 0; q < 3; q++) v[q] = phi_of(x[q]);
-#pragma unroll
-          for (int q = 0; q < 3; q++)
-            // times -1 or 1 by the sign product; with no NaN (ParallelMode 0
-            // never runs a NaN bitplane) that is the sign bit flipped
-            c2v[q] = MODE1 ? (((R[q] ^ ph[q]) >> 31) ? v[q] * -1.0f : v[q] * 1.0f)
-                           : u2f((f2u(v[q]) & 0x7fffffffu) | ((f2u(v[q]) ^ R[q] ^ ph[q]) & 0x80000000u));
-          float tmp = llr;
-          tmp += c2v[0];
-          tmp += c2v[1];
-          tmp += c2v[2];
+          const float tmp = column_total<MODE1>(row, pos, llr, rowTot, phi, phi_of, c2v);
           if (!mode1) {
             dec = f2u(tmp) >> 31;
           } else {
@@ -412,28 +453,11 @@ __global__ __launch_bounds__(T) void bp_persistent_kernel(BpArgs a) {
             if (t == 0) changed |= !exact || as_global(pd.carry)[k] != (uint8_t)dec;
             else changed |= ((decBits[k >> 5] >> (k & 31)) & 1u) != dec;
           }
-          if (dec) {
+          if (dec) column_parity(rows, row, parBits[t & 1]);
+          float f[3];
+          column_messages(tmp, c2v, phi_of, f);
 #pragma unroll
-            for (int q = 0; q < 3; q++) {
-              // word row >> 5 = bits 5..12 of the column word, extracted by one
-              // v_bfe_u32 (kept as written, so that the word's address is one
-              // shift-and-add); the bit's shift takes the row's low 5 bits
-              uint32_t w;
-              __asm__("v_bfe_u32 %0, %1, 5, 8" : "=v"(w) : "v"(rows.e[q]));
-              atomicXor(&parBits[t & 1][w], 1u << (row[q] & 31));
-            }
-          }
-          uint32_t sg[3];
-#pragma unroll
-          for (int q = 0; q < 3; q++) {
-            const float v2c = tmp - c2v[q];
-            sg[q] = f2u(v2c) >> 31;
-            x[q] = (sg[q] ? -1.0f : 1.0f) * v2c;
-          }
-#pragma unroll
-          for (int q = 0; q < 3; q++) v[q] = phi_of(x[q]);
-#pragma unroll
-          for (int q = 0; q < 3; q++) at_byte(phi, pos[q]) = copysignf(v[q], u2f(sg[q] << 31));
+          for (int q = 0; q < 3; q++) at_byte(phi, pos[q]) = f[q];
         }
         const uint64_t bal = __ballot(dec);
         if (lane == 0) {
@@ -499,6 +523,350 @@ __global__ __launch_bounds__(T) void bp_persistent_kernel(BpArgs a) {
       pd.rec[level] = make_int4(iters, status == 1 ? 1 : (status == 3 ? 3 : 0), -1, 0);
     }
     if (tid == 0 && mode1) pd.bcase[level] = bcaseSlot;
+    __syncthreads();
+  }
+}
+
+// ------------------------------------------------------------------ split BP
+// A codeword on one CU is bound by that CU's VALU: 16 us per CIF iteration, with
+// most of the chip idle when a launch has few bitplanes.  Here a cluster of up to
+// 8 workgroups works on one codeword.  Every member holds the whole codeword's
+// messages in LDS and sums all rows, but updates only its share of the columns
+// (64-column groups, dealt round); after the variable pass the members exchange
+// their new messages and decisions through memory and go on with the same state,
+// so they take every decision alike and only the leader (member 0) reports.
+//
+// Exchange: agent-scope relaxed stores in column order (whole lines; each reader
+// puts the messages into row order itself, its column words loaded while it
+// waits), a wait for their completion, then the member's counter; the others poll
+// the counters and read with agent-scope loads.  Two buffers and two sets of
+// counters alternate, and either is rewritten only after a later exchange that
+// every reader of it has arrived at.  Every item handed to the members has at
+// least one exchange, so the leader does not hand out the next one before all of
+// them have seen it.
+//
+// No wait can be for a workgroup that is not running: a cluster is closed by its
+// leader with the members that have arrived within 30 us of it, a later one
+// leaves at once, and every wait is for members or the leader of a closed
+// cluster.  The polls are bounded all the same; a member that runs into the bound
+// leaves, and the host finds the records missing.
+//
+// With 8 members an iteration takes 7.2 us against 16: row sums 1.7, columns 1.4,
+// stores until complete 1.7, counters 1.0, reading and reordering 1.6.  A CIF
+// bitplane's batch decode 0.84 -> 0.42 ms, its plain search over 3 codes 2.16 ->
+// 1.08.  (Messages stored in row order, so that they are read without reordering:
+// 4-byte stores to as many lines, 0.62 and 1.66; parities taken from everybody's
+// decisions while reordering, the LDS atomics then on no arithmetic's back, 0.48
+// and 1.23.)
+template <int N, int T, bool MODE1>
+__global__ __launch_bounds__(T) void bp_split_kernel(BpArgs a) {
+  constexpr int NWS = (N + 63) / 64, SYN = (N + 31) / 32, W = T / 64;
+  constexpr size_t BUF = split_buf_words(N);
+  constexpr int PACK = 2, FLAG = 16, FLAG_STEP = 8;  // words of a control block
+  static_assert(FLAG + 2 * kSplitMax * FLAG_STEP <= kCtlWords, "control block too small");
+  constexpr int kSpin = 1 << 22;
+  __shared__ __align__(16) double s_phitab[2 * DVC_PHI_LOGTAB];
+  __shared__ __align__(16) float phi[3 * N + 4];
+  __shared__ float rowTot[N];
+  __shared__ uint16_t rowPtr[N + 2];
+  __shared__ uint32_t decBits[2 * NWS];
+  __shared__ uint32_t synBits[SYN], parBits[2 * NWS], parMine[2 * NWS];
+  __shared__ int s_item, s_size, s_rank, s_cluster, s_cancel, s_changed, s_abort;
+  __shared__ uint32_t s_crc[W];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const LadderDev L = a.lad;
+  for (int e = tid; e < DVC_PHI_LOGTAB; e += T) dvc_phi_logtab_entry(e, s_phitab);
+  auto ld32 = [](const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  auto ld64 = [](const uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  auto st32 = [](uint32_t *p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  auto st64 = [](uint64_t *p, uint64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+
+  // ---- join a cluster
+  if (tid == 0) {
+    const uint32_t ticket = __hip_atomic_fetch_add(a.area, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int cluster = (int)(ticket / (uint32_t)a.split);
+    uint32_t *state = a.area + (size_t)kCtlWords * (1 + cluster);  // members joined, bit 8: closed
+    s_cluster = cluster;
+    s_abort = 0;
+    if (ticket % (uint32_t)a.split == 0) {
+      const uint64_t t0 = wall_clock64();  // 100 MHz
+      while ((int)(ld32(state) & 0xffu) < a.split - 1 && wall_clock64() - t0 < 3000) __builtin_amdgcn_s_sleep(1);
+      const uint32_t old = __hip_atomic_fetch_or(state, 0x100u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      s_rank = 0;
+      s_size = 1 + (int)(old & 0xffu);
+    } else {
+      const uint32_t old = __hip_atomic_fetch_add(state, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      s_rank = (old & 0x100u) ? -1 : 1 + (int)(old & 0xffu);
+    }
+  }
+  __syncthreads();
+  const int rank = s_rank;
+  if (rank < 0) return;
+  uint32_t *ctl = a.area + (size_t)kCtlWords * (1 + s_cluster);
+  uint32_t *xbuf = a.area + kSplitCtlWords + (size_t)s_cluster * 2 * BUF;
+  uint32_t xc = 0;  // exchanges so far, over all items
+
+  for (uint32_t seq = 1;; seq++) {
+    // ---- the leader grabs the next item and hands it to the members with the
+    // cluster's size: (seq, size << 28 | item + 1) in one word
+    if (tid == 0) {
+      uint32_t low = 0;
+      if (rank == 0) {
+        int item = -1;
+        for (;;) {
+          const int w = atomicAdd(a.next, 1);
+          if (w >= a.total) break;
+          const int b = w % a.nplanes, off = w / a.nplanes;
+          PlaneState *st = a.planes[b].state;
+          const int level = st->run + off;
+          if (off >= a.max_offset || level >= L.numCodes - 1) continue;
+          if (a.rate_step && !dynstep_tries(off)) continue;
+          if (__hip_atomic_load(&st->best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < level) continue;
+          if (!MODE1 && st->taint) {
+            a.planes[b].rec[level] = make_int4(a.max_iter, REC_FAILED, -1, 0);
+            continue;
+          }
+          item = w;
+          break;
+        }
+        low = (uint32_t)s_size << 28 | (uint32_t)(item + 1);
+        st64((uint64_t *)(ctl + PACK), (uint64_t)seq << 32 | low);
+      } else {
+        for (int n = 0; n < kSpin; n++) {
+          const uint64_t v = ld64((const uint64_t *)(ctl + PACK));
+          if ((uint32_t)(v >> 32) == seq) {
+            low = (uint32_t)v;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+      }
+      s_item = (int)(low & 0x0fffffffu) - 1;
+      s_size = (int)(low >> 28);
+    }
+    __syncthreads();
+    const int w = s_item, size = s_size;
+    if (w < 0) return;
+    const int b = w % a.nplanes;
+    const PlaneDesc pd = a.planes[b];
+    PlaneState *st = pd.state;
+    const int run = st->run;
+    const int level = run + w / a.nplanes;
+    const bool taint = st->taint != 0;
+    auto phi_of = [&](float x) {
+      const float v = dvc_bp_phi_fast(x, s_phitab);
+      return (MODE1 && taint && x != x) ? x : v;
+    };
+    const bool mode1 = MODE1, exact = level == run;
+    const int m = L.syndLength[level];
+    const ColEdges *gcol = L.colRows + (size_t)level * N;
+    gfloat_t *gLLR = as_global(pd.LLR);
+
+    // ---- the code's row starts, the syndrome and the first messages, as in
+    // bp_persistent_kernel, on every member
+    const uint16_t *growPtr = L.rowPtr + (size_t)level * (N + 1);
+    for (int i = tid; i <= m; i += T) rowPtr[i] = growPtr[i];
+    for (int wd = tid; wd < SYN; wd += T) {
+      uint32_t bits = 0;
+      for (int q = 0; q < 32; q++) {
+        const int k = wd * 32 + q;
+        if (k < m) {
+          const int cur = L.tx[(size_t)level * N + k];
+          uint32_t s = acc_bit(as_global(pd.acc), cur);
+          if (k > 0) s ^= acc_bit(as_global(pd.acc), L.tx[(size_t)level * N + k - 1]);
+          bits |= s << q;
+        }
+      }
+      synBits[wd] = bits;
+    }
+    for (int k = tid; k < N; k += T) {
+      const float v = gLLR[k];
+      const float mag = (f2u(v) >> 31 ? -1.0f : 1.0f) * v;
+      const float f = copysignf(phi_of(mag), v);
+      int row[3];
+      uint32_t off[3];
+      col_edges(gcol[k], row, off);
+#pragma unroll
+      for (int q = 0; q < 3; q++) at_byte(phi, off[q]) = f;
+    }
+    if (tid == 0) s_cancel = s_changed = 0;
+    for (int wd = tid; wd < 2 * NWS; wd += T) parMine[wd] = 0u;
+    // this wave's first column group, the same in every iteration
+    const int k0 = (rank + size * wave) * 64 + lane;
+    const ColEdges rows0 = k0 < N ? gcol[k0] : ColEdges{{0u, 0u, 0u}};
+    const float llr0 = k0 < N ? gLLR[k0] : 0.0f;
+    __syncthreads();
+
+    int status = 0, iters = 0;
+    int sameCount = 0, bcaseSlot = 0;
+    for (int t = 0;; t++) {
+      // ---- check pass over all rows
+      int fail = 0;
+      for (int r = tid; r < m; r += T) {
+        const uint32_t syn = (synBits[r >> 5] >> (r & 31)) & 1u;
+        rowTot[r] = check_row(phi, rowPtr[r], rowPtr[r + 1], syn);
+        if (t > 0 && (syn ^ ((parBits[r >> 5] >> (r & 31)) & 1u))) fail = 1;
+      }
+      if (mode1 && t > 0) sameCount = s_changed ? 0 : sameCount + 1;
+      const bool cancel = s_cancel != 0;
+      const int anyFail = __syncthreads_or(fail);
+      if (mode1 && !exact && t == 4 && sameCount == 3 && rank == 0) {
+        if (tid == 0) s_item = atomicAdd(a.slot_count, 1);
+        __syncthreads();
+        const int bs = s_item;
+        if (bs < a.slot_capacity) {
+          uint8_t *dst = a.slots + (size_t)bs * N;
+          for (int k = tid; k < N; k += T) dst[k] = (uint8_t)((decBits[k >> 5] >> (k & 31)) & 1u);
+        }
+        bcaseSlot = bs + 1;
+        __syncthreads();
+      }
+      if (mode1 && sameCount == 4) { status = 0; iters = t; break; }
+      if (t > 0 && !anyFail) { status = 1; iters = t; break; }
+      if (cancel) { status = 3; iters = t; break; }
+      if (t == a.max_iter) { status = 0; iters = t; break; }
+      if (tid == 0) s_changed = 0;
+      for (int wd = tid; wd < 2 * NWS; wd += T) parBits[wd] = 0u;
+
+      // ---- variable pass over this member's columns
+      uint32_t *xb = xbuf + (xc & 1u) * BUF;
+      uint64_t *xdec = (uint64_t *)(xb + 3 * N), *xpar = xdec + NWS;
+      uint32_t stop = 0;
+      if (tid == 0 && rank == 0 && t % a.poll == 0)
+        stop = __hip_atomic_load(&st->best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < level;
+      for (int i = wave; rank + size * i < NWS; i += W) {
+        const int ws = rank + size * i, k = ws * 64 + lane;
+        uint32_t dec = 0;
+        if (k < N) {
+          const ColEdges rows = i == wave ? rows0 : gcol[k];
+          const float llr = i == wave ? llr0 : gLLR[k];
+          float c2v[3], f[3];
+          int row[3];
+          uint32_t pos[3];
+          col_edges(rows, row, pos);
+          const float tmp = column_total<MODE1>(row, pos, llr, rowTot, phi, phi_of, c2v);
+          dec = mode1 ? tmp < 0.0f : f2u(tmp) >> 31;
+          if (dec) column_parity(rows, row, parMine);
+          column_messages(tmp, c2v, phi_of, f);
+#pragma unroll
+          for (int q = 0; q < 3; q++) st32(xb + q * N + k, f2u(f[q]));
+        }
+        const uint64_t bal = __ballot(dec);
+        if (lane == 0) st64(xdec + ws, bal);
+      }
+      // the columns whose messages this thread brings into row order, two at a
+      // time, and the counter once this workgroup's stores have completed
+      constexpr int PAIRS = (N / 2 + T - 1) / T;
+      __syncthreads();  // parMine is complete
+      if (tid < NWS) st64(xpar + rank * NWS + tid, (uint64_t)parMine[2 * tid + 1] << 32 | parMine[2 * tid]);
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (tid == 0) st32(ctl + FLAG + FLAG_STEP * (kSplitMax * (xc & 1u) + rank), (xc + 1) << 1 | stop);
+      uint2 edge[PAIRS][3];
+#pragma unroll
+      for (int i = 0; i < PAIRS; i++)
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+          if (tid + i * T < N / 2) edge[i][q] = ((const uint2 *)gcol)[3 * (tid + i * T) + q];
+      if (wave == 0) {
+        uint32_t v = 0;
+        for (int n = 0;; n++) {
+          if (lane < size) v = ld32(ctl + FLAG + FLAG_STEP * (kSplitMax * (xc & 1u) + lane));
+          if (!__ballot(lane < size && v >> 1 != ((xc + 1) & 0x7fffffffu))) break;
+          if (n == kSpin) {
+            s_abort = 1;
+            break;
+          }
+        }
+        const uint64_t cancelled = __ballot(v & 1u);
+        if (lane == 0) s_cancel = cancelled != 0;
+      }
+      __syncthreads();
+      if (s_abort) return;
+      // ---- everybody's messages and decisions
+      {
+        const uint64_t *xm = (const uint64_t *)xb;
+        uint64_t f[PAIRS][3], dv = 0, pv = 0;
+#pragma unroll
+        for (int i = 0; i < PAIRS; i++)
+#pragma unroll
+          for (int q = 0; q < 3; q++)
+            if (tid + i * T < N / 2) f[i][q] = ld64(xm + q * (N / 2) + tid + i * T);
+        if (tid < NWS) dv = ld64(xdec + tid);
+        static_assert(kSplitMax * NWS <= T, "a thread per word of the members' parities");
+        if (tid < size * NWS) pv = ld64(xpar + tid);
+        bool changed = mode1 && t == 0 && !exact;
+#pragma unroll
+        for (int i = 0; i < PAIRS; i++) {
+          if (tid + i * T >= N / 2) break;
+          const ColEdges two[2] = {{{edge[i][0].x, edge[i][0].y, edge[i][1].x}},
+                                   {{edge[i][1].y, edge[i][2].x, edge[i][2].y}}};
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            int row[3];
+            uint32_t pos[3];
+            col_edges(two[h], row, pos);
+#pragma unroll
+            for (int q = 0; q < 3; q++) at_byte(phi, pos[q]) = u2f((uint32_t)(f[i][q] >> (32 * h)));
+          }
+        }
+        if (tid < NWS) {
+          const uint32_t lo = (uint32_t)dv, hi = (uint32_t)(dv >> 32);
+          if (mode1 && t > 0) changed |= decBits[2 * tid] != lo || decBits[2 * tid + 1] != hi;
+          if (mode1 && t == 0 && exact)
+            for (int k = 64 * tid; k < min(N, 64 * tid + 64); k++)
+              changed |= as_global(pd.carry)[k] != (uint8_t)(dv >> (k & 63) & 1u);
+          decBits[2 * tid] = lo;
+          decBits[2 * tid + 1] = hi;
+        }
+        if (tid < size * NWS) {
+          const int wd = 2 * (tid % NWS);
+          if ((uint32_t)pv) atomicXor(&parBits[wd], (uint32_t)pv);
+          if ((uint32_t)(pv >> 32)) atomicXor(&parBits[wd + 1], (uint32_t)(pv >> 32));
+        }
+        if (tid < NWS) parMine[2 * tid] = parMine[2 * tid + 1] = 0u;
+        if (changed) s_changed = 1;
+      }
+      xc++;
+      __syncthreads();
+    }
+    if (rank != 0) {
+      __syncthreads();  // s_item is no longer read
+      continue;
+    }
+
+    // ---- the leader's report, as in bp_persistent_kernel
+    int ok = 0;
+    if (status == 1) {
+      uint32_t crc = 0;
+      for (int k = tid; k < N; k += T)
+        if ((decBits[k >> 5] >> (k & 31)) & 1u) crc ^= L.crcBasis[k];
+      for (int o = 32; o > 0; o >>= 1) crc ^= __shfl_xor(crc, o);
+      if (lane == 0) s_crc[wave] = crc;
+      __syncthreads();
+      uint32_t tot = 0;
+      for (int i = 0; i < W; i++) tot ^= s_crc[i];
+      ok = tot == pd.crc;
+    }
+    // decisions are kept for an accepted code, in ParallelMode 1 for every
+    // code that ran to its end
+    int slot = -1;
+    if (ok || (mode1 && status != 3)) {
+      if (tid == 0) s_item = atomicAdd(a.slot_count, 1);
+      __syncthreads();
+      slot = s_item;
+      if (slot < a.slot_capacity) {
+        uint8_t *dst = a.slots + (size_t)slot * N;
+        for (int k = tid; k < N; k += T) dst[k] = (uint8_t)((decBits[k >> 5] >> (k & 31)) & 1u);
+      }
+    }
+    if (tid == 0) {
+      pd.rec[level] = make_int4(iters, ok ? REC_ACCEPTED : status == 1 ? REC_CRC_MISMATCH
+                                          : status == 3 ? REC_CANCELLED : REC_FAILED, slot, 0);
+      if (ok) atomicMin(&st->best, level);
+      if (mode1) pd.bcase[level] = bcaseSlot;
+    }
     __syncthreads();
   }
 }
@@ -688,6 +1056,17 @@ hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStrea
   if (threads == 1024) return launch_bp<1584, 1024>(a, grid, s);
   if (threads == 512) return launch_bp<1584, 512>(a, grid, s);
   return launch_bp<1584, 256>(a, grid, s);
+}
+
+hipError_t launch_bp_split(int N, const BpArgs &a, int clusters, hipStream_t s) {
+  if (N != 6336 || !a.lad.regular || a.max_iter < 1 || a.split < 2 || a.split > kSplitMax || clusters < 1 || clusters > kSplitClusters || !a.area)
+    return hipErrorInvalidValue;
+  const hipError_t e = launch_zero_ints((int *)a.area, kSplitCtlWords, s);
+  if (e != hipSuccess) return e;
+  const dim3 grid(clusters * a.split);
+  if (a.mode == 1) hipLaunchKernelGGL((bp_split_kernel<6336, 1024, true>), grid, dim3(1024), 0, s, a);
+  else hipLaunchKernelGGL((bp_split_kernel<6336, 1024, false>), grid, dim3(1024), 0, s, a);
+  return hipGetLastError();
 }
 
 hipError_t launch_ce_llr(const PlaneDesc *d_planes, int n, int fixed_start, const Ladder &l1584,

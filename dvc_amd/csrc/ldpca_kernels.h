@@ -78,7 +78,23 @@ struct BpArgs {
   int poll;           // iterations between polls of the bitplane's best code (>= 1)
   int mode;           // 0: beliefPropagation, 1: beliefPropagation_OpenMP (ParallelMode 1)
   int rate_step;      // 1: only the codes the DYNAMICSTEP search tries (dynstep_tries)
+  // a launch that splits its codewords over up to `split` workgroups (0, 1: none):
+  // the area of split_area_words(N) words that they meet in, its first
+  // kSplitCtlWords cleared before the launch
+  int split = 0;
+  uint32_t *area = nullptr;
 };
+
+// Split BP (bp_split_kernel): at most kSplitMax workgroups per codeword and
+// kSplitClusters codewords at a time; per cluster a control block of kCtlWords
+// words, cleared before a launch (block 0 hands out the tickets), then two
+// exchange buffers.
+constexpr int kSplitMax = 8, kSplitClusters = 64, kCtlWords = 256;
+constexpr int kSplitCtlWords = kCtlWords * (kSplitClusters + 1);
+constexpr size_t split_buf_words(int N) {  // messages, decisions, every member's parities
+  return (size_t)3 * N + (kSplitMax + 1) * 2 * ((N + 63) / 64);
+}
+constexpr size_t split_area_words(int N) { return kSplitCtlWords + (size_t)kSplitClusters * 2 * split_buf_words(N); }
 
 // DYNAMICSTEP rate search (LdpcaDecoder.cpp:19-21, 669-672, 760-768): after
 // the r-th failed request (r = 0, 1, ...) the search moves 1 + {0,1,2,3}[min(r,3)]
@@ -107,6 +123,9 @@ enum { REC_FAILED = 0, REC_CRC_MISMATCH = 1, REC_ACCEPTED = 2, REC_CANCELLED = 3
 
 LadderDev ladder_dev(const Ladder &L);
 hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStream_t s);
+// The split form of a launch on a regular ladder: clears the area's control
+// blocks, then `clusters` groups of a.split workgroups.
+hipError_t launch_bp_split(int N, const BpArgs &a, int clusters, hipStream_t s);
 hipError_t launch_zero_ints(int *p, int n, hipStream_t s);
 hipError_t launch_mode1_resolve(const PlaneDesc *planes, int n, int numCodes, int N, const uint8_t *slots,
                                 int slot_capacity, int *rerun_count, hipStream_t s);
