@@ -180,7 +180,7 @@ int dvc_ctx_create(const dvc_params *params, dvc_ctx **out) {
     return rc;
   }
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking);
+  if (e == hipSuccess) e = create_stream_beside(c->stream, &c->stream2);
   if (e != hipSuccess) { dvc_ctx_destroy(c); set_error("hipStreamCreate failed"); return DVC_EDEVICE; }
   if ((rc = noalloc_attach(c))) {
     dvc_ctx_destroy(c);

@@ -1040,7 +1040,6 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
     l.oSegs = align_up(l.oPlanes + sizeof(PlaneDesc) * M);
     l.stageBytes = align_up(l.oSegs + sizeof(CopySeg) * 4 * M);
     err = hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking);
-    if (err == hipSuccess) err = hipStreamCreateWithFlags(&l.s2, hipStreamNonBlocking);
     for (hipEvent_t *ev : {&l.fork, &l.join})
       if (err == hipSuccess) err = hipEventCreateWithFlags(ev, hipEventDisableTiming);
     if (err == hipSuccess) err = hipHostMalloc((void **)&l.h_stage, l.stageBytes * kStageRing, hipHostMallocDefault);
@@ -1058,6 +1057,10 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_counters, 6 * sizeof(int));
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_area, sizeof(uint32_t) * split_area_words(6336));
   }
+  // after the lanes' own streams, so that these lie on as many hardware queues as
+  // there are
+  for (Lane &l : e->lanes)
+    if (err == hipSuccess) err = create_stream_beside(l.s, &l.s2);
   if (err != hipSuccess) {
     set_error(std::string("dvc_engine_create: ") + hipGetErrorString(err));
     engine_destroy(e);

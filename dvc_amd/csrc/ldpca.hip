@@ -1026,7 +1026,47 @@ __global__ void zero_ints_kernel(int *p, int n) {
   if (i < n) p[i] = 0;
 }
 
+// Waits for flag[0] for at most 200 us and says in flag[1] whether it came.
+__global__ void await_flag_kernel(int *flag) {
+  const uint64_t t0 = wall_clock64();  // 100 MHz
+  int seen = 0;
+  while (!seen && wall_clock64() - t0 < 20000) seen = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  flag[1] = seen;
+}
+__global__ void raise_flag_kernel(int *flag) {
+  __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ------------------------------------------------------------------ host side
+// The runtime spreads streams over a few hardware queues, and kernels of two
+// streams on the same queue run one after the other: 60 mixed bitplanes, whose two
+// launches share the CUs, took 2.5 ms on such a pair and 1.55 on others.  So a
+// stream that is to run beside s is tried with a kernel that waits on s for one on
+// the new stream (it gives up after 200 us), and replaced, four times at most.
+hipError_t create_stream_beside(hipStream_t s, hipStream_t *out) {
+  hipStream_t tried[4] = {};
+  int *flag = nullptr, got[2] = {0, 0}, n = 0;
+  *out = nullptr;
+  hipError_t e = hipMalloc((void **)&flag, 2 * sizeof(int));
+  while (e == hipSuccess && n < 4 && !got[1]) {
+    e = hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking);
+    if (e != hipSuccess) break;
+    n++;
+    if ((e = launch_zero_ints(flag, 2, s)) == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) break;
+    hipLaunchKernelGGL(await_flag_kernel, dim3(1), dim3(1), 0, s, flag);
+    hipLaunchKernelGGL(raise_flag_kernel, dim3(1), dim3(1), 0, tried[n - 1], flag);
+    if ((e = hipGetLastError()) == hipSuccess) e = hipStreamSynchronize(tried[n - 1]);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = hipMemcpy(got, flag, sizeof(got), hipMemcpyDeviceToHost);
+  }
+  for (int k = 0; k < n; k++)
+    if (e == hipSuccess && k == n - 1) *out = tried[k];
+    else (void)hipStreamDestroy(tried[k]);
+  if (flag) (void)hipFree(flag);
+  return e;
+}
+
 hipError_t launch_mode1_resolve(const PlaneDesc *planes, int n, int numCodes, int N, const uint8_t *slots,
                                 int slot_capacity, int *rerun_count, hipStream_t s) {
   hipLaunchKernelGGL(mode1_resolve_kernel, dim3(n), dim3(64), 0, s, planes, n, numCodes, N, slots, slot_capacity,
