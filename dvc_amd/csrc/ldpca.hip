@@ -601,10 +601,13 @@ __global__ __launch_bounds__(T) void bp_split_kernel(BpArgs a) {
     }
   }
   __syncthreads();
-  const int rank = s_rank;
+  // out of LDS into scalar registers, and the addresses formed from them too (15
+  // vector registers spilled without it, 8 with: 7.69 -> 7.54 us per iteration of a
+  // plain search, launches included)
+  const int rank = __builtin_amdgcn_readfirstlane(s_rank), cluster = __builtin_amdgcn_readfirstlane(s_cluster);
   if (rank < 0) return;
-  uint32_t *ctl = a.area + (size_t)kCtlWords * (1 + s_cluster);
-  uint32_t *xbuf = a.area + kSplitCtlWords + (size_t)s_cluster * 2 * BUF;
+  uint32_t *ctl = a.area + (size_t)kCtlWords * (1 + cluster);
+  uint32_t *xbuf = a.area + kSplitCtlWords + (size_t)cluster * 2 * BUF;
   uint32_t xc = 0;  // exchanges so far, over all items
 
   for (uint32_t seq = 1;; seq++) {
@@ -646,7 +649,7 @@ __global__ __launch_bounds__(T) void bp_split_kernel(BpArgs a) {
       s_size = (int)(low >> 28);
     }
     __syncthreads();
-    const int w = s_item, size = s_size;
+    const int w = __builtin_amdgcn_readfirstlane(s_item), size = __builtin_amdgcn_readfirstlane(s_size);
     if (w < 0) return;
     const int b = w % a.nplanes;
     const PlaneDesc pd = a.planes[b];
@@ -758,6 +761,7 @@ __global__ __launch_bounds__(T) void bp_split_kernel(BpArgs a) {
       // the columns whose messages this thread brings into row order, two at a
       // time, and the counter once this workgroup's stores have completed
       constexpr int PAIRS = (N / 2 + T - 1) / T;
+      const auto has = [&](int i) { return (i + 1) * T <= N / 2 || tid + i * T < N / 2; };
       __syncthreads();  // parMine is complete
       if (tid < NWS) st64(xpar + rank * NWS + tid, (uint64_t)parMine[2 * tid + 1] << 32 | parMine[2 * tid]);
       __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -768,7 +772,7 @@ __global__ __launch_bounds__(T) void bp_split_kernel(BpArgs a) {
       for (int i = 0; i < PAIRS; i++)
 #pragma unroll
         for (int q = 0; q < 3; q++)
-          if (tid + i * T < N / 2) edge[i][q] = ((const uint2 *)gcol)[3 * (tid + i * T) + q];
+          if (has(i)) edge[i][q] = ((const uint2 *)gcol)[3 * (tid + i * T) + q];
       if (wave == 0) {
         uint32_t v = 0;
         for (int n = 0;; n++) {
@@ -792,14 +796,14 @@ __global__ __launch_bounds__(T) void bp_split_kernel(BpArgs a) {
         for (int i = 0; i < PAIRS; i++)
 #pragma unroll
           for (int q = 0; q < 3; q++)
-            if (tid + i * T < N / 2) f[i][q] = ld64(xm + q * (N / 2) + tid + i * T);
+            if (has(i)) f[i][q] = ld64(xm + q * (N / 2) + tid + i * T);
         if (tid < NWS) dv = ld64(xdec + tid);
         static_assert(kSplitMax * NWS <= T, "a thread per word of the members' parities");
         if (tid < size * NWS) pv = ld64(xpar + tid);
         bool changed = mode1 && t == 0 && !exact;
 #pragma unroll
         for (int i = 0; i < PAIRS; i++) {
-          if (tid + i * T >= N / 2) break;
+          if (!has(i)) break;
           const ColEdges two[2] = {{{edge[i][0].x, edge[i][0].y, edge[i][1].x}},
                                    {{edge[i][1].y, edge[i][2].x, edge[i][2].y}}};
 #pragma unroll
