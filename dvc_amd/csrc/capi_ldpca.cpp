@@ -358,7 +358,8 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     for (int l = 0; l < C; l++) hRec[(size_t)i * C + l] = make_int4(0, REC_NOT_RUN, -1, 0);
   }
   DVC_HIP(hipMemcpyAsync(dev, host, o.inEnd, hipMemcpyHostToDevice, s));
-  TIMED(c, "ce_llr", s, launch_ce_llr(dPlanes, n, 1, c->lad1584, c->lad6336, dCounters, s));
+  uint32_t *area = N == 6336 ? (uint32_t *)(dev + o.area) : nullptr;
+  TIMED(c, "ce_llr", s, launch_ce_llr(dPlanes, n, 1, c->lad1584, c->lad6336, dCounters, area, s));
   std::vector<PlaneState> state(n);
   if (perCode) {
     DVC_HIP(hipMemcpyAsync(state.data(), dState, sizeof(PlaneState) * n, hipMemcpyDeviceToHost, s));
@@ -379,7 +380,7 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
         DVC_HIP(hipMemcpyAsync(dCounters, zero, sizeof(zero), hipMemcpyHostToDevice, s));
         BpArgs a{ld, dPlanes + i, 1, dCounters, 1, 1, c->max_iter, dSlots, dCounters + 1, slots.bp, c->bp_poll,
                  c->bp_mode, c->rate_step};
-        a.area = (uint32_t *)(dev + o.area);
+        a.area = area;
         TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp(c, N, 1, 0, 1, true, a, s));
         DVC_HIP(hipMemcpyAsync(&r, dRec + (size_t)i * C + level, sizeof(r), hipMemcpyDeviceToHost, s));
         DVC_HIP(hipStreamSynchronize(s));
@@ -404,8 +405,10 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
     const int maxOff = C - 1;
     BpArgs a{ld, dPlanes, n, dCounters, n * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, slots.bp,
              c->bp_poll, c->bp_mode, c->rate_step};
-    a.area = (uint32_t *)(dev + o.area);
+    a.area = area;
+    a.area_clear = 1;
     TIMED(c, N == 6336 ? "bp_6336" : "bp_1584", s, launch_bp(c, N, n, other, 1, sequential, a, s));
+    a.area_clear = 0;
     for (int round = 0; mode1; round++) {
       // ParallelMode 1: resolve with the carried decisions; resume the
       // bitplanes that reach a code this launch did not finish

@@ -246,7 +246,7 @@ int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, in
   LadderDev ld = ladder_dev(*L);
   const int maxOff = C - 1;
   const char *name = N == 6336 ? "bp_6336" : "bp_1584";
-  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
+  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, d_area, s));
   BpArgs a{ld, d_planes, n, d_counters, n * maxOff, maxOff, c->max_iter, d_slots, d_counters + 1, slots.bp, c->bp_poll,
            c->bp_mode, c->rate_step};
   a.area = d_area;
@@ -256,10 +256,13 @@ int dvc::bp_step_launch(dvc_ctx *c, int N, int n, bool sequential, int other, in
     for (int i = 0; i < n; i++) {
       if (i) DVC_HIP(launch_zero_ints(d_counters, 1, s));  // queue head only: the step's slots accumulate
       a.planes = d_planes + i;
+      a.area_clear = i == 0;
       TIMED_LAUNCH(c, name, s, launch_bp(c, N, 1, 0, lanes, true, a, s));
     }
   } else {
+    a.area_clear = 1;
     TIMED_LAUNCH(c, name, s, launch_bp(c, N, n, other, lanes, false, a, s));
+    a.area_clear = 0;
     for (int round = 0; c->bp_mode == 1; round++) {
       // ParallelMode 1: resolve with the carried decisions and resume the
       // bitplanes that reach a code the launch did not finish (host-synchronous)
@@ -285,7 +288,7 @@ int dvc::bp_step_codes(dvc_ctx *c, int N, const std::vector<PlaneDesc> &planes, 
   Ladder *L = c->ladder(N);
   const int n = (int)planes.size(), C = L->numCodes;
   LadderDev ld = ladder_dev(*L);
-  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, s));
+  TIMED_LAUNCH(c, "ce_llr", s, launch_ce_llr(d_planes, n, 1, c->lad1584, c->lad6336, d_counters, d_area, s));
   // Every host-side source below stays alive until the stream is drained.
   std::vector<PlaneState> st(n);
   for (int i = 0; i < n; i++)

@@ -83,48 +83,183 @@ __device__ __forceinline__ uint32_t acc_bit(gbyte_t *acc, int i) {
 // ------------------------------------------------------------------ CE + LLR
 // ComputeCE (LdpcaDecoder.cpp:127-143) and the LR -> LLR conversion (:663-667)
 // for one bitplane per workgroup.  The entropy is the reference's sequential
-// float sum over the columns, a chain of N dependent additions, and that chain
-// is what bounds the kernel: one wave does nothing but add (64 terms to one LDS
-// latency), the other 15 compute the terms one chunk ahead of it.  The start
-// code is found by comparing all code rates at once.  With every lane of a
-// 256-thread workgroup waiting for one lane's loop over the terms, and then for
-// its loop over the rates, a CIF bitplane took 71 us and a QCIF one 22; now 24
-// and 8.7 (sums of 16 terms with the next 16 read meanwhile: 34 and 12).
+// float sum over the columns, N dependent additions, 16 us of a CIF bitplane when
+// one lane makes them (the whole kernel then takes 24 us, the terms computed
+// meanwhile).  sum_terms gets the same bits from a scan: while the sum s stays
+// within one binade, adding a term t >= 0 moves s by a whole number of its ulps u,
+// floor(t/u) or one more, which hangs on s only by its lowest bit, for a t that
+// ends in exactly half an ulp (ties go to even).  So a run of terms is a pair of
+// whole numbers, the ulps it adds to an even and to an odd s, and two runs compose.
+//   * Every thread takes CH consecutive terms.  Approximate sums before and after
+//     them, with a bound on how far the sequential sum can be from those, say
+//     whether s stays within one binade meanwhile.
+//   * Threads of one wave and binade compose their runs by a segmented scan; those
+//     near a power of two keep their terms.
+//   * The pieces, 35 or so, are applied in order: a run by an addition to s's bits,
+//     the rest term by term.
+// More than 64 pieces (sums that dwell at a power of two) and terms that are
+// negative, not numbers or above 2 (no likelihood ratio of a decoder gives such)
+// go lane by lane as before.
+// A CIF bitplane takes 15.7 us so, 26 with the additions by one lane (the terms are
+// 9 of them: 99 waves' worth of three logf on one CU).  A QCIF one's 1584 additions
+// take no longer than the scan (10.3 and 10.4 us): it keeps them.
 #define DVC_LOG2 (0.693147181f)
-constexpr int CE_T = 1024, CE_CHUNK = CE_T - 64;  // a multiple of 64
-// It also clears the step's launch counters (a kernel's store, so that a captured
-// step holds no memset).
+constexpr int CE_T = 1024, CE_W = CE_T / 64, CE_SCAN = 4096;
+
+struct CeShared {
+  __align__(16) float tot[CE_W];  // sums of the waves' terms
+  int pieces[CE_W];
+  int4 piece[64];  // thread of the terms or -1, ulps for an even and an odd sum
+};
+
+// The six steps of a scan over a wave: the value of the lane 1, 2, 4, 8 back in
+// the row of 16, then of the last lane of the row or of the two rows before.  Where
+// a step brings nothing it gives 0.
+template <int STEP>
+__device__ __forceinline__ int scan_from(int v) {
+  if constexpr (STEP < 4) return __builtin_amdgcn_update_dpp(0, v, 0x110 | 1 << STEP, 0xf, 0xf, false);
+  if constexpr (STEP == 4) return __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  return __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+}
+template <int STEP>
+__device__ __forceinline__ void scan_sum(float &v) {
+  v += u2f((uint32_t)scan_from<STEP>((int)f2u(v)));
+}
+// Two runs composed, unless a segment begins in between.
+template <int STEP>
+__device__ __forceinline__ void scan_runs(int &inc0, int &inc1, int &head) {
+  const int a0 = scan_from<STEP>(inc0), a1 = scan_from<STEP>(inc1), h = scan_from<STEP>(head);
+  const int n0 = a0 + (a0 & 1 ? inc1 : inc0), n1 = a1 + (a1 & 1 ? inc0 : inc1);
+  inc0 = head ? inc0 : n0;
+  inc1 = head ? inc1 : n1;
+  head |= h;
+}
+
+// True: wave 0 has the sum.  Every thread of the workgroup calls it.
+template <int CH>
+__device__ bool sum_terms(const float *terms, int N, CeShared &sh, float *sum) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, first = tid * CH;
+  float t[CH], local = 0.0f;
+#pragma unroll
+  for (int i = 0; i < CH; i++) {
+    t[i] = first + i < N ? terms[first + i] : 0.0f;
+    local += t[i];
+  }
+  float upto = local;
+  scan_sum<0>(upto), scan_sum<1>(upto), scan_sum<2>(upto);
+  scan_sum<3>(upto), scan_sum<4>(upto), scan_sum<5>(upto);
+  float before = __shfl_up(upto, 1);
+  if (lane == 0) before = 0.0f;
+  if (lane == 63) sh.tot[wave] = upto;
+  __syncthreads();
+  float waves = 0.0f;
+#pragma unroll
+  for (int w = 0; w < CE_W; w++) waves += w < wave ? sh.tot[w] : 0.0f;
+  before += waves;
+  upto += waves;
+  // k float additions of terms >= 0 end within k ulps' halves (2^-24 each) of the
+  // exact sum, relative to it; the sums here within 30 of them
+  const float tol = (float)(first + CH + 64) * 6.3e-8f;
+  const uint32_t e = f2u(before * (1.0f - tol)) >> 23;
+  const bool valid = first < N, clear = e > 64u && e == f2u(upto * (1.0f + tol)) >> 23;
+  int inc0 = 0, inc1 = 1;  // inc1 starts at an odd sum
+  if (clear) {
+    const float scale = u2f((277u - e) << 23);  // 1/u = 2^(150 - e)
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+      const float q = t[i] * scale, fl = floorf(q), fr = q - fl;  // all exact, q < 2^24
+      const int k = (int)fl, half = fr == 0.5f, up = fr > 0.5f;
+      inc0 += k;
+      inc1 += k;
+      inc0 += up | (half & inc0);
+      inc1 += up | (half & inc1);
+    }
+  }
+  inc1 -= 1;
+  const int key = clear ? (int)e : -1, key1 = __shfl_up(key, 1);
+  int head = lane == 0 || !valid || key < 0 || key != key1;
+  const uint64_t heads = __ballot(head);
+  scan_runs<0>(inc0, inc1, head), scan_runs<1>(inc0, inc1, head), scan_runs<2>(inc0, inc1, head);
+  scan_runs<3>(inc0, inc1, head), scan_runs<4>(inc0, inc1, head), scan_runs<5>(inc0, inc1, head);
+  const bool tail = valid && (lane == 63 || (heads >> (lane + 1) & 1u));
+  const uint64_t tails = __ballot(tail);
+  if (lane == 0) sh.pieces[wave] = __popcll(tails);
+  __syncthreads();
+  int at = __popcll(tails & ((1ull << lane) - 1)), all = 0;
+#pragma unroll
+  for (int w = 0; w < CE_W; w++) {
+    const int n = sh.pieces[w];
+    at += w < wave ? n : 0;
+    all += n;
+  }
+  if (all > 64) return false;
+  if (tail) sh.piece[at] = make_int4(clear ? -1 : tid, inc0, inc1, 0);
+  __syncthreads();
+  if (wave != 0) return true;
+  const int4 p = lane < all ? sh.piece[lane] : make_int4(-1, 0, 0, 0);
+  float own[CH];
+#pragma unroll
+  for (int i = 0; i < CH; i++) own[i] = p.x >= 0 && p.x * CH + i < N ? terms[p.x * CH + i] : 0.0f;
+  float s = 0.0f;
+  for (int j = 0; j < all; j++) {
+    if (__builtin_amdgcn_readlane(p.x, j) < 0) {
+      const int i0 = __builtin_amdgcn_readlane(p.y, j), i1 = __builtin_amdgcn_readlane(p.z, j);
+      s = u2f(f2u(s) + (uint32_t)(f2u(s) & 1u ? i1 : i0));
+    } else {
+#pragma unroll
+      for (int i = 0; i < CH; i++) s += u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(own[i]), j));
+    }
+  }
+  *sum = s;
+  return true;
+}
+
+// It also clears the step's launch counters and, with the workgroups beyond the
+// bitplanes', the control blocks of a split BP launch (a kernel's stores, so that a
+// captured step holds no memset; a launch of their own took 5 us).
 __global__ __launch_bounds__(CE_T) void ce_llr_kernel(const PlaneDesc *planes, int nplanes, int fixed_start,
                                                       const float *codeRate1584, const float *codeRate6336,
-                                                      int numCodes1584, int numCodes6336, int *counters) {
+                                                      int numCodes1584, int numCodes6336, int *counters,
+                                                      uint4 *clear, int clearQuads) {
   __shared__ __align__(16) float terms[6336 + 64];  // spare: the last group of 64
-  const int p = blockIdx.x;
-  if (p >= nplanes) return;
+  __shared__ CeShared sh;
+  const int p = blockIdx.x, tid = threadIdx.x;
+  if (p >= nplanes) {
+    const int i = (p - nplanes) * CE_T + tid;
+    if (i < clearQuads) clear[i] = make_uint4(0u, 0u, 0u, 0u);
+    return;
+  }
   const PlaneDesc d = planes[p];
-  const int N = d.N, tid = threadIdx.x;
+  const int N = d.N;
   if (p == 0 && tid < 3) counters[tid] = 0;
-  int nan = 0;
-  float rlb = 0.0f;
+  int flags = 0;  // 1: a NaN LLR, 2: a term that sum_terms does not take
   if (tid < 64) terms[N + tid] = 0.0f;
-  for (int c0 = -CE_CHUNK; c0 < N; c0 += CE_CHUNK) {
-    // chunk c0 is summed by wave 0 while the others compute chunk c0 + CE_CHUNK
-    const int k = c0 + tid + CE_CHUNK - 64;
-    if (tid >= 64) {
-      if (k < N) {
-        const float lr = as_global(d.LR)[k];
-        const float Pco = lr / (1.0f + lr);
-        const float tmp = dvc_logf(1 - Pco);
-        terms[k] = (Pco * (-dvc_logf(Pco) + tmp) - tmp) / DVC_LOG2;
-        const float llr = dvc_logf(lr);
-        d.LLR[k] = llr;
-        nan |= llr != llr;
-      }
-    } else if (c0 >= 0) {
-      // past the last column the terms are +0, which leaves the sum as it is
-      const float4 *q = (const float4 *)(terms + c0);
-      const int groups = ((N - c0 < CE_CHUNK ? N - c0 : CE_CHUNK) + 63) >> 6;
+  constexpr int PER = (6336 + CE_T - 1) / CE_T;
+  float lrs[PER];
+#pragma unroll
+  for (int j = 0; j < PER; j++)
+    if (tid + j * CE_T < N) lrs[j] = as_global(d.LR)[tid + j * CE_T];
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const int k = tid + j * CE_T;
+    if (k >= N) break;
+    const float lr = lrs[j];
+    const float Pco = lr / (1.0f + lr);
+    const float tmp = dvc_logf(1 - Pco);
+    const float term = (Pco * (-dvc_logf(Pco) + tmp) - tmp) / DVC_LOG2;
+    terms[k] = term;
+    const float llr = dvc_logf(lr);
+    d.LLR[k] = llr;
+    flags |= (llr != llr ? 1 : 0) | (term >= 0.0f && term <= 2.0f ? 0 : 2);
+  }
+  const int nan = __syncthreads_or(flags & 1), slow = __syncthreads_or((flags & 2) != 0);
+  float rlb = 0.0f;
+  if (N < CE_SCAN || slow || !sum_terms<PER>(terms, N, sh, &rlb)) {
+    // past the last column the terms are +0, which leaves the sum as it is
+    const float4 *q = (const float4 *)terms;
+    if (tid < 64)
 #pragma unroll 1
-      for (int g = 0; g < groups; g++, q += 16) {
+      for (int g = 0; g < (N + 63) >> 6; g++, q += 16) {
         float4 a[16];
 #pragma unroll
         for (int i = 0; i < 16; i++) a[i] = q[i];
@@ -137,10 +272,7 @@ __global__ __launch_bounds__(CE_T) void ce_llr_kernel(const PlaneDesc *planes, i
           rlb += a[i].w;
         }
       }
-    }
-    __syncthreads();
   }
-  nan = __syncthreads_or(nan);
   if (tid >= 64) return;
   rlb /= (float)N;
   // A NaN likelihood ratio makes the entropy NaN; the x86 path's is its
@@ -1109,8 +1241,10 @@ hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStrea
 hipError_t launch_bp_split(int N, const BpArgs &a, int clusters, hipStream_t s) {
   if (N != 6336 || !a.lad.regular || a.max_iter < 1 || a.split < 2 || a.split > kSplitMax || clusters < 1 || clusters > kSplitClusters || !a.area)
     return hipErrorInvalidValue;
-  const hipError_t e = launch_zero_ints((int *)a.area, kSplitCtlWords, s);
-  if (e != hipSuccess) return e;
+  if (!a.area_clear) {
+    const hipError_t e = launch_zero_ints((int *)a.area, kSplitCtlWords, s);
+    if (e != hipSuccess) return e;
+  }
   const dim3 grid(clusters * a.split);
   if (a.mode == 1) hipLaunchKernelGGL((bp_split_kernel<6336, 1024, true>), grid, dim3(1024), 0, s, a);
   else hipLaunchKernelGGL((bp_split_kernel<6336, 1024, false>), grid, dim3(1024), 0, s, a);
@@ -1118,9 +1252,12 @@ hipError_t launch_bp_split(int N, const BpArgs &a, int clusters, hipStream_t s) 
 }
 
 hipError_t launch_ce_llr(const PlaneDesc *d_planes, int n, int fixed_start, const Ladder &l1584,
-                         const Ladder &l6336, int *counters, hipStream_t s) {
-  hipLaunchKernelGGL(ce_llr_kernel, dim3(n), dim3(CE_T), 0, s, d_planes, n, fixed_start, l1584.d_codeRate,
-                     l6336.d_codeRate, l1584.numCodes, l6336.numCodes, counters);
+                         const Ladder &l6336, int *counters, uint32_t *area, hipStream_t s) {
+  static_assert(kSplitCtlWords % 4 == 0, "cleared in quads");
+  const int quads = area ? kSplitCtlWords / 4 : 0;
+  hipLaunchKernelGGL(ce_llr_kernel, dim3(n + (quads + CE_T - 1) / CE_T), dim3(CE_T), 0, s, d_planes, n, fixed_start,
+                     l1584.d_codeRate, l6336.d_codeRate, l1584.numCodes, l6336.numCodes, counters, (uint4 *)area,
+                     quads);
   return hipGetLastError();
 }
 

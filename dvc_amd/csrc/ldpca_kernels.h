@@ -80,9 +80,11 @@ struct BpArgs {
   int rate_step;      // 1: only the codes the DYNAMICSTEP search tries (dynstep_tries)
   // a launch that splits its codewords over up to `split` workgroups (0, 1: none):
   // the area of split_area_words(N) words that they meet in, its first
-  // kSplitCtlWords cleared before the launch
+  // kSplitCtlWords cleared before the launch, by the launch itself unless
+  // area_clear says that launch_ce_llr did it and none has used it since
   int split = 0;
   uint32_t *area = nullptr;
+  int area_clear = 0;
 };
 
 // Split BP (bp_split_kernel): at most kSplitMax workgroups per codeword and
@@ -124,7 +126,7 @@ enum { REC_FAILED = 0, REC_CRC_MISMATCH = 1, REC_ACCEPTED = 2, REC_CANCELLED = 3
 LadderDev ladder_dev(const Ladder &L);
 hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStream_t s);
 // The split form of a launch on a regular ladder: clears the area's control
-// blocks, then `clusters` groups of a.split workgroups.
+// blocks if they are not, then `clusters` groups of a.split workgroups.
 hipError_t launch_bp_split(int N, const BpArgs &a, int clusters, hipStream_t s);
 hipError_t launch_zero_ints(int *p, int n, hipStream_t s);
 // A non-blocking stream whose kernels run beside s's, if the device has one left.
@@ -132,9 +134,11 @@ hipError_t create_stream_beside(hipStream_t s, hipStream_t *out);
 hipError_t launch_mode1_resolve(const PlaneDesc *planes, int n, int numCodes, int N, const uint8_t *slots,
                                 int slot_capacity, int *rerun_count, hipStream_t s);
 // Entropy, LLRs and start codes of n bitplanes; also clears the three launch
-// counters (queue head, decision slots handed out, bitplanes to resume).
+// counters (queue head, decision slots handed out, bitplanes to resume) and, if
+// there is one, the control blocks of the area of a split BP launch (16-byte
+// aligned).
 hipError_t launch_ce_llr(const PlaneDesc *d_planes, int n, int fixed_start, const Ladder &l1584,
-                         const Ladder &l6336, int *counters, hipStream_t s);
+                         const Ladder &l6336, int *counters, uint32_t *area, hipStream_t s);
 // BP on an irregular ladder (bp_irregular_kernel).
 hipError_t launch_bp_irregular(const BpArgs &a, int grid, hipStream_t s);
 // Full-rate inverse of the bitplanes whose BP codes all failed, bitplane p's

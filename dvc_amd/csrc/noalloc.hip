@@ -198,7 +198,7 @@ extern "C" int dvc_ldpca_decode_batch_noalloc(dvc_ctx *c, int n, dvc_ldpca_item 
     hipLaunchKernelGGL(noalloc_setup_kernel, dim3(1), dim3(256), 0, s, dItems, n, N, C, dIndex, dPlanes, dState, dRec,
                        dLLR);
     DVC_HIP(hipGetLastError());
-    DVC_HIP(launch_ce_llr(dPlanes, ng, 1, c->lad1584, c->lad6336, dCounters, s));
+    DVC_HIP(launch_ce_llr(dPlanes, ng, 1, c->lad1584, c->lad6336, dCounters, nullptr, s));
     const LadderDev ld = ladder_dev(*L);
     BpArgs a{ld, dPlanes, ng, dCounters, ng * maxOff, maxOff, c->max_iter, dSlots, dCounters + 1, sp.bp,
              c->bp_poll, c->bp_mode, c->rate_step};
