@@ -61,7 +61,7 @@ __global__ __launch_bounds__(IR_T) void bp_irregular_kernel(BpArgs a) {
   __shared__ uint16_t rowPtr[IR_NMAX + 2];
   __shared__ uint8_t dec[IR_NMAX];
   __shared__ uint32_t synBits[(IR_NMAX + 31) / 32];
-  __shared__ int s_item, s_cancel;
+  __shared__ int s_item, s_fail[2], s_cancel[2];  // by iteration parity, as in bp_persistent_kernel
   __shared__ uint32_t s_crc[T / 64];
   __shared__ int s_changed[2];
 
@@ -137,9 +137,11 @@ __global__ __launch_bounds__(IR_T) void bp_irregular_kernel(BpArgs a) {
     }
     __syncthreads();
     for (int l = tid; l < E; l += T) phi[l] = colTot[gslot[l] >> 13];
+    const uint32_t edge0 = tid < E ? gslot[tid] : 0u;  // this thread's first, the same in every iteration
+    if (tid == 0) s_cancel[0] = s_fail[0] = 0;
     __syncthreads();
 
-    int status = 0, iters = 0;
+    int status = 0, iters = 0, poll = 0;
     int sameCount = 0, bcaseSlot = 0;
     for (int t = 0;; t++) {
       // ---- check pass: |phi| sums and sign products; parity of the previous
@@ -191,12 +193,11 @@ __global__ __launch_bounds__(IR_T) void bp_irregular_kernel(BpArgs a) {
         }
       }
       if (mode1 && t > 0) sameCount = s_changed[(t - 1) & 1] ? 0 : sameCount + 1;
-      if (tid == 0) {
-        s_changed[t & 1] = 0;
-        s_cancel = (t % a.poll == 0) &&
-                   __hip_atomic_load(&st->best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < level;
-      }
-      const int anyFail = __syncthreads_or(fail);
+      if (tid == 0) s_changed[t & 1] = 0;
+      if (fail) s_fail[t & 1] = 1;
+      __syncthreads();
+      const int anyFail = s_fail[t & 1];
+      const bool cancel = s_cancel[t & 1] != 0;
       if (mode1 && !exact && t == 4 && sameCount == 3) {
         // iterations 0-3 decided alike: keep the decisions for the resolution
         if (tid == 0) s_item = atomicAdd(a.slot_count, 1);
@@ -211,11 +212,19 @@ __global__ __launch_bounds__(IR_T) void bp_irregular_kernel(BpArgs a) {
       }
       if (mode1 && sameCount == 4) { status = 0; iters = t; break; }
       if (t > 0 && !anyFail) { status = 1; iters = t; break; }
-      if (s_cancel) { status = 3; iters = t; break; }
+      if (cancel) { status = 3; iters = t; break; }
       if (t == a.max_iter) { status = 0; iters = t; break; }
 
       // ---- variable pass (:512-548).  c2v of every slot
-      uint32_t eNext = tid < E ? gslot[tid] : 0u;
+      // (lane 0 looks whether a lower code has been accepted, for the next check pass)
+      int best = level;
+      const bool ask = poll == 0;
+      poll = ask ? a.poll - 1 : poll - 1;
+      if (tid == 0) {
+        s_fail[(t + 1) & 1] = 0;
+        if (ask) best = __hip_atomic_load(&st->best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      uint32_t eNext = edge0;
       for (int l = tid; l < E; l += T) {
         const uint32_t e = eNext;
         if (l + T < E) eNext = gslot[l + T];
@@ -255,7 +264,7 @@ __global__ __launch_bounds__(IR_T) void bp_irregular_kernel(BpArgs a) {
       if (changed) s_changed[t & 1] = 1;
       __syncthreads();
       // each slot's next v2c
-      eNext = tid < E ? gslot[tid] : 0u;
+      eNext = edge0;
       for (int l = tid; l < E; l += T) {
         const uint32_t e = eNext;
         if (l + T < E) eNext = gslot[l + T];
@@ -268,6 +277,7 @@ __global__ __launch_bounds__(IR_T) void bp_irregular_kernel(BpArgs a) {
         const uint64_t bal = __ballot(mode1 ? tot < 0.0f : ir_f2u(tot) >> 31 != 0u);
         if (lane == 0) slotDec[l >> 6] = bal;
       }
+      if (tid == 0) s_cancel[(t + 1) & 1] = best < level;
       __syncthreads();
     }
 
