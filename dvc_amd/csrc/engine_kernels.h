@@ -41,6 +41,12 @@ struct CopySeg {
   size_t bytes;
 };
 
+// Copies the next block of a ring in pinned host memory (blocks of `bytes`, a
+// multiple of 16) to dst.  Which one is next the device counts itself, in turn (two
+// words, 0 at first), so that a captured launch replays with another block each
+// time: a copy before each replay kept the GPU idle for 12 us and took 4 (24 mixed
+// frames 38.9 -> 38.2 ms, 256 CIF frames 397 -> 394).
+hipError_t launch_take_block(const void *ring, int blocks, size_t bytes, void *dst, unsigned *turn, hipStream_t s);
 hipError_t launch_job_init(const JobInitDev *items, int n, hipStream_t s);
 hipError_t launch_keyframe_batch(const KeyFrameJob *jobs, int n, int maxW, int maxH, hipStream_t s);
 hipError_t launch_copy_segments(const CopySeg *segs, int n, hipStream_t s);

@@ -347,15 +347,16 @@ struct Lane {
   std::vector<Job *> inflight;
   std::vector<Job *> finished;  // retired by the engine after the step
   // A step's descriptors, written to one of kStageRing pinned host blocks in turn
-  // and uploaded to the one device mirror with one copy: frame descriptors, five frame lists of
+  // and copied to the one device mirror by a kernel: frame descriptors, five frame lists of
   // cap entries (stepped, starting a band, ending a band, set up, finishing),
   // BP frame links, plane descriptors, result copy segments (3 per frame).
-  // The copy is ordered behind the previous step's kernels, so only the host
+  // The kernel is ordered behind the previous step's, so only the host
   // block has to wait for it, and the host prepares and queues the next steps
   // while this one runs: nothing in a step depends on its predecessors' results.
   uint8_t *h_stage = nullptr, *d_stage = nullptr;  // h_stage: kStageRing blocks
+  unsigned *d_turn = nullptr;                      // launch_take_block's count
   size_t stageBytes = 0, oLists = 0, oLinks = 0, oPlanes = 0, oSegs = 0;
-  hipEvent_t staged[kStageRing] = {};  // block k's last upload
+  hipEvent_t staged[kStageRing] = {};  // block k has been read
   unsigned steps = 0;
   FrameDev *h_frames = nullptr, *d_frames = nullptr;
   int *h_lists = nullptr, *d_lists = nullptr;
@@ -644,7 +645,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
   // the staging block used kStageRing steps ago, once its upload is done.  (With
   // the stream drained after every step, a CIF frame decoded alone left the GPU
   // idle for 40 us of each of its 63 steps.)
-  const int slot = (int)(ln.steps++ % kStageRing);
+  const int slot = (int)(ln.steps % kStageRing);
   uint8_t *stage = ln.h_stage + slot * ln.stageBytes;
   DVC_HIP(hipEventSynchronize(ln.staged[slot]));
   ln.h_frames = (FrameDev *)stage;
@@ -742,9 +743,22 @@ static int lane_step(dvc_engine *e, Lane &ln) {
     if (job_needs_host_recons(e, j)) ln.h_segs[nseg++] = CopySeg{j.fd.recons, o + align_up(bs) + align_up(br), FS};
     if (e->deviceBuffers) ln.h_segs[nseg++] = CopySeg{j.fd.recons, j.spec.recons, FS};
   }
-  // ---- one upload of the step's descriptors
-  DVC_HIP(hipMemcpyAsync(ln.d_stage, stage, ln.stageBytes, hipMemcpyHostToDevice, s));
-  DVC_HIP(hipEventRecord(ln.staged[slot], s));
+  // (ParallelMode 1 steps read a resolution count back, so they are not captured)
+  const bool steady = e->graphs && !c->profiling && c->bp_mode == 0 && !active.empty() && setup.empty() &&
+                      starting.empty() && ending.empty();
+  // ---- the step's descriptors, brought up by a kernel: a steady step's graph
+  // holds it too.  The block is used up once that kernel is queued.
+  auto bring_up = [&]() {
+    return launch_take_block(ln.h_stage, kStageRing, ln.stageBytes, ln.d_stage, ln.d_turn, s);
+  };
+  auto used_up = [&]() {
+    ln.steps++;
+    return hipEventRecord(ln.staged[slot], s);
+  };
+  if (!steady) {
+    DVC_HIP(bring_up());
+    DVC_HIP(used_up());
+  }
   // ---- setup of newly admitted frames: SI, noise parameters, OCT, SMF
   if (!setup.empty()) {
     const int nf = (int)setup.size();
@@ -796,15 +810,14 @@ static int lane_step(dvc_engine *e, Lane &ln) {
       TIMED_LAUNCH(c, "put_bitplane", s, launch_put_bitplane(ln.d_frames, L0, ln.d_links, na, maxN, s));
       return DVC_OK;
     };
-    // (ParallelMode 1 steps read a resolution count back, so they are not captured)
-    const bool steady = e->graphs && !c->profiling && c->bp_mode == 0 && setup.empty() &&
-                        starting.empty() && ending.empty();
     if (steady) {
       const auto key = std::make_tuple(na, n0, n1, maxN, e->busyLanes);
       auto it = ln.graphs.find(key);
       if (it == ln.graphs.end()) {
         DVC_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        const int lrc = launches();
+        const hipError_t be = bring_up();
+        const int lrc = be == hipSuccess ? launches() : DVC_EDEVICE;
+        if (be != hipSuccess) set_error(std::string("launch_take_block: ") + hipGetErrorString(be));
         hipGraph_t graph = nullptr;
         const hipError_t ce = hipStreamEndCapture(s, &graph);
         if (lrc) {
@@ -819,6 +832,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
         it = ln.graphs.emplace(key, exec).first;
       }
       DVC_HIP(hipGraphLaunch(it->second, s));
+      DVC_HIP(used_up());
     } else if ((rc = launches())) {
       return rc;
     }
@@ -1064,6 +1078,8 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
       if (err == hipSuccess) err = hipEventCreateWithFlags(ev, hipEventDisableTiming);
     if (err == hipSuccess) err = hipHostMalloc((void **)&l.h_stage, l.stageBytes * kStageRing, hipHostMallocDefault);
     if (err == hipSuccess) err = hipMalloc((void **)&l.d_stage, l.stageBytes);
+    if (err == hipSuccess) err = hipMalloc((void **)&l.d_turn, 2 * sizeof(unsigned));
+    if (err == hipSuccess) err = launch_zero_ints((int *)l.d_turn, 2, l.s);
     for (int r = 0; r < kStageRing && err == hipSuccess; r++) err = hipEventCreateWithFlags(&l.staged[r], hipEventDisableTiming);
     if (err == hipSuccess) {
       memset(l.h_stage, 0, l.stageBytes * kStageRing);
@@ -1097,7 +1113,7 @@ static void engine_destroy(dvc_engine *e) {
     for (Job *j : l.inflight) { if (j->mem) (void)hipFree(j->mem); delete j; }
     for (Job *j : l.finished) { if (j->mem) (void)hipFree(j->mem); delete j; }
     for (auto &g : l.graphs) (void)hipGraphExecDestroy(g.second);
-    void *ptrs[] = {l.d_stage, l.d_out, l.d_slots, l.d_counters, l.d_area};
+    void *ptrs[] = {l.d_stage, l.d_turn, l.d_out, l.d_slots, l.d_counters, l.d_area};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
     if (l.h_stage) (void)hipHostFree(l.h_stage);
