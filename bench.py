@@ -305,9 +305,8 @@ def bench_wz(args):
 
 def bench_wz_plain(args, ctx, jobs, dev, outs):
     """The plain drop-in path: one frame at a time (an engine with one frame
-    in flight) with the sequential rate search (one BP launch per code, the
-    host choosing the next code), inputs resident in HBM as in the batched
-    leg, through one long-lived engine.  Also one dvc_decode_wz_frames call
+    in flight) with the sequential rate search (code after code within one
+    BP launch per bitplane), inputs resident in HBM as in the batched leg, through one long-lived engine.  Also one dvc_decode_wz_frames call
     (batched = 0), which sets up and tears down its own engine, timed
     separately as the per-call set-up cost."""
     from dvc_amd import _lib
