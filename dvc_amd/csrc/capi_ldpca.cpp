@@ -438,6 +438,8 @@ static int decode_group(dvc_ctx *c, int N, int n, dvc_ldpca_item *items, int seq
       const int4 r = rec[(size_t)i * C + best];
       DVC_CHECK(r.y == REC_ACCEPTED && r.z >= 0 && r.z < slots.total, DVC_ESTATE,
                 "dvc_ldpca_decode_batch: missing accepted record");
+      DVC_CHECK(unfinished_code(&rec[(size_t)i * C], std::max(state[i].start, 0), best, c->rate_step) < 0, DVC_ESTATE,
+                "dvc_ldpca: a code below the accepted one did not finish");
       memcpy(items[i].decoded, host + o.out + (size_t)i * N, N);
     }
   }

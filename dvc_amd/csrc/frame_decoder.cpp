@@ -598,6 +598,8 @@ static int finish_job(dvc_engine *e, Job &j, const uint8_t *out, int slot_cap) {
     DVC_CHECK(r.y == REC_ACCEPTED, DVC_ESTATE, "WZ frame decode: bitplane without accepted code");
     DVC_CHECK(r.z >= 0 && r.z < slot_cap, DVC_ENOMEM,
               "WZ frame decode: decision slots exhausted (an accepted bitplane's decisions were not stored)");
+    DVC_CHECK(unfinished_code(rec + (size_t)kMaxCodes * b, std::max(ps[b].start, 0), best, c->rate_step) < 0, DVC_ESTATE,
+              "WZ frame decode: a code below the accepted one did not finish");
   }
   if (!e->deviceBuffers) memcpy(j.spec.recons, rec8, FS);
   dvc_frame_stats *st = j.spec.stats;

@@ -700,7 +700,9 @@ __global__ __launch_bounds__(T) void bp_persistent_kernel(BpArgs a) {
 // leader with the members that have arrived within 30 us of it, a later one
 // leaves at once, and every wait is for members or the leader of a closed
 // cluster.  The polls are bounded all the same; a member that runs into the bound
-// leaves, and the host finds the records missing.
+// leaves, and its codes' records stay unfinished.  In ParallelMode 0 the search
+// then ends at a higher code or at the full rate, which the host refuses
+// (unfinished_code); a ParallelMode 1 resolution runs such codes again.
 //
 // With 8 members an iteration takes 7.2 us against 16: row sums 1.7, columns 1.4,
 // stores until complete 1.7, counters 1.0, reading and reordering 1.6.  A CIF

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "rate_search.h"
 
 namespace dvc {
 
@@ -98,18 +99,6 @@ constexpr size_t split_buf_words(int N) {  // messages, decisions, every member'
 }
 constexpr size_t split_area_words(int N) { return kSplitCtlWords + (size_t)kSplitClusters * 2 * split_buf_words(N); }
 
-// DYNAMICSTEP rate search (LdpcaDecoder.cpp:19-21, 669-672, 760-768): after
-// the r-th failed request (r = 0, 1, ...) the search moves 1 + {0,1,2,3}[min(r,3)]
-// codes up, so it tries the codes start + 0, 1, 3, 6, 10, 14, 18, ... below
-// the full rate, then the full rate.
-__host__ __device__ inline bool dynstep_tries(int off) {
-  return off == 0 || off == 1 || off == 3 || off == 6 || (off >= 10 && (off - 10) % 4 == 0);
-}
-// The offset from the start code tried after offset `off` fails.
-__host__ __device__ inline int dynstep_next(int off) {
-  return off < 1 ? 1 : off < 3 ? 3 : off < 6 ? 6 : off < 10 ? 10 : off + 4;
-}
-
 // Decision slots of a launch of n bitplanes over C codes.  The BP kernel hands
 // out the first `bp` of them: ParallelMode 0 accepts each (bitplane, code) at
 // most once, and a bitplane that accepts code C - 1 does so through the inverse;
@@ -119,9 +108,6 @@ struct SlotPlan { int bp, total; };
 inline SlotPlan slot_plan(int n, int C, int mode) {
   return mode == 1 ? SlotPlan{2 * C * n + 1, 2 * C * n + 1 + n} : SlotPlan{(C - 1) * n + 1, C * n + 1};
 }
-
-// record.y status values
-enum { REC_FAILED = 0, REC_CRC_MISMATCH = 1, REC_ACCEPTED = 2, REC_CANCELLED = 3, REC_NOT_RUN = -1 };
 
 LadderDev ladder_dev(const Ladder &L);
 hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStream_t s);
