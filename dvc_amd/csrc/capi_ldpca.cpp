@@ -180,7 +180,6 @@ int dvc_ctx_create(const dvc_params *params, dvc_ctx **out) {
     return rc;
   }
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = create_stream_beside(c->stream, &c->stream2);
   if (e != hipSuccess) { dvc_ctx_destroy(c); set_error("hipStreamCreate failed"); return DVC_EDEVICE; }
   if ((rc = noalloc_attach(c))) {
     dvc_ctx_destroy(c);
@@ -499,6 +498,10 @@ int dvc_ldpca_decode_batch(dvc_ctx *c, int n, dvc_ldpca_item *items) {
   }
   // both code lengths at once, each on its own stream and host thread: one after
   // the other, the second waited for the last codes of the first (see bp_grid)
+  // (the second stream is made when a batch first needs it: a queue taken by one
+  // that never runs is missing to an engine's lanes)
+  bool both = !g[0].empty() && !g[1].empty();
+  if (both && !c->stream2) both = create_stream_beside(&c->stream, 1, &c->stream2, nullptr) == hipSuccess;
   int rcs[2] = {DVC_OK, DVC_OK};
   std::string err[2];
   auto run = [&](int k, hipStream_t s) {
@@ -507,10 +510,10 @@ int dvc_ldpca_decode_batch(dvc_ctx *c, int n, dvc_ldpca_item *items) {
       err[k] = "hipSetDevice failed";
       return;
     }
-    rcs[k] = decode_group(c, k ? 6336 : 1584, (int)g[k].size(), g[k].data(), 0, (int)g[1 - k].size(), s);
+    rcs[k] = decode_group(c, k ? 6336 : 1584, (int)g[k].size(), g[k].data(), 0, both ? (int)g[1 - k].size() : 0, s);
     if (rcs[k]) err[k] = dvc_last_error();
   };
-  if (!g[0].empty() && !g[1].empty()) {
+  if (both) {
     std::thread th;
     try {
       th = std::thread(run, 0, c->stream2);

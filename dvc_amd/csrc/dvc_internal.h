@@ -157,7 +157,7 @@ struct dvc_ctx {
     void *dev = nullptr, *host = nullptr;
     size_t devBytes = 0, hostBytes = 0;
   } ld[2];
-  hipStream_t stream2 = nullptr;  // the second code length of a mixed batch
+  hipStream_t stream2 = nullptr;  // the second code length of a mixed batch (made with the first one)
   void *noalloc_scratch = nullptr;  // device address of noalloc.hip's scratch array on this device
   dvc::BandState *band = nullptr;   // per-band entry points' frame state (dvc_band_frame_init)
   dvc::Ladder *ladder(int N) { return N == 1584 ? &lad1584 : (N == 6336 ? &lad6336 : nullptr); }

@@ -341,6 +341,7 @@ constexpr int kStageRing = 4;
 // lanes' kernels.
 struct Lane {
   hipStream_t s = nullptr, s2 = nullptr;  // s2: QCIF bitplanes beside CIF ones
+  int queue = 0;  // the first lane whose hardware queue s shares (its own number: none)
   hipEvent_t fork = nullptr, join = nullptr;
   int cap = 0;
   SlotPlan slots{};  // decision slots of each code length
@@ -378,7 +379,7 @@ struct Lane {
   std::vector<PlaneDesc> groups[2];
   // Captured launch sequences of steady steps (no frame starts or ends a
   // band), keyed by their launch shape: frames stepped, planes of each code
-  // length, largest code length, lanes stepping (which the BP launches share the
+  // length, largest code length, queues stepping (which the BP launches share the
   // CUs with).  Their kernels read the step's frame list,
   // frame descriptors and plane descriptors from this lane's buffers, which
   // are uploaded before each replay.
@@ -397,7 +398,7 @@ struct dvc_engine {
   uint64_t nextTicket = 1, clock = 0;
   std::deque<dvc::Job *> pending;
   std::vector<dvc::Lane> lanes;
-  int busyLanes = 1;  // lanes with frames in the current dvc_engine_step
+  int busyQueues = 1;  // hardware queues of the lanes with frames in the current dvc_engine_step
   std::map<uint64_t, int> doneTickets;  // ticket -> 1
   std::map<uint64_t, dvc::KeyEntry> keys;
   // device blocks of retired frames and dropped key frames, kept for reuse
@@ -797,9 +798,9 @@ static int lane_step(dvc_engine *e, Lane &ln) {
         hipStream_t gs = both && g == 0 ? ln.s2 : s;
         uint8_t *slots = ln.d_slots + (size_t)(g ? ln.slots.total : 0) * 6336;
         const int r = e->sequentialBp && c->bp_mode == 1
-                          ? bp_step_codes(c, g ? 6336 : 1584, ln.groups[g], e->busyLanes, slots, ln.slots,
+                          ? bp_step_codes(c, g ? 6336 : 1584, ln.groups[g], e->busyQueues, slots, ln.slots,
                                           ln.d_counters + 3 * g, g ? ln.d_area : nullptr, ln.d_planes + off, gs)
-                          : bp_step_launch(c, g ? 6336 : 1584, ng, e->sequentialBp, both ? (g ? n0 : n1) : 0, e->busyLanes,
+                          : bp_step_launch(c, g ? 6336 : 1584, ng, e->sequentialBp, both ? (g ? n0 : n1) : 0, e->busyQueues,
                                            slots, ln.slots, ln.d_counters + 3 * g, g ? ln.d_area : nullptr,
                                            ln.d_planes + off, gs);
         if (r) return r;
@@ -813,7 +814,7 @@ static int lane_step(dvc_engine *e, Lane &ln) {
       return DVC_OK;
     };
     if (steady) {
-      const auto key = std::make_tuple(na, n0, n1, maxN, e->busyLanes);
+      const auto key = std::make_tuple(na, n0, n1, maxN, e->busyQueues);
       auto it = ln.graphs.find(key);
       if (it == ln.graphs.end()) {
         DVC_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -896,18 +897,42 @@ static int lane_step(dvc_engine *e, Lane &ln) {
   return DVC_OK;
 }
 
+// Lane k's own stream, beside those of the lanes before it while there are hardware
+// queues left.  Lanes whose streams share a queue run one after the other; left to
+// the runtime, the streams of two lanes came to lie on one queue whenever the
+// process had made as many others before (one trace had 0.01 ms of overlap in 709
+// ms of kernels).
+static hipError_t lane_stream(dvc_engine *e, int k) {
+  Lane &l = e->lanes[k];
+  l.queue = k;
+  if (k == 0) return hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking);
+  std::vector<hipStream_t> with;
+  for (int i = 0; i < std::min(k, kBesideMax); i++) with.push_back(e->lanes[i].s);
+  uint32_t beside = 0;
+  const hipError_t err = create_stream_beside(with.data(), (int)with.size(), &l.s, &beside);
+  for (int i = (int)with.size() - 1; i >= 0; i--)
+    if (!(beside >> i & 1u)) l.queue = e->lanes[i].queue;
+  return err;
+}
+
 // What a lane needs for the code lengths of its frames, made with the first of
 // them: where split CIF launches meet, and the second stream of a lane with both
 // lengths (made after all lanes' own streams, so that these lie on as many hardware
-// queues as there are).  Finding a stream that runs beside the lane's takes up to
-// 0.9 ms, and a call that decodes one frame makes an engine for it: one CIF frame
-// 14.6 -> 14.1 ms, one QCIF frame the plain way 20.3 -> 19.7.
+// queues as there are, and beside the other lanes' streams if it can be).  Finding a
+// stream that runs beside others takes up to 0.9 ms, and a call that decodes one
+// frame makes an engine for it: one CIF frame 14.6 -> 14.1 ms, one QCIF frame the
+// plain way 20.3 -> 19.7.
 static int lane_prepare(dvc_engine *e, Lane &l) {
   bool have[2] = {false, false};
   for (const Job *j : l.inflight) have[j->N == 6336] = true;
   if (have[1] && !l.d_area) DVC_HIP(hipMalloc((void **)&l.d_area, sizeof(uint32_t) * split_area_words(6336)));
-  if (have[0] && have[1] && !l.s2 && !e->sequentialBp && e->c->bp_mode == 0)
-    DVC_HIP(create_stream_beside(l.s, &l.s2));
+  if (have[0] && have[1] && !l.s2 && !e->sequentialBp && e->c->bp_mode == 0) {
+    std::vector<hipStream_t> with = {l.s};
+    for (const Lane &o : e->lanes)
+      for (hipStream_t s : {o.s, o.s2})
+        if (&o != &l && s && (int)with.size() < kBesideMax) with.push_back(s);
+    DVC_HIP(create_stream_beside(with.data(), (int)with.size(), &l.s2, nullptr));
+  }
   return DVC_OK;
 }
 
@@ -958,7 +983,11 @@ static int engine_step(dvc_engine *e, int *completed) {
   for (auto &l : e->lanes)
     if (!l.inflight.empty()) busy.push_back(&l);
   if (busy.empty()) return DVC_OK;
-  e->busyLanes = (int)busy.size();
+  // lanes on one queue run one after the other: they do not share the CUs
+  std::vector<int> queues;
+  for (Lane *l : busy) queues.push_back(l->queue);
+  std::sort(queues.begin(), queues.end());
+  e->busyQueues = (int)(std::unique(queues.begin(), queues.end()) - queues.begin());
   for (Lane *l : busy)
     if ((rc = lane_prepare(e, *l))) return rc;
   // a lane keeps stepping without waiting for the others until one of its
@@ -1075,7 +1104,7 @@ static int engine_create(dvc_ctx *c, const dvc_engine_params *p, dvc_engine **ou
     l.oPlanes = align_up(l.oLinks + sizeof(BpFrameLink) * M);
     l.oSegs = align_up(l.oPlanes + sizeof(PlaneDesc) * M);
     l.stageBytes = align_up(l.oSegs + sizeof(CopySeg) * 4 * M);
-    err = hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking);
+    err = lane_stream(e, k);
     for (hipEvent_t *ev : {&l.fork, &l.join})
       if (err == hipSuccess) err = hipEventCreateWithFlags(ev, hipEventDisableTiming);
     if (err == hipSuccess) err = hipHostMalloc((void **)&l.h_stage, l.stageBytes * kStageRing, hipHostMallocDefault);

@@ -1189,44 +1189,69 @@ __global__ void zero_ints_kernel(int *p, int n) {
   if (i < n) p[i] = 0;
 }
 
-// Waits for flag[0] for at most 200 us and says in flag[1] whether it came.
-__global__ void await_flag_kernel(int *flag) {
+// Waits for flag[0] for at most 200 us and says in flag[1 + which] whether it came.
+__global__ void await_flag_kernel(int *flag, int which) {
   const uint64_t t0 = wall_clock64();  // 100 MHz
   int seen = 0;
   while (!seen && wall_clock64() - t0 < 20000) seen = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  flag[1] = seen;
+  flag[1 + which] = seen;
 }
 __global__ void raise_flag_kernel(int *flag) {
   __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ------------------------------------------------------------------ host side
-// The runtime spreads streams over a few hardware queues, and kernels of two
-// streams on the same queue run one after the other: 60 mixed bitplanes, whose two
-// launches share the CUs, took 2.5 ms on such a pair and 1.55 on others.  So a
-// stream that is to run beside s is tried with a kernel that waits on s for one on
-// the new stream (it gives up after 200 us), and replaced, four times at most.
-hipError_t create_stream_beside(hipStream_t s, hipStream_t *out) {
-  hipStream_t tried[4] = {};
-  int *flag = nullptr, got[2] = {0, 0}, n = 0;
+// The runtime spreads streams over a few hardware queues (four by default), and
+// kernels of two streams on the same queue run one after the other: 60 mixed
+// bitplanes, whose two launches share the CUs, took 2.5 ms on such a pair and 1.55
+// on others.  So a stream that is to run beside others is tried: a kernel on each
+// of them waits for one on the new stream (and gives up after 200 us).  The streams
+// tried meanwhile are kept, so that the next one lands on another queue, eight at
+// most; the one that ran beside with[0], then beside the most of the others, stays.
+hipError_t create_stream_beside(const hipStream_t *with, int n, hipStream_t *out, uint32_t *beside) {
+  constexpr int kTries = 8;
+  if (n < 1 || n > kBesideMax) return hipErrorInvalidValue;
+  const uint32_t all = (1u << n) - 1;
+  hipStream_t tried[kTries] = {};
+  int *flag = nullptr, got[1 + kBesideMax] = {}, made = 0, best = 0;
+  uint32_t bestMask = 0;
   *out = nullptr;
-  hipError_t e = hipMalloc((void **)&flag, 2 * sizeof(int));
-  while (e == hipSuccess && n < 4 && !got[1]) {
-    e = hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking);
+  hipError_t e = hipMalloc((void **)&flag, sizeof(got));
+  while (e == hipSuccess && made < kTries && bestMask != all) {
+    hipStream_t t;
+    if ((e = hipStreamCreateWithFlags(&t, hipStreamNonBlocking)) != hipSuccess) break;
+    tried[made++] = t;
+    if ((e = launch_zero_ints(flag, 1 + n, t)) == hipSuccess) e = hipStreamSynchronize(t);
     if (e != hipSuccess) break;
-    n++;
-    if ((e = launch_zero_ints(flag, 2, s)) == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) break;
-    hipLaunchKernelGGL(await_flag_kernel, dim3(1), dim3(1), 0, s, flag);
-    hipLaunchKernelGGL(raise_flag_kernel, dim3(1), dim3(1), 0, tried[n - 1], flag);
-    if ((e = hipGetLastError()) == hipSuccess) e = hipStreamSynchronize(tried[n - 1]);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    for (int k = 0; k < n; k++) hipLaunchKernelGGL(await_flag_kernel, dim3(1), dim3(1), 0, with[k], flag, k);
+    hipLaunchKernelGGL(raise_flag_kernel, dim3(1), dim3(1), 0, t, flag);
+    e = hipGetLastError();
+    const hipError_t et = hipStreamSynchronize(t);
+    if (e == hipSuccess) e = et;
+    for (int k = 0; k < n; k++) {
+      const hipError_t ek = hipStreamSynchronize(with[k]);
+      if (e == hipSuccess) e = ek;
+    }
     if (e == hipSuccess) e = hipMemcpy(got, flag, sizeof(got), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) break;
+    uint32_t mask = 0;
+    for (int k = 0; k < n; k++) mask |= got[1 + k] ? 1u << k : 0u;
+    auto score = [](uint32_t m) { return (m & 1u) * 64 + (uint32_t)__builtin_popcount(m); };
+    if (score(mask) > score(bestMask)) {
+      best = made - 1;
+      bestMask = mask;
+    }
   }
-  for (int k = 0; k < n; k++)
-    if (e == hipSuccess && k == n - 1) *out = tried[k];
-    else (void)hipStreamDestroy(tried[k]);
+  // with no more streams or memory to be had, the best one so far will do
+  if (made > 0) {
+    *out = tried[best];
+    if (e != hipSuccess) (void)hipGetLastError();
+    e = hipSuccess;
+  }
+  for (int k = 0; k < made; k++)
+    if (k != best) (void)hipStreamDestroy(tried[k]);
   if (flag) (void)hipFree(flag);
+  if (beside) *beside = bestMask;
   return e;
 }
 

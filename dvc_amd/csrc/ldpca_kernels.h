@@ -115,8 +115,11 @@ hipError_t launch_bp_any(int N, int threads, const BpArgs &a, int grid, hipStrea
 // blocks if they are not, then `clusters` groups of a.split workgroups.
 hipError_t launch_bp_split(int N, const BpArgs &a, int clusters, hipStream_t s);
 hipError_t launch_zero_ints(int *p, int n, hipStream_t s);
-// A non-blocking stream whose kernels run beside s's, if the device has one left.
-hipError_t create_stream_beside(hipStream_t s, hipStream_t *out);
+// A non-blocking stream whose kernels run beside those of the n streams `with`, or,
+// where the hardware queues do not suffice, beside with[0] and as many of the
+// others as can be.  Bit k of *beside (may be NULL): it runs beside with[k].
+constexpr int kBesideMax = 31;
+hipError_t create_stream_beside(const hipStream_t *with, int n, hipStream_t *out, uint32_t *beside);
 hipError_t launch_mode1_resolve(const PlaneDesc *planes, int n, int numCodes, int N, const uint8_t *slots,
                                 int slot_capacity, int *rerun_count, hipStream_t s);
 // Entropy, LLRs and start codes of n bitplanes; also clears the three launch

@@ -1,0 +1,59 @@
+"""Engine lanes run beside one another on the GPU, whatever streams the process
+made before, and decode what one lane decodes (few CIF frames a lane, so that the
+lanes' split BP launches share the CUs)."""
+import time
+
+import numpy as np
+import pytest
+
+from dvc_amd import _lib
+from dvc_amd import workload as W
+
+pytestmark = pytest.mark.gpu
+
+KERNELS = ("bp_6336", "ce_llr", "invh", "condbit", "put_bitplane", "noise_dist", "update_si", "oct", "update_smf",
+           "update_si_ml", "reconstruct", "inverse_transform", "create_si", "noise_param")
+PER_LANE = 4
+
+
+def _frames(n):
+    vid = W.synthetic_video(352, 288, 3, 4, seed=301)
+    wz = W.encode_wz_frame(vid[1], 6)
+    return [dict(past=vid[0], fut=vid[2], wz=wz)] * n
+
+
+def _run(ctx, frames, lanes):
+    """Results, and the sum of the kernels' durations over the time taken."""
+    eng = _lib.Engine(ctx, max_inflight=len(frames), lanes=lanes, lane_steps=1 << 20)
+    eng.decode_all(frames)
+    ctx.profile(True)
+    t0 = time.perf_counter()
+    out = eng.decode_all(frames)
+    wall = time.perf_counter() - t0
+    total = sum(ctx.profile_get(k)[0] for k in KERNELS)
+    ctx.profile(False)
+    eng.close()
+    return out, total / 1e3 / wall
+
+
+@pytest.mark.parametrize("lanes", [2, 3])
+def test_lanes_overlap(lanes):
+    """With k lanes of equal work side by side the kernels' durations add up to
+    nearly k times the time taken (0.86 to 0.9 of it on one lane, the rest are
+    gaps); with two lanes on one hardware queue to at most (k - 1) times it, and to
+    0.9 with two lanes in all.  0.68 k lies between."""
+    frames = _frames(PER_LANE * lanes)
+    others = []
+    try:
+        for extra in range(4):
+            ctx = _lib.Context(max_iter=50)
+            others.append(ctx)  # its streams stay while the next one is made
+            out, ratio = _run(ctx, frames, lanes)
+            print(f"lanes {lanes}, {extra} other contexts: {ratio:.2f}", flush=True)
+            one, _ = _run(ctx, frames[:PER_LANE], 1)
+            for rec, st in out:
+                assert np.array_equal(rec, one[0][0]) and st == one[0][1]
+            assert ratio > 0.68 * lanes, extra
+    finally:
+        for c in others:
+            c.close()
