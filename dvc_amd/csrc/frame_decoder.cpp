@@ -28,6 +28,7 @@
 #include "frame_kernels.h"
 #include "ldpca_kernels.h"
 #include "engine_kernels.h"
+#include "stage_plan.h"
 
 namespace dvc {
 
@@ -1218,13 +1219,13 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
   if (rc) return rc;
   hipStream_t s = c->stream;
   // One device allocation, kept for later calls (grown when too small): first
-  // what goes up with one copy (frame descriptors, key-frame jobs, list, key
-  // frames), then what comes back (side information, residue and alpha of one
-  // request after another), then per request the filtered key frames and the
-  // motion-field scratch.  The first two regions have a pinned host mirror,
-  // which the caller's buffers are copied to and from by several threads: with
-  // five pageable copies per request, 64 CIF pairs took 13.2 ms, 2 of them
-  // kernels; now 7.2, most of it the first touch of 58 MB of results.
+  // what goes up (frame descriptors, key-frame jobs, list, key frames), then what
+  // comes back (side information, residue and alpha of one request after another),
+  // then per request the filtered key frames and the motion-field scratch.  The
+  // first two regions travel through a ring of pinned slots, which the caller's
+  // buffers are copied to and from by several threads: with five pageable copies
+  // per request, 64 CIF pairs took 13.2 ms, 2 of them kernels; now 7.2, most of it
+  // the first touch of 58 MB of results.
   std::vector<size_t> up(n + 1), out(n + 1), own(n + 1);
   const size_t oFrames = 0, oJobs = align_up(sizeof(FrameDev) * n), oList = oJobs + align_up(sizeof(KeyFrameJob) * 2 * n);
   up[0] = oList + align_up(sizeof(int) * n);
@@ -1255,11 +1256,10 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
     DVC_HIP(hipMalloc(&c->si_scratch, own[n]));
     c->si_scratch_bytes = own[n];
   }
-  if ((rc = pinned_grow(&c->si_host, &c->si_host_bytes, own[0]))) return rc;
-  uint8_t *dev = (uint8_t *)c->si_scratch, *host = c->si_host;
-  FrameDev *hf = (FrameDev *)(host + oFrames);
-  KeyFrameJob *hk = (KeyFrameJob *)(host + oJobs);
-  std::vector<HostCopy> copies;
+  uint8_t *dev = (uint8_t *)c->si_scratch;
+  std::vector<uint8_t> head(up[0]);  // the descriptors
+  FrameDev *hf = (FrameDev *)(head.data() + oFrames);
+  KeyFrameJob *hk = (KeyFrameJob *)(head.data() + oJobs);
   for (int i = 0; i < n; i++) {
     const dvc_si_request &r = reqs[i];
     const int W = r.width, H = r.height;
@@ -1284,43 +1284,79 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
     f.holes = (double *)take(16 * (FS / 256));
     f.npPart = (uint2 *)take(np_part_bytes(FS / 16));
     f.npMom = (float2 *)take(kNpMomBytes);
-    ((int *)(host + oList))[i] = i;
-    copies.push_back(HostCopy{host + up[i], r.past, FS});
-    copies.push_back(HostCopy{host + up[i] + FS, r.fut, FS});
+    ((int *)(head.data() + oList))[i] = i;
     hk[2 * i] = KeyFrameJob{dev + up[i], kp, kp + FS, kp + 2 * FS, W, H};
     hk[2 * i + 1] = KeyFrameJob{dev + up[i] + FS, kf, kf + FS, kf + 2 * FS, W, H};
   }
-  host_copy(c, copies);
+  // what goes up is cut anywhere, results between requests
+  std::vector<HostCopy> rising{HostCopy{nullptr, head.data(), head.size()}};
+  for (int i = 0; i < n; i++) {
+    const size_t FS = (size_t)reqs[i].width * reqs[i].height;
+    rising.push_back(HostCopy{nullptr, reqs[i].past, FS});
+    rising.push_back(HostCopy{nullptr, reqs[i].fut, FS});
+  }
+  const size_t upSlot = std::min(up[n], kStageSlot);
+  const int ups = (int)((up[n] + upSlot - 1) / upSlot);
+  const std::vector<int> cut = stage_pieces(out, std::min(8, (n + 3) / 4));
+  const int downs = (int)cut.size() - 1, slots = std::min(kStageSlots, std::max(ups, downs));
+  const size_t slotBytes = align_up(std::max(upSlot, stage_slot_bytes(out, cut)));
+  if ((rc = pinned_grow(&c->si_host, &c->si_host_bytes, slots * slotBytes))) return rc;
+  hipEvent_t ev[kStageSlots] = {};  // the slot's transfer is done
+  auto slot = [&](int k) { return c->si_host + (k % slots) * slotBytes; };
+  auto transferred = [&](int k) -> int {
+    hipEvent_t &e = ev[k % slots];
+    if (!e) DVC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    DVC_HIP(hipEventRecord(e, s));
+    return DVC_OK;
+  };
   const FrameDev *df = (const FrameDev *)(dev + oFrames);
   const int *dl = (const int *)(dev + oList);
-  constexpr int kChunks = 8;  // the results come back in up to this many copies
-  hipEvent_t ev[kChunks] = {};
-  const int chunks = std::min(kChunks, (n + 3) / 4);
-  auto first = [&](int k) { return (int)((long)n * k / chunks); };
+  std::vector<HostCopy> copies;
   auto run = [&]() -> int {
-    DVC_HIP(hipMemcpyAsync(dev, host, up[n], hipMemcpyHostToDevice, s));
+    size_t src = 0, done = 0;  // in `rising`
+    for (int k = 0; k < ups; k++) {
+      if (k >= slots) DVC_HIP(hipEventSynchronize(ev[k % slots]));
+      const size_t a = k * upSlot, bytes = std::min(upSlot, up[n] - a);
+      copies.clear();
+      for (size_t at = 0; at < bytes;) {
+        const size_t len = std::min(bytes - at, rising[src].bytes - done);
+        copies.push_back(HostCopy{slot(k) + at, (const uint8_t *)rising[src].src + done, len});
+        at += len;
+        done += len;
+        if (done == rising[src].bytes) {
+          src++;
+          done = 0;
+        }
+      }
+      host_copy(c, copies);
+      DVC_HIP(hipMemcpyAsync(dev + a, slot(k), bytes, hipMemcpyHostToDevice, s));
+      if (ups > slots && (rc = transferred(k))) return rc;
+    }
     TIMED_LAUNCH(c, "keyframe_filters", s,
                  launch_keyframe_batch((const KeyFrameJob *)(dev + oJobs), 2 * n, maxW, maxH, s));
     CostTables ct{c->d_costFme, c->d_costUsi};
     TIMED_LAUNCH(c, "create_si", s, launch_create_si(df, dl, n, maxMB, ct, s));
     TIMED_LAUNCH(c, "noise_param", s, launch_noise_param(df, dl, n, maxN, s));
-    for (int k = 0; k < chunks; k++) {
-      const size_t a = out[first(k)], b = out[first(k + 1)];
-      DVC_HIP(hipMemcpyAsync(host + a, dev + a, b - a, hipMemcpyDeviceToHost, s));
-      DVC_HIP(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
-      DVC_HIP(hipEventRecord(ev[k], s));
-    }
-    for (int k = 0; k < chunks; k++) {
-      DVC_HIP(hipEventSynchronize(ev[k]));
+    auto fetch = [&](int k) -> int {
+      const size_t a = out[cut[k]];
+      DVC_HIP(hipMemcpyAsync(slot(k), dev + a, out[cut[k + 1]] - a, hipMemcpyDeviceToHost, s));
+      return transferred(k);
+    };
+    for (int k = 0; k < std::min(slots, downs); k++)
+      if ((rc = fetch(k))) return rc;
+    for (int k = 0; k < downs; k++) {
+      DVC_HIP(hipEventSynchronize(ev[k % slots]));
       copies.clear();
-      for (int i = first(k); i < first(k + 1); i++) {
+      for (int i = cut[k]; i < cut[k + 1]; i++) {
         const dvc_si_request &r = reqs[i];
         const size_t FS = (size_t)r.width * r.height;
-        copies.push_back(HostCopy{r.si, host + out[i], FS});
-        if (r.residue) copies.push_back(HostCopy{r.residue, host + out[i] + FS, 4 * FS});
-        if (r.alpha) copies.push_back(HostCopy{r.alpha, host + out[i] + 5 * FS, 4 * FS});
+        const uint8_t *h = slot(k) + (out[i] - out[cut[k]]);
+        copies.push_back(HostCopy{r.si, h, FS});
+        if (r.residue) copies.push_back(HostCopy{r.residue, h + FS, 4 * FS});
+        if (r.alpha) copies.push_back(HostCopy{r.alpha, h + 5 * FS, 4 * FS});
       }
       host_copy(c, copies);
+      if (k + slots < downs && (rc = fetch(k + slots))) return rc;
     }
     return DVC_OK;
   };
