@@ -1239,13 +1239,15 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
     maxH = std::max(maxH, reqs[i].height);
   }
   out[0] = align_up(up[n]);
-  for (int i = 0; i < n; i++) out[i + 1] = out[i] + 9 * (size_t)reqs[i].width * reqs[i].height;
+  // (a result that a request leaves out stays with the request's own buffers)
+  for (int i = 0; i < n; i++)
+    out[i + 1] = out[i] + si_result_bytes((size_t)reqs[i].width * reqs[i].height, reqs[i].residue, reqs[i].alpha);
   own[0] = align_up(out[n]);
   for (int i = 0; i < n; i++) {
     const size_t FS = (size_t)reqs[i].width * reqs[i].height;
     size_t t = 0;
     for (size_t b : {12 * FS, 4 * FS, sizeof(MVs) * (FS / 64), sizeof(MVd) * (FS / 256), 16 * (FS / 256),
-                     np_part_bytes(FS / 16), kNpMomBytes})
+                     np_part_bytes(FS / 16), kNpMomBytes, reqs[i].residue ? 0 : 4 * FS, reqs[i].alpha ? 0 : 4 * FS})
       t = align_up(t + b);
     own[i + 1] = own[i] + t;
   }
@@ -1276,8 +1278,15 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
     f.past = kp; f.past_lp = kp + FS; f.past_half = kp + 2 * FS;
     f.fut = kf; f.fut_lp = kf + FS; f.fut_half = kf + 2 * FS;
     f.si = dev + out[i];
-    f.residue = (int *)(dev + out[i] + FS);
-    f.alpha = (float *)(dev + out[i] + 5 * FS);
+    uint8_t *next = dev + out[i] + FS;
+    auto result = [&](const void *wanted) {
+      if (!wanted) return take(4 * FS);
+      uint8_t *q = next;
+      next += 4 * FS;
+      return q;
+    };
+    f.residue = (int *)result(r.residue);
+    f.alpha = (float *)result(r.alpha);
     f.sideTrans = (int *)take(4 * FS);
     f.bmv = (MVs *)take(sizeof(MVs) * (FS / 64));
     f.fwd = (MVd *)take(sizeof(MVd) * (FS / 256));
@@ -1352,8 +1361,10 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
         const size_t FS = (size_t)r.width * r.height;
         const uint8_t *h = slot(k) + (out[i] - out[cut[k]]);
         copies.push_back(HostCopy{r.si, h, FS});
-        if (r.residue) copies.push_back(HostCopy{r.residue, h + FS, 4 * FS});
-        if (r.alpha) copies.push_back(HostCopy{r.alpha, h + 5 * FS, 4 * FS});
+        h += FS;
+        if (r.residue) copies.push_back(HostCopy{r.residue, h, 4 * FS});
+        if (r.residue) h += 4 * FS;
+        if (r.alpha) copies.push_back(HostCopy{r.alpha, h, 4 * FS});
       }
       host_copy(c, copies);
       if (k + slots < downs && (rc = fetch(k + slots))) return rc;

@@ -38,4 +38,10 @@ inline size_t stage_slot_bytes(const std::vector<size_t> &at, const std::vector<
   return m;
 }
 
+// Bytes that come back for one side-information request: a byte a pixel of side
+// information and four each of residue and alpha, nothing of what it leaves out.
+inline size_t si_result_bytes(size_t pixels, bool residue, bool alpha) {
+  return pixels * (1 + (residue ? 4 : 0) + (alpha ? 4 : 0));
+}
+
 }  // namespace dvc

@@ -42,6 +42,9 @@ int main() {
   for (int i = 0; i < 64; i++) at.push_back(at.back() + cif);
   expect(stage_pieces(at, 8) == std::vector<int>({0, 8, 16, 24, 32, 40, 48, 56, 64}), "eights", 64, 0);
   expect(kStageSlots * kStageSlot <= (64u << 20), "ring", 0, 0);
+  expect(si_result_bytes(100, false, false) == 100 && si_result_bytes(100, true, false) == 500 &&
+             si_result_bytes(100, false, true) == 500 && si_result_bytes(100, true, true) == 900,
+         "result bytes", 0, 0);
   puts(failures ? "FAILED" : "ok");
   return failures != 0;
 }

@@ -3,6 +3,7 @@ pieces: the same results as pair by pair."""
 import numpy as np
 import pytest
 
+from dvc_amd import _lib
 from dvc_amd import workload as W
 
 pytestmark = pytest.mark.gpu
@@ -31,3 +32,26 @@ def test_batches_larger_than_the_ring(ctx, cif, qcif):
         (one,) = ctx.side_info_batch([p])
         for a, b in zip(g, one):
             assert np.array_equal(a, b), k
+
+
+def test_results_left_out(ctx):
+    """Requests without residue, without alpha and without either beside full ones:
+    what is asked for is the same, and nothing else is written."""
+    sizes = [(352, 288), (176, 144), (176, 144), (352, 288), (176, 144)] * 8
+    pairs = _pairs(sizes)
+    want = ctx.side_info_batch(pairs)
+    reqs = (_lib.SIRequest * len(pairs))()
+    got = []
+    for k, p in enumerate(pairs):
+        h, w = p["past"].shape
+        out = (np.full((h, w), 7, np.uint8), np.full((h, w), 7, np.int32), np.full((h, w), 7, np.float32))
+        got.append(out)
+        pi, ci, fi = p["idx"]
+        reqs[k] = _lib.SIRequest(w, h, p["qindex"], pi, ci, fi, p["past"].ctypes.data, p["fut"].ctypes.data,
+                                 out[0].ctypes.data, out[1].ctypes.data if k % 2 else None,
+                                 out[2].ctypes.data if k % 3 else None)
+    _lib._check(_lib.lib.dvc_side_info_batch(ctx.h, len(pairs), reqs), "dvc_side_info_batch")
+    for k, (a, b) in enumerate(zip(got, want)):
+        assert np.array_equal(a[0], b[0])
+        assert np.array_equal(a[1], b[1] if k % 2 else np.full_like(a[1], 7)), k
+        assert np.array_equal(a[2], b[2] if k % 3 else np.full_like(a[2], 7)), k
