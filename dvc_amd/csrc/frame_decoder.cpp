@@ -1307,9 +1307,10 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
   const size_t upSlot = std::min(up[n], kStageSlot);
   const int ups = (int)((up[n] + upSlot - 1) / upSlot);
   const std::vector<int> cut = stage_pieces(out, std::min(8, (n + 3) / 4));
-  const int downs = (int)cut.size() - 1, slots = std::min(kStageSlots, std::max(ups, downs));
+  const int downs = (int)cut.size() - 1, slots = std::min(kStageSlots, ups + downs);
   const size_t slotBytes = align_up(std::max(upSlot, stage_slot_bytes(out, cut)));
   if ((rc = pinned_grow(&c->si_host, &c->si_host_bytes, slots * slotBytes))) return rc;
+  // transfer t, of the pieces up and then those down, uses slot t % slots
   hipEvent_t ev[kStageSlots] = {};  // the slot's transfer is done
   auto slot = [&](int k) { return c->si_host + (k % slots) * slotBytes; };
   auto transferred = [&](int k) -> int {
@@ -1348,18 +1349,18 @@ int dvc_side_info_batch(dvc_ctx *c, int n, const dvc_si_request *reqs) {
     TIMED_LAUNCH(c, "noise_param", s, launch_noise_param(df, dl, n, maxN, s));
     auto fetch = [&](int k) -> int {
       const size_t a = out[cut[k]];
-      DVC_HIP(hipMemcpyAsync(slot(k), dev + a, out[cut[k + 1]] - a, hipMemcpyDeviceToHost, s));
-      return transferred(k);
+      DVC_HIP(hipMemcpyAsync(slot(ups + k), dev + a, out[cut[k + 1]] - a, hipMemcpyDeviceToHost, s));
+      return transferred(ups + k);
     };
     for (int k = 0; k < std::min(slots, downs); k++)
       if ((rc = fetch(k))) return rc;
     for (int k = 0; k < downs; k++) {
-      DVC_HIP(hipEventSynchronize(ev[k % slots]));
+      DVC_HIP(hipEventSynchronize(ev[(ups + k) % slots]));
       copies.clear();
       for (int i = cut[k]; i < cut[k + 1]; i++) {
         const dvc_si_request &r = reqs[i];
         const size_t FS = (size_t)r.width * r.height;
-        const uint8_t *h = slot(k) + (out[i] - out[cut[k]]);
+        const uint8_t *h = slot(ups + k) + (out[i] - out[cut[k]]);
         copies.push_back(HostCopy{r.si, h, FS});
         h += FS;
         if (r.residue) copies.push_back(HostCopy{r.residue, h, 4 * FS});
