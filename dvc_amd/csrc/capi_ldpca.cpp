@@ -5,10 +5,10 @@
 #include <string.h>
 #include <dlfcn.h>
 #include <string>
-#include <thread>
 #include <vector>
 #include <algorithm>
 #include "dvc_internal.h"
+#include "host_pair.h"
 #include "ldpca_kernels.h"
 
 namespace dvc {
@@ -504,27 +504,23 @@ int dvc_ldpca_decode_batch(dvc_ctx *c, int n, dvc_ldpca_item *items) {
   if (both && !c->stream2) both = create_stream_beside(&c->stream, 1, &c->stream2, nullptr) == hipSuccess;
   int rcs[2] = {DVC_OK, DVC_OK};
   std::string err[2];
-  auto run = [&](int k, hipStream_t s) {
-    if (hipSetDevice(c->device) != hipSuccess) {
-      rcs[k] = DVC_EDEVICE;
-      err[k] = "hipSetDevice failed";
-      return;
-    }
-    rcs[k] = decode_group(c, k ? 6336 : 1584, (int)g[k].size(), g[k].data(), 0, both ? (int)g[1 - k].size() : 0, s);
-    if (rcs[k]) err[k] = dvc_last_error();
+  auto part = [&](int k, hipStream_t s) -> int {
+    DVC_HIP(hipSetDevice(c->device));
+    return decode_group(c, k ? 6336 : 1584, (int)g[k].size(), g[k].data(), 0, both ? (int)g[1 - k].size() : 0, s);
+  };
+  auto told = [&](int k, hipStream_t s) -> int {  // its error text is the thread's
+    const int rc = part(k, s);
+    if (rc) err[k] = dvc_last_error();
+    return rc;
   };
   if (both) {
-    std::thread th;
-    try {
-      th = std::thread(run, 0, c->stream2);
-    } catch (...) {  // no thread to be had: on this one, first
-    }
-    if (!th.joinable()) run(0, c->stream2);
-    run(1, c->stream);
-    if (th.joinable()) th.join();
+    run_pair([&] { return told(0, c->stream2); }, [&] { return told(1, c->stream); }, DVC_ENOMEM, rcs, err);
+    // what a part that failed left on its stream still reads the staging
+    if (rcs[0]) (void)hipStreamSynchronize(c->stream2);
+    if (rcs[1]) (void)hipStreamSynchronize(c->stream);
   } else {
     for (int k = 0; k < 2; k++)
-      if (!g[k].empty()) run(k, c->stream);
+      if (!g[k].empty()) rcs[k] = told(k, c->stream);
   }
   for (int k = 0; k < 2; k++) {
     if (rcs[k]) {
