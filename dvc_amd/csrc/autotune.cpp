@@ -89,6 +89,13 @@ int time_batch(dvc_ctx *c, Batch &b, double *ms) {
   return DVC_OK;
 }
 
+void apply(dvc_ctx *c, const dvc_tuning &t) {
+  c->bp_threads_cif = t.cif_threads;
+  c->bp_threads_qcif = t.qcif_threads;
+  c->bp_wg_per_cu_qcif = t.qcif_wg_per_cu;
+  c->bp_poll = t.poll;
+}
+
 }  // namespace
 
 extern "C" {
@@ -111,10 +118,7 @@ int dvc_set_tuning(dvc_ctx *c, const dvc_tuning *t) {
             "dvc_set_tuning: qcif_threads must be 256 or 512");
   DVC_CHECK(t->qcif_wg_per_cu >= 1 && t->qcif_wg_per_cu <= 4, DVC_EINVAL, "dvc_set_tuning: qcif_wg_per_cu must be 1..4");
   DVC_CHECK(t->poll >= 1 && t->poll <= 8, DVC_EINVAL, "dvc_set_tuning: poll must be 1..8");
-  c->bp_threads_cif = t->cif_threads;
-  c->bp_threads_qcif = t->qcif_threads;
-  c->bp_wg_per_cu_qcif = t->qcif_wg_per_cu;
-  c->bp_poll = t->poll;
+  apply(c, *t);
   return DVC_OK;
 }
 
@@ -126,55 +130,63 @@ int dvc_autotune(dvc_ctx *c, int planes, dvc_tuning *out) {
   Batch cif, qcif;
   make_batch(c->lad6336, n, 0x6336ull, cif);
   make_batch(c->lad1584, n, 0x1584ull, qcif);
+  // A setting that batches of this size do not reach is left as it is: its variants
+  // would all be the same launch, and the fastest of them chance.
+  std::vector<int> cifThreads{cur.cif_threads}, qcifThreads{cur.qcif_threads}, qcifPerCu{cur.qcif_wg_per_cu};
+  if (bp_tuned(c, 6336, n)) cifThreads = {1024, 704, 512};
+  if (bp_tuned(c, 1584, n)) {
+    qcifThreads = {256, 512};
+    qcifPerCu = {4, 2};
+  }
   int rc;
   // every variant must decode exactly what the first one decodes
   auto check_same = [](const Batch &b, const std::vector<std::vector<uint8_t>> &ref) { return b.out == ref; };
   std::vector<std::vector<uint8_t>> refC, refQ;
   double bestC = 1e30, bestQ = 1e30;
   dvc_tuning best = cur;
-  for (int T : {1024, 704, 512}) {
+  for (int T : cifThreads) {
     dvc_tuning t = cur;
     t.cif_threads = T;
-    dvc_set_tuning(c, &t);
+    apply(c, t);
     double ms;
-    if ((rc = time_batch(c, cif, &ms))) { dvc_set_tuning(c, &cur); return rc; }
+    if ((rc = time_batch(c, cif, &ms))) { apply(c, cur); return rc; }
     if (refC.empty()) {
       refC = cif.out;
-      if (refC != cif.bits) { dvc_set_tuning(c, &cur); set_error("dvc_autotune: calibration batch decoded wrongly"); return DVC_ESTATE; }
+      if (refC != cif.bits) { apply(c, cur); set_error("dvc_autotune: calibration batch decoded wrongly"); return DVC_ESTATE; }
     }
-    else if (!check_same(cif, refC)) { dvc_set_tuning(c, &cur); set_error("dvc_autotune: variants decoded differently"); return DVC_ESTATE; }
+    else if (!check_same(cif, refC)) { apply(c, cur); set_error("dvc_autotune: variants decoded differently"); return DVC_ESTATE; }
     if (ms < bestC) { bestC = ms; best.cif_threads = T; }
   }
-  for (int T : {256, 512})
-    for (int w : {4, 2}) {
+  for (int T : qcifThreads)
+    for (int w : qcifPerCu) {
       dvc_tuning t = cur;
       t.qcif_threads = T;
       t.qcif_wg_per_cu = w;
-      dvc_set_tuning(c, &t);
+      apply(c, t);
       double ms;
-      if ((rc = time_batch(c, qcif, &ms))) { dvc_set_tuning(c, &cur); return rc; }
+      if ((rc = time_batch(c, qcif, &ms))) { apply(c, cur); return rc; }
       if (refQ.empty()) {
         refQ = qcif.out;
-        if (refQ != qcif.bits) { dvc_set_tuning(c, &cur); set_error("dvc_autotune: calibration batch decoded wrongly"); return DVC_ESTATE; }
+        if (refQ != qcif.bits) { apply(c, cur); set_error("dvc_autotune: calibration batch decoded wrongly"); return DVC_ESTATE; }
       }
-      else if (!check_same(qcif, refQ)) { dvc_set_tuning(c, &cur); set_error("dvc_autotune: variants decoded differently"); return DVC_ESTATE; }
+      else if (!check_same(qcif, refQ)) { apply(c, cur); set_error("dvc_autotune: variants decoded differently"); return DVC_ESTATE; }
       if (ms < bestQ) { bestQ = ms; best.qcif_threads = T; best.qcif_wg_per_cu = w; }
     }
   double bestTot = 1e30;
   for (int poll : {1, 2, 4}) {
     dvc_tuning t = best;
     t.poll = poll;
-    dvc_set_tuning(c, &t);
+    apply(c, t);
     double a, b;
-    if ((rc = time_batch(c, cif, &a)) || (rc = time_batch(c, qcif, &b))) { dvc_set_tuning(c, &cur); return rc; }
+    if ((rc = time_batch(c, cif, &a)) || (rc = time_batch(c, qcif, &b))) { apply(c, cur); return rc; }
     if (!check_same(cif, refC) || !check_same(qcif, refQ)) {
-      dvc_set_tuning(c, &cur);
+      apply(c, cur);
       set_error("dvc_autotune: variants decoded differently");
       return DVC_ESTATE;
     }
     if (a + b < bestTot) { bestTot = a + b; best.poll = poll; best.cif_ms = a; best.qcif_ms = b; }
   }
-  dvc_set_tuning(c, &best);
+  apply(c, best);
   if (out) *out = best;
   return DVC_OK;
 }

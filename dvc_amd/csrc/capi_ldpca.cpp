@@ -70,11 +70,18 @@ int bp_grid(const dvc_ctx *c, int N, int items, int planes, int other) {
 // hangs on how many codes the bitplanes need (16: 0.91 against 0.99, 20: 1.12
 // against 1.02).  One bitplane: 0.84 unsplit, 0.48 with 4, 0.42 with 8.  A QCIF
 // codeword's iteration is shorter than an exchange between workgroups: never.
-static int bp_split(const dvc_ctx *c, int N, int planes, int other, int lanes, bool sequential, const BpArgs &a) {
-  if (!a.area || N != 6336 || !a.lad.regular || a.max_iter < 1) return 1;
-  const int cus = launch_cus(c, N, planes, other) / lanes, codewords = sequential ? 1 : 8 * planes;
+static int split_width(int cus, int codewords) {
   if (3 * codewords > cus) return 1;
   return std::max(4, std::min(kSplitMax, cus / codewords));
+}
+static int bp_split(const dvc_ctx *c, int N, int planes, int other, int lanes, bool sequential, const BpArgs &a) {
+  if (!a.area || N != 6336 || !a.lad.regular || a.max_iter < 1) return 1;
+  return split_width(launch_cus(c, N, planes, other) / lanes, sequential ? 1 : 8 * planes);
+}
+
+bool bp_tuned(const dvc_ctx *c, int N, int planes) {
+  if (N == 6336) return split_width(c->sm_count, 8 * planes) == 1;
+  return c->lad1584.regular && bp_threads(c, N, planes) == c->bp_threads_qcif;
 }
 
 hipError_t launch_bp(const dvc_ctx *c, int N, int planes, int other, int lanes, bool sequential, const BpArgs &a,

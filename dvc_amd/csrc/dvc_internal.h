@@ -75,6 +75,10 @@ int load_ladder(const std::string &dir, const char *kind, int N, Ladder &L);
 // tuning, but for small QCIF launches).
 int bp_threads(const dvc_ctx *c, int N, int planes);
 int bp_grid(const dvc_ctx *c, int N, int items, int planes, int other);
+// Whether a batch of `planes` bitplanes of one length runs in the launch shape that
+// the tuning names; fewer bitplanes run split or with 1024 threads, and an irregular
+// ladder has one shape.
+bool bp_tuned(const dvc_ctx *c, int N, int planes);
 // The BP launch of `planes` bitplanes' queued items (a.total of them): persistent,
 // or split over several workgroups per codeword when a.area is given and the
 // launch would leave most CUs idle.  lanes: launches like it that other streams

@@ -40,7 +40,7 @@ typedef struct {
                             (LdpcaDecoder.h:4); <= 0 selects 50 */
   const char *data_dir;  /* directory with reg1584.ladder / reg6336.ladder; NULL = the
                             library's own data directory */
-  int bp_threads;        /* threads per BP workgroup for N=6336 (0 = default 1024; see dvc_autotune) */
+  int bp_threads;        /* threads per BP workgroup for N=6336 (0 = default 1024; see dvc_tuning.cif_threads) */
   int parallel_mode;     /* BP semantics: 0 = beliefPropagation (ParallelMode 0/2, LdpcaDecoder.cpp:462-580);
                             1 = beliefPropagation_OpenMP (ParallelMode 1, :164-306): decisions LLR < 0 and a
                             failure after 4 consecutive iterations with unchanged decisions, compared first
@@ -143,11 +143,15 @@ int dvc_ldpca_decode_batch_noalloc(dvc_ctx *ctx, int n, dvc_ldpca_item *items);
  * autotuner).  dvc_autotune decodes a synthetic calibration batch of
  * `planes` bitplanes per code length (0: 128) with each variant, checks that
  * all variants decode the same bits, keeps the fastest in the context and
- * returns it.  The choice changes time only, never results. */
+ * returns it; a setting that batches of that size do not use is left as it was.
+ * The choice changes time only, never results. */
 typedef struct {
-  int cif_threads;      /* threads per workgroup for N = 6336: 512, 704 or 1024 */
+  int cif_threads;      /* threads per workgroup for N = 6336: 512, 704 or 1024 (launches of
+                           few bitplanes, up to ten on 256 CUs, split each codeword over
+                           several workgroups of 1024 whatever is set) */
   int qcif_threads;     /* threads per workgroup for N = 1584: 256 or 512 (launches of few
-                           bitplanes use 1024 whatever is set) */
+                           bitplanes, up to 32 on 256 CUs, use 1024 whatever is set, and so
+                           does the irregular ladder) */
   int qcif_wg_per_cu;   /* QCIF codewords (workgroups) per CU in the persistent grid: 1..4 */
   int poll;             /* BP iterations between a speculative item's cancellation polls: 1..8 */
   double cif_ms, qcif_ms;  /* dvc_autotune: calibration time of the chosen variant */
