@@ -1479,9 +1479,14 @@ hipError_t launch_keyframe_filters(const uint8_t *in, uint8_t *lp, uint8_t *half
   return hipGetLastError();
 }
 hipError_t launch_keyframe_batch(const KeyFrameJob *jobs, int n, int maxW, int maxH, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_keyframe_batch, dim3((2 * maxW + 127) / 128, maxH, n), dim3(128), 0, s, jobs);
-  return hipGetLastError();
+  constexpr int kMost = 32768;  // a side-information batch has two per pair, whose grids take 65535
+  for (int k = 0; k < n; k += kMost) {
+    hipLaunchKernelGGL(k_keyframe_batch, dim3((2 * maxW + 127) / 128, maxH, n - k < kMost ? n - k : kMost), dim3(128), 0, s,
+                       jobs + k);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 hipError_t launch_create_si(const FrameDev *F, const int *list, int n, int maxMB, CostTables ct, hipStream_t s) {
   // 4x4 tiles of 8x8 blocks: a CIF frame's 11 x 9, more than a QCIF frame's 6 x 5

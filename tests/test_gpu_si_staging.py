@@ -55,3 +55,21 @@ def test_results_left_out(ctx):
         assert np.array_equal(a[0], b[0])
         assert np.array_equal(a[1], b[1] if k % 2 else np.full_like(a[1], 7)), k
         assert np.array_equal(a[2], b[2] if k % 3 else np.full_like(a[2], 7)), k
+
+
+def test_more_pairs_than_a_grid_has_planes():
+    """33000 QCIF pairs have 66000 key frames, more than a launch takes in one
+    dimension (65535)."""
+    n, pairs = 33000, _pairs([(176, 144)] * 4)
+    with _lib.Context() as c:
+        want = [s for s, _, _ in c.side_info_batch(pairs)]
+        got = np.zeros((n, 144, 176), np.uint8)
+        reqs = (_lib.SIRequest * n)()
+        for k in range(n):
+            p = pairs[k % 4]
+            pi, ci, fi = p["idx"]
+            reqs[k] = _lib.SIRequest(176, 144, p["qindex"], pi, ci, fi, p["past"].ctypes.data, p["fut"].ctypes.data,
+                                     got[k].ctypes.data, None, None)
+        _lib._check(_lib.lib.dvc_side_info_batch(c.h, n, reqs), "dvc_side_info_batch")
+    for k in range(4):
+        assert (got[k::4] == want[k]).all(), k
