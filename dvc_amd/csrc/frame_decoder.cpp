@@ -1,20 +1,19 @@
 // frame_decoder.cpp -- host orchestration of WZ frame decoding on the GPU.
 //
-// The per-frame loop is decodeGOP's body (DvcDec/src/DVC_Decoder.cpp:26-474)
-// with skip/intra/deblocking off: side information, residue transform and
-// noise parameters, over-complete transform, then for each zig-zag band with
-// bits: noise distribution; for each bit from MSB: conditional bit
-// probability, conditional entropy, LDPCA rate search, bitplane insertion;
-// then reconstruction, inverse transform, SI refresh, over-complete
-// transform and motion learning; finally the inverse transform.
+// The per-frame loop is decodeGOP's body (DvcDec/src/DVC_Decoder.cpp:26-474):
+// side information, residue transform and noise parameters, over-complete
+// transform, then for each zig-zag band with bits: noise distribution; for each
+// bit from MSB: conditional bit probability, conditional entropy, LDPCA rate
+// search, bitplane insertion; then reconstruction, inverse transform, SI
+// refresh, over-complete transform and motion learning; finally the inverse
+// transform, skip blocks and deblocking.
 //
 // All frame state stays on the device.  A batch of frames advances in
 // lockstep, one bitplane per step; each kernel launch covers every frame that
 // needs it in that step (frames of different sizes and quantisers mix freely,
 // each following its own band schedule).  The host only decides which frames
-// start or finish a band, and reads back, once per finished band, the rare
-// reconstruction entries that lie within a rounding margin (recomputed with
-// the C library's exp so the integers equal the CPU path's).
+// start or finish a band, queues a step's launches without waiting for the step
+// before, and reads back the results of the frames that a step finishes.
 #include <math.h>
 #include <string.h>
 #include <algorithm>
